@@ -1,0 +1,335 @@
+// One pseudo-time step of the z-line preconditioner in one kernel: the
+// right-hand side s + deta (H s - b) (H: the horizontal 22-point part of the
+// operator; FIRST: deta (0 - b), from s = 0) and the line solve in z that
+// follows it (apply_preconditioner!.jl:40-124), shared by the FP64
+// preconditioner and the FP32 one.
+#pragma once
+
+#include <type_traits>
+
+#include "pcf_internal.hpp"
+
+namespace pcf {
+namespace {
+
+// The grid is cut into tiles of 32 x 2 columns.  A tile's coefficients lie
+// together in memory, [tile][k][coefficient][64 columns], and so do its
+// line-solve factors, [tile][k][P, E, Q][64 columns] (k_line_pack): the 128
+// levels of a block's columns are then one contiguous stream.  With x-fastest
+// arrays every level and coefficient of a column lies on a page of its own,
+// and the same kernel took 234 us instead of 120 at 256 x 256 x 128 (bf16).
+//
+// A block takes one tile; thread (x, seg) owns the NPL consecutive levels
+// from seg NPL of W adjacent columns, so the block has CX ceil(nz / NPL)
+// threads, CX = 64 / W.  A thread evaluates the right-hand side of
+// its levels in registers.  The two recurrences of the line solve,
+// s_k = (r_k + e_k s_(k-1)) p_k upwards and y_k = s_k + q_k y_(k+1)
+// downwards, are affine maps: a thread composes those of its levels, the
+// segments' maps meet in LDS, and each thread composes the segments below
+// (above) it and replays its own levels with the value that enters them.  So
+// the right-hand side never goes to memory, all loads of a column are
+// independent of each other, and a grid with few columns still fills the
+// chip with nz / NPL threads per column.
+//
+// What bounds it: on a large grid memory traffic (72 B per cell with bf16
+// coefficients and an FP64 right-hand side: 604 MB in 122 us, 5.0 TB/s, at
+// 256 x 256 x 128; a horizontal kernel and a line solve apart took 128), on a
+// small one the round trips of a thread's loads (48 x 40 x 64: 11 us against
+// 23).  Before, a thread walked each column alone: 30 us for the first step
+// at 128 x 128 x 128, 10.5 now.
+
+// x-fastest coefficients and line-solve factors
+template <typename T>
+struct LineCoefs {
+  const T* a[T_COUNT];
+  const T *P, *E, *Q;
+};
+
+constexpr int kTileX = 32, kTileY = 2, kTileCols = kTileX * kTileY;
+
+__host__ __device__ inline int line_tiles(int nx, int ny) {
+  return ((nx + kTileX - 1) / kTileX) * ((ny + kTileY - 1) / kTileY);
+}
+
+// bytes of dynamic LDS of a block of `threads` threads
+template <typename R, int W>
+constexpr unsigned line_lds(int threads) {
+  return (unsigned)(4 * threads * W * sizeof(R));
+}
+
+// W consecutive values of a vector (W a power of two, the address aligned to
+// them), cached or streamed past the caches
+template <int W, typename T>
+struct LineVec {
+  typedef T type __attribute__((ext_vector_type(W)));
+};
+template <typename T>
+struct LineVec<1, T> {
+  typedef T type;
+};
+template <int W, bool STREAM, typename T>
+__device__ __forceinline__ void line_load(const T* p, T (&o)[W]) {
+  using V = typename LineVec<W, T>::type;
+  V v;
+  if constexpr (STREAM) v = __builtin_nontemporal_load((const V*)p);
+  else v = *(const V*)p;
+  if constexpr (W == 1) o[0] = v;
+  else
+#pragma unroll
+    for (int c = 0; c < W; ++c) o[c] = v[c];
+}
+template <int W, typename T, typename R>
+__device__ __forceinline__ void line_store(T* p, const R (&o)[W]) {
+  typename LineVec<W, T>::type v;
+  if constexpr (W == 1) v = (T)o[0];
+  else
+#pragma unroll
+    for (int c = 0; c < W; ++c) v[c] = (T)o[c];
+  *(typename LineVec<W, T>::type*)p = v;
+}
+// W coefficients as loaded (FP64, FP32, or bf16 bits, two to a word) and one
+// of them in the arithmetic type
+template <int W, typename CT>
+struct LineCoef {
+  static constexpr bool pairs = sizeof(CT) == 2 && W > 1;
+  static constexpr int N = pairs ? W / 2 : W;
+  using T = std::conditional_t<pairs, unsigned, CT>;
+  T v[N];
+  __device__ __forceinline__ void load(const CT* p) { line_load<N, true>((const T*)p, v); }
+  template <typename R>
+  __device__ __forceinline__ R get(int c) const {
+    if constexpr (pairs) return __uint_as_float(c & 1 ? v[c / 2] & 0xffff0000u : v[c / 2] << 16);
+    else if constexpr (sizeof(CT) == 2) return __uint_as_float((unsigned)v[c] << 16);
+    else return v[c];
+  }
+};
+
+// The line solve of the right-hand sides r of a thread's levels; y: the
+// solution there, left in r.  f: the packed factors (of k_pc_factors) of the
+// thread's first level and column; lds: line_lds bytes.
+template <typename R, int W, int NPL>
+__device__ __forceinline__ void line_solve_segments(const R* __restrict__ f, int k0, int nz, int tx, int seg, int nseg,
+                                                    R (&r)[NPL][W], R* lds) {
+  constexpr int CX = kTileCols / W;
+  R *la = lds, *lb = lds + CX * W * nseg, *lc = lb + CX * W * nseg, *ld = lc + CX * W * nseg;
+  const int at = (seg * CX + tx) * W;
+  R e[NPL][W], p[NPL][W], q[NPL][W];
+  R A[W], B[W];
+#pragma unroll
+  for (int c = 0; c < W; ++c) {
+    A[c] = 0;
+    B[c] = 1;
+  }
+#pragma unroll
+  for (int u = 0; u < NPL; ++u) {
+    const R* fu = f + 3 * kTileCols * (min(k0 + u, nz - 1) - k0);
+    line_load<W, true>(fu, p[u]);
+    line_load<W, true>(fu + kTileCols, e[u]);
+    line_load<W, true>(fu + 2 * kTileCols, q[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < NPL; ++u) {
+    const int k = k0 + u;
+    const bool in = k < nz;  // else the identity map
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      const bool bottom = u == 0 && k == 0;  // the lowest level's P is the pivot itself
+      const R rr = bottom ? r[u][c] / p[u][c] : r[u][c];
+      r[u][c] = in ? rr : (R)0;
+      p[u][c] = in && !bottom ? p[u][c] : (R)1;
+      e[u][c] = bottom ? (R)0 : (in ? e[u][c] : (R)1);
+      q[u][c] = k == nz - 1 ? (R)0 : (in ? q[u][c] : (R)1);
+      A[c] = (r[u][c] + e[u][c] * A[c]) * p[u][c];
+      B[c] = e[u][c] * B[c] * p[u][c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < W; ++c) {
+    la[at + c] = A[c];
+    lb[at + c] = B[c];
+  }
+  __syncthreads();
+  R sv[W];
+#pragma unroll
+  for (int c = 0; c < W; ++c) sv[c] = 0;
+#pragma unroll 4
+  for (int t = 0; t < seg; ++t)
+#pragma unroll
+    for (int c = 0; c < W; ++c) sv[c] = la[(t * CX + tx) * W + c] + lb[(t * CX + tx) * W + c] * sv[c];
+#pragma unroll
+  for (int u = 0; u < NPL; ++u)
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      sv[c] = (r[u][c] + e[u][c] * sv[c]) * p[u][c];
+      r[u][c] = k0 + u < nz ? sv[c] : (R)0;
+    }
+#pragma unroll
+  for (int c = 0; c < W; ++c) {
+    A[c] = 0;
+    B[c] = 1;
+  }
+#pragma unroll
+  for (int u = NPL - 1; u >= 0; --u)
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      A[c] = r[u][c] + q[u][c] * A[c];
+      B[c] = q[u][c] * B[c];
+    }
+#pragma unroll
+  for (int c = 0; c < W; ++c) {
+    lc[at + c] = A[c];
+    ld[at + c] = B[c];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < W; ++c) sv[c] = 0;
+#pragma unroll 4
+  for (int t = nseg - 1; t > seg; --t)
+#pragma unroll
+    for (int c = 0; c < W; ++c) sv[c] = lc[(t * CX + tx) * W + c] + ld[(t * CX + tx) * W + c] * sv[c];
+#pragma unroll
+  for (int u = NPL - 1; u >= 0; --u)
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      sv[c] = r[u][c] + q[u][c] * sv[c];
+      r[u][c] = sv[c];
+    }
+}
+
+// The same line solve for a column of any height in one thread: rhs(k) gives
+// the right-hand sides in ascending order, f points to the packed factors,
+// col[c + stride k] keeps the upward sweep, put(k, y) takes the solution from
+// the top down.
+template <typename R, class Rhs, class Put>
+__device__ __forceinline__ void line_solve_column(const R* f, R* col, size_t c, size_t stride, int nz, Rhs rhs,
+                                                  Put put) {
+  R s = 0;
+  for (int k = 0; k < nz; ++k) {
+    const R* fk = f + (size_t)3 * kTileCols * k;
+    s = k == 0 ? rhs(k) / fk[0] : (rhs(k) + fk[kTileCols] * s) * fk[0];
+    col[c + stride * k] = s;
+  }
+  put(nz - 1, s);
+  for (int k = nz - 2; k >= 0; --k) {
+    s = col[c + stride * k] + f[(size_t)3 * kTileCols * k + 2 * kTileCols] * s;
+    put(k, s);
+  }
+}
+
+// Pack a grid's x-fastest coefficients and factors (SrcT) into tiles: block
+// (tile, group of 4 levels) of 64 x 4 threads.  The columns beyond the grid
+// of a partial tile get zero coefficients and the identity's factors.
+template <typename SrcT, typename CT, typename R>
+__global__ void __launch_bounds__(256) k_line_pack(LineCoefs<SrcT> A, CT* __restrict__ coefs, R* __restrict__ factors,
+                                                   int nx, int ny, int nz) {
+  const int lane = threadIdx.x, k = blockIdx.y * 4 + threadIdx.y, tile = blockIdx.x;
+  if (k >= nz) return;
+  const int tx = (nx + kTileX - 1) / kTileX;
+  const int i = (tile % tx) * kTileX + lane % kTileX, j = (tile / tx) * kTileY + lane / kTileX;
+  const bool in = i < nx && j < ny;
+  const size_t o = in ? (size_t)i + (size_t)nx * (j + (size_t)ny * k) : 0;
+  CT* c = coefs + ((size_t)tile * nz + k) * T_COUNT * kTileCols + lane;
+  R* f = factors + ((size_t)tile * nz + k) * 3 * kTileCols + lane;
+  for (int t = 0; t < T_COUNT; ++t) {
+    if constexpr (sizeof(CT) == 2) {
+      const unsigned u = in ? __float_as_uint((float)A.a[t][o]) : 0u;
+      c[t * kTileCols] = (CT)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);  // round to nearest even
+    } else {
+      c[t * kTileCols] = in ? (CT)A.a[t][o] : (CT)0;
+    }
+  }
+  f[0] = in ? (R)A.P[o] : (R)1;
+  f[kTileCols] = in ? (R)A.E[o] : (R)0;
+  f[2 * kTileCols] = in ? (R)A.Q[o] : (R)0;
+}
+
+// The block a launch's b-th workgroup takes: consecutive workgroups go to
+// the 8 XCDs in turn, so each XCD gets a contiguous range of blocks (rows
+// whose neighbours are then in its own L2).
+__device__ __forceinline__ int xcd_block(int b, int nb) {
+  const int per = nb / 8;
+  return b < 8 * per ? (b % 8) * per + b / 8 : b;
+}
+
+// At a thread's levels k0 ... k0 + NPL - 1 of the columns (i ... i + W - 1, j)
+// of an x-fastest grid: the right-hand side s + deta (H s - b), or with
+// RESID the residual b - A s of all 25 points.  a: the packed coefficients of
+// the thread's first level and column; rd(ii, jj, kk, v[W]) and
+// rd(ii, jj, kk): the iterate at W cells and at one cell inside the grid.
+// The walk up the levels keeps the five levels of s it needs in registers, so
+// each is loaded once per thread.
+template <typename R, int W, int NPL, int DEPTH, bool RESID, typename CT, typename BT, class Rd>
+__device__ __forceinline__ void line_rhs(const CT* __restrict__ a, Rd rd, const BT* __restrict__ b, int nx, int ny,
+                                         int nz, R deta, int i, int j, int k0, R (&r)[NPL][W]) {
+  const size_t sxy = (size_t)nx * ny;
+  const int im = i == 0 ? nx - 1 : i - 1, ip = i + W == nx ? 0 : i + W;
+  const int jm = j == 0 ? ny - 1 : j - 1, jp = j + 1 == ny ? 0 : j + 1;
+  // s on the levels k0 - 2 ... k0 + NPL + 1.  Every load is unconditional (at
+  // a level inside the grid; those beyond the walls are zeroed where they are
+  // used), so that no branch comes between the loads.  DEPTH >= 0: the
+  // coefficients of the next DEPTH levels are loaded before a level is
+  // evaluated and those beyond it after, which a compiler barrier at the
+  // level's result keeps (without it the loads are hoisted until the registers
+  // spill); DEPTH < 0 leaves the order to the compiler.
+  constexpr int LAG = DEPTH < 0 ? 0 : DEPTH, AHEAD = 4 + LAG;  // levels of s loaded before the first is evaluated
+  R C[NPL + 4][W + 2], F[NPL + 4][W], B[NPL + 4][W];  // C with its x neighbours
+  auto level = [&](int w) {
+    const int kk = min(max(k0 - 2 + w, 0), nz - 1);
+    R v[W];
+    rd(i, j, kk, v);
+#pragma unroll
+    for (int c = 0; c < W; ++c) C[w][c + 1] = v[c];
+    C[w][0] = rd(im, j, kk);
+    C[w][W + 1] = rd(ip, j, kk);
+    rd(i, jp, kk, F[w]);
+    rd(i, jm, kk, B[w]);
+  };
+  LineCoef<W, CT> T[LAG + 1][T_COUNT];
+  BT bv[LAG + 1][W];
+  auto coefs = [&](int u) {
+    const int d = u % (LAG + 1), v = min(k0 + u, nz - 1) - k0;  // v < 0 only for idle segments
+    const CT* av = a + T_COUNT * kTileCols * v;
+#pragma unroll
+    for (int t = 0; t < T_COUNT; ++t)
+      if (RESID || (t != T_AC && t != T_AD && t != T_AU)) T[d][t].load(av + t * kTileCols);
+    line_load<W, true>(b + ((size_t)i + (size_t)nx * j + sxy * (size_t)(k0 + v)), bv[d]);
+  };
+#pragma unroll
+  for (int w = 0; w < AHEAD && w < NPL + 4; ++w) level(w);
+#pragma unroll
+  for (int u = 0; u < LAG; ++u) coefs(u);
+#pragma unroll
+  for (int u = 0; u < NPL; ++u) {
+    const int m = u + 2, d = u % (LAG + 1);
+    if (AHEAD + u < NPL + 4) level(AHEAD + u);
+    if (u + LAG < NPL) coefs(u + LAG);
+    const int k = k0 + u;
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      auto A = [&](int t) -> R { return T[d][t].template get<R>(c); };
+      // the levels two below ... two above; zero beyond the walls
+      auto Z = [&](R x, int w) -> R {
+        const int kk = k0 + w - 2;
+        return w == m ? x : ((unsigned)kk < (unsigned)nz ? x : (R)0);
+      };
+      auto XL = [&](int w) -> R { return Z(C[w][c], w); };
+      auto XR = [&](int w) -> R { return Z(C[w][c + 2], w); };
+      auto X0 = [&](int w) -> R { return Z(C[w][c + 1], w); };
+      auto YF = [&](int w) -> R { return Z(F[w][c], w); };
+      auto YB = [&](int w) -> R { return Z(B[w][c], w); };
+      R v = A(T_AL) * XL(m) + A(T_AR) * XR(m) + A(T_AF) * YF(m) + A(T_AB) * YB(m);
+      if constexpr (RESID) v += A(T_AU) * X0(m + 1) + A(T_AD) * X0(m - 1) + A(T_AC) * X0(m);
+      v += A(T_ARU) * XR(m + 1) + A(T_ARD) * XR(m - 1) + A(T_ALU) * XL(m + 1) + A(T_ALD) * XL(m - 1) +
+           A(T_AFU) * YF(m + 1) + A(T_AFD) * YF(m - 1) + A(T_ABU) * YB(m + 1) + A(T_ABD) * YB(m - 1) +
+           A(T_AUU) * X0(m + 2) + A(T_ADD) * X0(m - 2) + A(T_ARUU) * XR(m + 2) + A(T_ARDD) * XR(m - 2) +
+           A(T_ALUU) * XL(m + 2) + A(T_ALDD) * XL(m - 2) + A(T_AFUU) * YF(m + 2) + A(T_AFDD) * YF(m - 2) +
+           A(T_ABUU) * YB(m + 2) + A(T_ABDD) * YB(m - 2);
+      const R rr = RESID ? (R)bv[d][c] - v : X0(m) + deta * (v - (R)bv[d][c]);
+      r[u][c] = k < nz ? rr : (R)0;
+      if constexpr (DEPTH >= 0) asm volatile("" : "+v"(r[u][c])::"memory");
+    }
+  }
+}
+
+}  // namespace
+}  // namespace pcf

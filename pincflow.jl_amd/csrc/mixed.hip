@@ -19,6 +19,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "line_step.hpp"
 #include "pcf_device.hpp"
 #include "solver_common.hpp"
 
@@ -28,7 +29,6 @@ namespace {
 
 typedef float flt4 __attribute__((ext_vector_type(4)));
 
-// CT: float, or uint16_t holding bf16 bits (the upper half of an FP32)
 // Memory layout of a level's arrays: x fastest (the finest level and the
 // levels smoothed with row-parallel kernels) or z fastest (the coarse levels
 // smoothed one column per wavefront, whose accesses are then contiguous
@@ -59,261 +59,136 @@ struct Lay {
   }
 };
 
+// A pseudo-time step's operands on an x-fastest grid: the packed coefficients
+// (CT: float, or uint16_t holding bf16 bits, the upper half of an FP32) and
+// factors, and the iterate.
 template <typename CT>
-struct PcArgs {
-  const CT* a[T_COUNT];  // the 22 horizontal coefficients are used here
+struct LineArgs {
+  const CT* coefs;
+  const float* factors;
   const float* s;
-  float* out;
   int nx, ny, nz;
-  // coarse-level correction added to s first (k_pc_rhs32<..., PRO = true>):
-  // s + omega e at the coarse cell (i >> sx, j >> sy, k) in layout cl
+  float deta;
+  // coarse-level correction added to s first (PRO = true): s + omega e at
+  // the coarse cell (i >> sx, j >> sy, k) in layout cl
   const float* e;
   float omega;
   int sx, sy;
   Lay cl;
 };
-using PcArgs32 = PcArgs<float>;
 
-template <typename CT>
-struct Coefs {
-  const CT* a[T_COUNT];
-};
-
-// W consecutive floats: W = 4 as one 16-byte access, W = 1 as a scalar.
-template <int W>
-__device__ __forceinline__ void ld(const float* p, float (&o)[W]) {
-  if constexpr (W == 4) {
-    const flt4 v = *(const flt4*)p;
-    o[0] = v.x;
-    o[1] = v.y;
-    o[2] = v.z;
-    o[3] = v.w;
-  } else {
-    o[0] = *p;
+// The iterate of a step: s, or with PRO s + omega P e, the multigrid
+// prolongation of the coarse-level correction fused into the first
+// post-smoothing step.
+template <int W, bool PRO, typename CT>
+struct LineRead {
+  const LineArgs<CT>& A;
+  __device__ __forceinline__ float operator()(int i, int j, int k) const {
+    float v = A.s[(size_t)i + (size_t)A.nx * (j + (size_t)A.ny * k)];
+    if constexpr (PRO) v += A.omega * A.e[A.cl.at(i >> A.sx, j >> A.sy, k)];
+    return v;
   }
-}
-template <int W>
-__device__ __forceinline__ void ld_stream(const float* p, float (&o)[W]) {
-  if constexpr (W == 4) {
-    const flt4 v = __builtin_nontemporal_load((const flt4*)p);
-    o[0] = v.x;
-    o[1] = v.y;
-    o[2] = v.z;
-    o[3] = v.w;
-  } else {
-    o[0] = __builtin_nontemporal_load(p);
-  }
-}
-template <int W>
-__device__ __forceinline__ void st_stream(float* p, const float (&v)[W]) {
-  if constexpr (W == 4) {
-    flt4 x;
-    x.x = v[0];
-    x.y = v[1];
-    x.z = v[2];
-    x.w = v[3];
-    __builtin_nontemporal_store(x, (flt4*)p);
-  } else {
-    __builtin_nontemporal_store(v[0], p);
-  }
-}
-
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-
-// W consecutive coefficients, streamed (not kept in the caches), as FP32.
-template <int W, typename CT>
-__device__ __forceinline__ void ld_coef(const CT* p, float (&o)[W]) {
-  if constexpr (sizeof(CT) == 4) {
-    ld_stream<W>((const float*)p, o);
-  } else if constexpr (W == 4) {
-    const u32x2 v = __builtin_nontemporal_load((const u32x2*)p);
-    o[0] = __uint_as_float(v.x << 16);
-    o[1] = __uint_as_float(v.x & 0xffff0000u);
-    o[2] = __uint_as_float(v.y << 16);
-    o[3] = __uint_as_float(v.y & 0xffff0000u);
-  } else {
-    o[0] = __uint_as_float((unsigned)__builtin_nontemporal_load(p) << 16);
-  }
-}
-
-// The later pseudo-time steps of the preconditioner in FP32:
-// out = s + deta (H s - sin) with H the horizontal 22-point part of the
-// operator (apply_preconditioner!.jl:62-63); sin: the FP64 or FP32 input.
-// W x-adjacent cells per thread, block = (64 / W) x (4 W) threads covering
-// 64 x (4 W) cells of one z-level; CT: the coefficients' storage.  PRO: the
-// iterate is s + omega P e, the multigrid prolongation of the coarse-level
-// correction fused into the first post-smoothing step.
-// The body takes the block's index, so that the ensemble kernel can run it
-// for a block of any member.
-template <int W, typename SinT, typename CT = float, bool PRO = false>
-__device__ __forceinline__ void pc_rhs32(const PcArgs<CT>& A, const SinT* __restrict__ sin, float deta, int bx,
-                                         int by, int bz) {
-  constexpr int BX = 64 / W;
-  const int i0 = (bx * BX + threadIdx.x) * W;
-  const int j = by * (4 * W) + threadIdx.y;
-  const int k = bz;
-  const int nx = A.nx, ny = A.ny, nz = A.nz;
-  if (i0 >= nx || j >= ny) return;
-  const size_t sxy = (size_t)nx * ny;
-  const size_t o = (size_t)i0 + (size_t)nx * j + sxy * k;
-  const int im = i0 == 0 ? nx - 1 : i0 - 1, ip = i0 + W == nx ? 0 : i0 + W;
-  const int jp = j + 1 == ny ? 0 : j + 1, jm = j == 0 ? ny - 1 : j - 1;
-  const float* s = A.s;
-  float C[5][W], F[5][W], B[5][W], L[5], R[5];
-#pragma unroll
-  for (int w = 0; w < 5; ++w) {
-    const int kk = k - 2 + w;
-    if (kk < 0 || kk >= nz) {
-#pragma unroll
-      for (int c = 0; c < W; ++c) C[w][c] = F[w][c] = B[w][c] = 0.0f;
-      L[w] = R[w] = 0.0f;
-      continue;
-    }
-    const size_t pl = sxy * kk;
-    ld<W>(s + pl + (size_t)nx * j + i0, C[w]);
-    ld<W>(s + pl + (size_t)nx * jp + i0, F[w]);
-    ld<W>(s + pl + (size_t)nx * jm + i0, B[w]);
-    L[w] = s[pl + (size_t)nx * j + im];
-    R[w] = s[pl + (size_t)nx * j + ip];
+  __device__ __forceinline__ void operator()(int i, int j, int k, float (&v)[W]) const {
+    line_load<W, false>(A.s + ((size_t)i + (size_t)A.nx * (j + (size_t)A.ny * k)), v);
     if constexpr (PRO) {
-      auto E = [&](int ii, int jj) -> float { return A.omega * A.e[A.cl.at(ii >> A.sx, jj >> A.sy, kk)]; };
-      if (W == 4 && A.sx == 1 && !A.cl.zf) {
-        // cells i0, i0 + 1 and i0 + 2, i0 + 3 share the coarse cells i0 / 2
-        // and i0 / 2 + 1: one 8-byte load per row
-        auto E2 = [&](int jj) -> float2 { return *(const float2*)(A.e + A.cl.at(i0 >> 1, jj >> A.sy, kk)); };
-        const float2 ec = E2(j), ef = E2(jp), eb = E2(jm);
+      if constexpr (W == 4) {
+        if (A.sx == 1 && !A.cl.zf) {  // the two coarse cells of the four fine ones
+          float e[2];
+          line_load<2, false>(A.e + A.cl.at(i >> 1, j >> A.sy, k), e);
 #pragma unroll
-        for (int c = 0; c < W; ++c) {
-          const float o = A.omega;
-          C[w][c] += o * (c < 2 ? ec.x : ec.y);
-          F[w][c] += o * (c < 2 ? ef.x : ef.y);
-          B[w][c] += o * (c < 2 ? eb.x : eb.y);
-        }
-      } else {
-#pragma unroll
-        for (int c = 0; c < W; ++c) {
-          C[w][c] += E(i0 + c, j);
-          F[w][c] += E(i0 + c, jp);
-          B[w][c] += E(i0 + c, jm);
+          for (int c = 0; c < 4; ++c) v[c] += A.omega * e[c / 2];
+          return;
         }
       }
-      L[w] += E(im, j);
-      R[w] += E(ip, j);
+#pragma unroll
+      for (int c = 0; c < W; ++c) v[c] += A.omega * A.e[A.cl.at((i + c) >> A.sx, j >> A.sy, k)];
     }
   }
-  float a[T_COUNT][W];
-#pragma unroll
-  for (int t = 0; t < T_COUNT; ++t) {
-    if (t == T_AC || t == T_AD || t == T_AU) continue;
-    ld_coef<W, CT>(A.a[t] + o, a[t]);
-  }
-  float out[W];
-#pragma unroll
-  for (int c = 0; c < W; ++c) {
-    auto XL = [&](int w) -> float { return c == 0 ? L[w] : C[w][c - 1]; };
-    auto XR = [&](int w) -> float { return c == W - 1 ? R[w] : C[w][c + 1]; };
-    auto X0 = [&](int w) -> float { return C[w][c]; };
-    auto YF = [&](int w) -> float { return F[w][c]; };
-    auto YB = [&](int w) -> float { return B[w][c]; };
-    float v = a[T_AL][c] * XL(2) + a[T_AR][c] * XR(2) + a[T_AF][c] * YF(2) + a[T_AB][c] * YB(2);
-    v += a[T_ARU][c] * XR(3) + a[T_ARD][c] * XR(1) + a[T_ALU][c] * XL(3) + a[T_ALD][c] * XL(1) +
-         a[T_AFU][c] * YF(3) + a[T_AFD][c] * YF(1) + a[T_ABU][c] * YB(3) + a[T_ABD][c] * YB(1) +
-         a[T_AUU][c] * X0(4) + a[T_ADD][c] * X0(0) + a[T_ARUU][c] * XR(4) + a[T_ARDD][c] * XR(0) +
-         a[T_ALUU][c] * XL(4) + a[T_ALDD][c] * XL(0) + a[T_AFUU][c] * YF(4) + a[T_AFDD][c] * YF(0) +
-         a[T_ABUU][c] * YB(4) + a[T_ABDD][c] * YB(0);
-    out[c] = X0(2) + deta * (v - (float)sin[o + c]);
-  }
-  st_stream<W>(A.out + o, out);
-}
-template <int W, typename SinT, typename CT = float, bool PRO = false>
-__global__ void __launch_bounds__(256) k_pc_rhs32(PcArgs<CT> A, const SinT* __restrict__ sin, float deta,
-                                                  const SolverScalars* sc) {
-  if (sc && sc->done) return;
-  pc_rhs32<W, SinT, CT, PRO>(A, sin, deta, blockIdx.x, blockIdx.y, blockIdx.z);
-}
+};
 
-// The preconditioner's line solve in z with FP32 factors (the recurrence of
-// the FP64 k_pc_thomas); SrcT / OutT: FP64 or FP32 input and output vectors.
-// One column per thread, blockDim.x = 64.  The upward sweep keeps its values
-// of the lowest NLDS levels in LDS (NLDS x 64 x 4 B per wavefront) and those
-// of higher levels in the FP32 scratch `col`.  FIRST: rhs = deta (0 - src).
-// The compiler barriers keep each batch of loads ahead of its recurrence
-// (without LDS, the possible aliasing of `col` does).  LDS pays where a level
-// has enough columns for several wavefronts per CU (kThomas32LdsColumns);
-// with fewer, the LDS round trips are not hidden and NLDS = 0 is faster.
-constexpr int kThomas32Lds = 128;
-constexpr size_t kThomas32LdsColumns = 32768;
+// The columns and levels of a thread of tile `tile` (line_step.hpp).
+template <int W, int NPL>
+struct LineThread {
+  int tx, seg, i, j, k0;
+  bool act;
+  size_t o, c;  // the first cell in the x-fastest arrays; its column in the tile's arrays
+  __device__ __forceinline__ LineThread(int tile, int nx, int ny, int nz) {
+    constexpr int CX = kTileCols / W;
+    const int tiles_x = (nx + kTileX - 1) / kTileX;
+    tx = threadIdx.x % CX;
+    seg = threadIdx.x / CX;
+    i = (tile % tiles_x) * kTileX + (tx * W) % kTileX;
+    j = (tile / tiles_x) * kTileY + (tx * W) / kTileX;
+    act = i < nx && j < ny;
+    if (i >= nx) i = nx - W;  // idle threads read cells of the grid
+    if (j >= ny) j = ny - 1;
+    k0 = seg * NPL;
+    o = (size_t)i + (size_t)nx * (j + (size_t)ny * k0);
+    c = (size_t)tile * nz + k0;
+  }
+};
 
-template <bool FIRST, typename SrcT, typename OutT, int NLDS = kThomas32Lds>
-__device__ __forceinline__ void pc_thomas32(const float* P, const float* E, const float* Q, const SrcT* src, OutT* out,
-                                            float* col, int nx, int ny, int nz, float deta, int bx, int by) {
-  __shared__ float up[NLDS > 0 ? NLDS : 1][64];
-  constexpr int U = 8;
-  const int tid = threadIdx.x;
-  const int i = bx * 64 + tid;
-  const int j = by;
-  if (i >= nx) return;
+// One pseudo-time step in FP32 of a tile (line_step.hpp); s and out must
+// differ.
+template <int W, int NPL, bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
+__device__ __forceinline__ void line_step32(const LineArgs<CT>& A, const BT* __restrict__ b, OutT* __restrict__ out,
+                                            int tile) {
+  extern __shared__ float line_shared[];
+  const int nx = A.nx, ny = A.ny, nz = A.nz;
+  const LineThread<W, NPL> t(tile, nx, ny, nz);
   const size_t sxy = (size_t)nx * ny;
-  const size_t c = (size_t)i + (size_t)nx * j;
-  auto rhs_of = [&](SrcT v) -> float { return FIRST ? deta * (0.0f - (float)v) : (float)v; };
-  auto keep = [&](int k, float v) {
-    if (k < NLDS)
-      up[k][tid] = v;
-    else
-      col[c + sxy * k] = v;
-  };
-  auto kept = [&](int k) -> float { return k < NLDS ? up[k][tid] : col[c + sxy * k]; };
-  float sk = rhs_of(src[c]) / P[c];
-  keep(0, sk);
-  int k = 1;
-  for (; k + U <= nz; k += U) {
-    float r[U], e[U], p[U];
+  float r[NPL][W];
+  if constexpr (FIRST) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const size_t o = c + sxy * (k + u);
-      r[u] = rhs_of(src[o]);
-      e[u] = E[o];
-      p[u] = P[o];
-    }
-    if constexpr (NLDS > 0) asm volatile("" ::: "memory");
+    for (int u = 0; u < NPL; ++u) {
+      BT v[W];
+      line_load<W, false>(b + (t.o + sxy * (ptrdiff_t)(min(t.k0 + u, nz - 1) - t.k0)), v);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      sk = (r[u] + e[u] * sk) * p[u];
-      keep(k + u, sk);
+      for (int c = 0; c < W; ++c) r[u][c] = t.k0 + u < nz ? A.deta * (0.0f - (float)v[c]) : 0.0f;
     }
+  } else {
+    // what the registers allow
+    constexpr int DEPTH = W == 1 && NPL == 8 && !PRO ? 1 : W == 4 && !PRO && sizeof(CT) == 2 ? -1 : 0;
+    line_rhs<float, W, NPL, DEPTH, false, CT, BT>(A.coefs + t.c * T_COUNT * kTileCols + t.tx * W, LineRead<W, PRO, CT>{A}, b,
+                                           nx, ny, nz, A.deta, t.i, t.j, t.k0, r);
   }
-  for (; k < nz; ++k) {
-    const size_t o = c + sxy * k;
-    sk = (rhs_of(src[o]) + E[o] * sk) * P[o];
-    keep(k, sk);
-  }
-  out[c + sxy * (nz - 1)] = (OutT)sk;
-  k = nz - 2;
-  for (; k - (U - 1) >= 0; k -= U) {
-    float r[U], q[U];
+  line_solve_segments<float, W, NPL>(A.factors + t.c * 3 * kTileCols + t.tx * W, t.k0, nz, t.tx, t.seg,
+                                     blockDim.x / (kTileCols / W), r, line_shared);
+  if (t.act) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      r[u] = kept(k - u);
-      q[u] = Q[c + sxy * (k - u)];
-    }
-    if constexpr (NLDS > 0) asm volatile("" ::: "memory");
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      sk = r[u] + q[u] * sk;
-      out[c + sxy * (k - u)] = (OutT)sk;
-    }
-  }
-  for (; k >= 0; --k) {
-    sk = kept(k) + Q[c + sxy * k] * sk;
-    out[c + sxy * k] = (OutT)sk;
+    for (int u = 0; u < NPL; ++u)
+      if (t.k0 + u < nz) line_store<W>(out + t.o + sxy * u, r[u]);
   }
 }
-template <bool FIRST, typename SrcT, typename OutT, int NLDS = kThomas32Lds>
-__global__ void __launch_bounds__(64) k_pc_thomas32(const float* P, const float* E, const float* Q, const SrcT* src,
-                                                    OutT* out, float* col, int nx, int ny, int nz, float deta,
-                                                    const SolverScalars* sc) {
+template <int W, int NPL, bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
+__global__ void __launch_bounds__(W == 4 ? 512 : 1024) __attribute__((amdgpu_waves_per_eu(W == 4 ? 2 : 4, W == 4 ? 2 : 4)))
+    k_line_step32(LineArgs<CT> A, const BT* __restrict__ b, OutT* __restrict__ out, const SolverScalars* sc) {
   if (sc && sc->done) return;
-  pc_thomas32<FIRST, SrcT, OutT, NLDS>(P, E, Q, src, out, col, nx, ny, nz, deta, blockIdx.x, blockIdx.y);
+  line_step32<W, NPL, FIRST, PRO, CT, BT, OutT>(A, b, out, xcd_block(blockIdx.x, gridDim.x));
+}
+
+// The same step for columns of more than kLineMaxNz levels, one thread per
+// column; col: FP32 scratch of the grid's size.
+template <bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
+__global__ void __launch_bounds__(kTileCols) k_line_tall32(LineArgs<CT> A, const BT* __restrict__ b,
+                                                           OutT* __restrict__ out, float* col,
+                                                           const SolverScalars* sc) {
+  if (sc && sc->done) return;
+  const LineThread<1, 1> t(blockIdx.x, A.nx, A.ny, A.nz);
+  if (!t.act) return;
+  const size_t sxy = (size_t)A.nx * A.ny;
+  auto rhs = [&](int k) -> float {
+    if constexpr (FIRST) {
+      return A.deta * (0.0f - (float)b[t.o + sxy * k]);
+    } else {
+      float r[1][1];
+      line_rhs<float, 1, 1, 0, false, CT, BT>(A.coefs + (t.c + k) * T_COUNT * kTileCols + t.tx, LineRead<1, PRO, CT>{A}, b,
+                                           A.nx, A.ny, A.nz, A.deta, t.i, t.j, k, r);
+      return r[0][0];
+    }
+  };
+  line_solve_column<float>(A.factors + t.c * 3 * kTileCols + t.tx, col, t.o, sxy, A.nz, rhs,
+                           [&](int k, float y) { out[t.o + sxy * k] = (OutT)y; });
 }
 
 __global__ void k_to_f32(const double* a, float* b, size_t n) {
@@ -462,77 +337,36 @@ __global__ void k_mg_sum(const float* __restrict__ r, float* __restrict__ bc, La
   bc[t] = sum;
 }
 
-// b_coarse = R (b - A s) for 2 x 2 aggregation and nx % 4 == 0: block
-// 16 x 16 threads, 4 x-adjacent fine cells per thread (the loads of
-// k_pc_rhs32); the x pairs are summed in the thread, the y pairs across the
-// lanes l and l + 16 of a wavefront (rows j and j + 1).
-template <typename BT, typename CT>
-__global__ void __launch_bounds__(256) k_resid_restrict4(Coefs<CT> A, const BT* __restrict__ b,
-                                                         const float* __restrict__ s, float* __restrict__ bc, int nx,
-                                                         int ny, int nz, Lay cl, const SolverScalars* sc) {
+// b_coarse = R (b - A s) for 2 x 2 aggregation: a block per tile as in the
+// line steps; the x pairs are summed in the thread (W = 4) or across lanes,
+// the rows j and j + 1 of a tile across lanes.
+template <int W, int NPL, typename BT, typename CT>
+__global__ void __launch_bounds__(W == 4 ? 512 : 1024)
+    __attribute__((amdgpu_waves_per_eu(W == 4 ? 2 : 4, W == 4 ? 2 : 4))) k_resid_restrict(LineArgs<CT> A, const BT* __restrict__ b,
+                                                         float* __restrict__ bc, const SolverScalars* sc) {
   if (sc && sc->done) return;
-  constexpr int W = 4;
-  const int i0 = (blockIdx.x * 16 + threadIdx.x) * W;
-  const int j = blockIdx.y * 16 + threadIdx.y;
-  const int k = blockIdx.z;
-  const bool act = i0 < nx && j < ny;
-  float c0 = 0.0f, c1 = 0.0f;
-  if (act) {
-    const size_t sxy = (size_t)nx * ny;
-    const size_t o = (size_t)i0 + (size_t)nx * j + sxy * k;
-    const int im = i0 == 0 ? nx - 1 : i0 - 1, ip = i0 + W == nx ? 0 : i0 + W;
-    const int jp = j + 1 == ny ? 0 : j + 1, jm = j == 0 ? ny - 1 : j - 1;
-    float C[5][W], F[5][W], B[5][W], L[5], R[5];
+  const int nx = A.nx, ny = A.ny, nz = A.nz;
+  const int tile = xcd_block(blockIdx.x, gridDim.x);
+  const LineThread<W, NPL> t(tile, nx, ny, nz);
+  float r[NPL][W];
+  line_rhs<float, W, NPL, W == 1 && NPL == 8 ? 1 : 0, true, CT, BT>(A.coefs + t.c * T_COUNT * kTileCols + t.tx * W, LineRead<W, false, CT>{A}, b,
+                                        nx, ny, nz, A.deta, t.i, t.j, t.k0, r);
+  constexpr int row = kTileX / W;  // threads per row of the tile
 #pragma unroll
-    for (int w = 0; w < 5; ++w) {
-      const int kk = k - 2 + w;
-      if (kk < 0 || kk >= nz) {
-#pragma unroll
-        for (int c = 0; c < W; ++c) C[w][c] = F[w][c] = B[w][c] = 0.0f;
-        L[w] = R[w] = 0.0f;
-        continue;
+  for (int u = 0; u < NPL; ++u) {
+    const int k = t.k0 + u;
+    if constexpr (W == 4) {
+      const float c0 = r[u][0] + r[u][1], c1 = r[u][2] + r[u][3];
+      // every lane takes part in the exchange
+      const float u0 = __shfl_down(c0, row), u1 = __shfl_down(c1, row);
+      if (t.act && k < nz && (t.tx & row) == 0) {
+        bc[A.cl.at(t.i / 2, t.j / 2, k)] = c0 + u0;
+        bc[A.cl.at(t.i / 2 + 1, t.j / 2, k)] = c1 + u1;
       }
-      const size_t pl = sxy * kk;
-      ld<W>(s + pl + (size_t)nx * j + i0, C[w]);
-      ld<W>(s + pl + (size_t)nx * jp + i0, F[w]);
-      ld<W>(s + pl + (size_t)nx * jm + i0, B[w]);
-      L[w] = s[pl + (size_t)nx * j + im];
-      R[w] = s[pl + (size_t)nx * j + ip];
-    }
-    float a[T_COUNT][W];
-#pragma unroll
-    for (int t = 0; t < T_COUNT; ++t) ld_coef<W, CT>(A.a[t] + o, a[t]);
-    float r[W];
-#pragma unroll
-    for (int c = 0; c < W; ++c) {
-      auto XL = [&](int w) -> float { return c == 0 ? L[w] : C[w][c - 1]; };
-      auto XR = [&](int w) -> float { return c == W - 1 ? R[w] : C[w][c + 1]; };
-      auto X0 = [&](int w) -> float { return C[w][c]; };
-      auto YF = [&](int w) -> float { return F[w][c]; };
-      auto YB = [&](int w) -> float { return B[w][c]; };
-      float v = a[T_AL][c] * XL(2) + a[T_AR][c] * XR(2) + a[T_AF][c] * YF(2) + a[T_AB][c] * YB(2) +
-                a[T_AU][c] * X0(3) + a[T_AD][c] * X0(1) + a[T_AC][c] * X0(2);
-      v += a[T_ARU][c] * XR(3) + a[T_ARD][c] * XR(1) + a[T_ALU][c] * XL(3) + a[T_ALD][c] * XL(1) +
-           a[T_AFU][c] * YF(3) + a[T_AFD][c] * YF(1) + a[T_ABU][c] * YB(3) + a[T_ABD][c] * YB(1) +
-           a[T_AUU][c] * X0(4) + a[T_ADD][c] * X0(0) + a[T_ARUU][c] * XR(4) + a[T_ARDD][c] * XR(0) +
-           a[T_ALUU][c] * XL(4) + a[T_ALDD][c] * XL(0) + a[T_AFUU][c] * YF(4) + a[T_AFDD][c] * YF(0) +
-           a[T_ABUU][c] * YB(4) + a[T_ABDD][c] * YB(0);
-      r[c] = (float)b[o + c] - v;
-    }
-    c0 = r[0] + r[1];
-    c1 = r[2] + r[3];
-  }
-  // every lane takes part in the exchange; lane + 16 is row j + 1 of the same x
-  const float u0 = __shfl_down(c0, 16), u1 = __shfl_down(c1, 16);
-  if (act && (j & 1) == 0) {
-    if (cl.zf) {
-      bc[cl.at(i0 / 2, j / 2, k)] = c0 + u0;
-      bc[cl.at(i0 / 2 + 1, j / 2, k)] = c1 + u1;
     } else {
-      float2 v;
-      v.x = c0 + u0;
-      v.y = c1 + u1;
-      *(float2*)(bc + cl.at(i0 / 2, j / 2, k)) = v;
+      const float c0 = r[u][0] + __shfl_down(r[u][0], 1);
+      const float u0 = __shfl_down(c0, row);
+      if (t.act && k < nz && (t.tx & row) == 0 && (t.i & 1) == 0) bc[A.cl.at(t.i / 2, t.j / 2, k)] = c0 + u0;
     }
   }
 }
@@ -617,33 +451,6 @@ __device__ __forceinline__ void line_maps(const float* P, const float* E, const 
   q = k == nz - 1 ? 0.0f : Q[o];
 }
 
-// Line solve of ncols columns, block 256 = 4 columns.  FIRST: rhs = deta (0 - src).
-template <int NPL, bool FIRST, typename SrcT, typename OutT>
-__global__ void __launch_bounds__(256) k_line_scan(const float* __restrict__ P, const float* __restrict__ E,
-                                                   const float* __restrict__ Q, const SrcT* __restrict__ src,
-                                                   OutT* __restrict__ out, int ncols, int nz, float deta,
-                                                   const SolverScalars* sc) {
-  if (sc && sc->done) return;
-  const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (c >= ncols) return;  // uniform over the wavefront
-  const int lane = threadIdx.x & 63;
-  float fa[NPL], fb[NPL], q[NPL], y[NPL];
-#pragma unroll
-  for (int u = 0; u < NPL; ++u) {
-    const int k = NPL * lane + u;
-    const size_t o = (size_t)c + (size_t)ncols * k;
-    float r = 0.0f;
-    if (k < nz) r = FIRST ? deta * (0.0f - (float)src[o]) : (float)src[o];
-    line_maps(P, E, Q, o, k, nz, r, fa[u], fb[u], q[u]);
-  }
-  scan_line<NPL>(fa, fb, q, nz, y);
-#pragma unroll
-  for (int u = 0; u < NPL; ++u) {
-    const int k = NPL * lane + u;
-    if (k < nz) out[(size_t)c + (size_t)ncols * k] = (OutT)y[u];
-  }
-}
-
 // One pseudo-time step of column (i, j): the right-hand side
 // s + deta (H s - b) at the lane's levels (FIRST: deta (0 - b), from s = 0),
 // then the line solve.  rd(i, j, k) reads the current iterate; the level's
@@ -686,13 +493,13 @@ __device__ __forceinline__ void column_step(const MgCoefs& A, const float* P, co
 // One smoothing step of a level with few columns, one wavefront per column
 // (block 256 = 4 columns); s_old and out must differ.  PRO: the iterate is
 // s_old + omega P e (e: the coarse-level correction in layout cl,
-// fx = 1 << sx, fy = 1 << sy).
+// fx = 1 << sx, fy = 1 << sy).  ol: the layout of out.
 template <int NPL, bool FIRST, bool PRO, typename BT, typename OutT>
 __global__ void __launch_bounds__(256) k_col_smooth(MgCoefs A, const float* __restrict__ P,
                                                     const float* __restrict__ E, const float* __restrict__ Q,
                                                     const BT* __restrict__ b, const float* __restrict__ s_old,
                                                     const float* __restrict__ e, float omega, int sx, int sy, Lay l,
-                                                    Lay cl, OutT* __restrict__ out, float deta,
+                                                    Lay cl, OutT* __restrict__ out, Lay ol, float deta,
                                                     const SolverScalars* sc) {
   if (sc && sc->done) return;
   const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -709,7 +516,7 @@ __global__ void __launch_bounds__(256) k_col_smooth(MgCoefs A, const float* __re
 #pragma unroll
   for (int u = 0; u < NPL; ++u) {
     const int k = NPL * lane + u;
-    if (k < l.nz) out[l.at32(i, j, k)] = (OutT)y[u];
+    if (k < l.nz) out[ol.at32(i, j, k)] = (OutT)y[u];
   }
 }
 
@@ -722,7 +529,7 @@ template <int NPL, typename BT, typename OutT>
 __global__ void __launch_bounds__(1024) k_coarse_solve(MgCoefs A, const float* __restrict__ P,
                                                        const float* __restrict__ E, const float* __restrict__ Q,
                                                        const BT* __restrict__ b, OutT* __restrict__ out, Lay l,
-                                                       float deta, int steps, const SolverScalars* sc) {
+                                                       Lay ol, float deta, int steps, const SolverScalars* sc) {
   if (sc && sc->done) return;
   extern __shared__ float lds[];
   const int nx = l.nx, nz = l.nz;
@@ -746,7 +553,7 @@ __global__ void __launch_bounds__(1024) k_coarse_solve(MgCoefs A, const float* _
           if (step + 1 < steps)
             nxt[k + nz * c] = y[u];
           else
-            out[l.at32(c % nx, c / nx, k)] = (OutT)y[u];
+            out[ol.at32(c % nx, c / nx, k)] = (OutT)y[u];
         }
       }
     }
@@ -756,76 +563,125 @@ __global__ void __launch_bounds__(1024) k_coarse_solve(MgCoefs A, const float* _
 
 Lay lay_of(const MgLevel& L) { return Lay{L.nx, L.ny, L.nz, L.zf}; }
 
+// The layout in which level L reads the coarse correction of level C: its
+// own.  (A z-fastest correction read by an x-fastest level's line step costs
+// a cache line per lane: 42 us against 27 for the first post-smoothing step
+// at 64 x 64 x 128; the coarse level's last smoothing step stores it across
+// instead.)
+Lay correction_layout(const MgLevel& L, const MgLevel& C) { return Lay{C.nx, C.ny, C.nz, L.zf}; }
+
 bool bf16_storage(const pcf_state* st) { return st->cfg.preconditioner_storage == PCF_STORAGE_BF16; }
 
-// out = s + deta (H s - sin) on an x-fastest level with FP32 coefficients
-// a32; the finest level reads its coefficients in the configured storage.
-template <typename SinT>
-void pc_rhs(pcf_state* st, float* const* a32, const uint16_t* const* a16, const float* s, float* out,
-            const SinT* sin, int nx, int ny, int nz, float deta, const SolverScalars* sc, const float* e = nullptr,
-            const MgLevel* F = nullptr, const MgLevel* C = nullptr) {
-  ProfScope prof(st, PCF_K_PC_RHS);
-  const bool quads = nx % 4 == 0;
-  const dim3 grd = quads ? dim3(blocks_for(nx, 64), blocks_for(ny, 16), nz)
-                         : dim3(blocks_for(nx, 64), blocks_for(ny, 4), nz);
-  const dim3 blk = quads ? dim3(16, 16) : dim3(64, 4);
-  auto go = [&](auto A) {
-    using CT = std::remove_const_t<std::remove_pointer_t<std::remove_reference_t<decltype(A.a[0])>>>;
-    A.s = s;
-    A.out = out;
-    A.nx = nx;
-    A.ny = ny;
-    A.nz = nz;
-    A.e = e;
-    A.omega = kMgOmega;
-    A.sx = F && F->fx == 2;
-    A.sy = F && F->fy == 2;
-    A.cl = C ? lay_of(*C) : Lay{1, 1, 1, false};
-    if (e) {
-      if (quads)
-        hipLaunchKernelGGL((k_pc_rhs32<4, SinT, CT, true>), grd, blk, 0, st->stream, A, sin, deta, sc);
-      else
-        hipLaunchKernelGGL((k_pc_rhs32<1, SinT, CT, true>), grd, blk, 0, st->stream, A, sin, deta, sc);
-    } else {
-      if (quads)
-        hipLaunchKernelGGL((k_pc_rhs32<4, SinT, CT>), grd, blk, 0, st->stream, A, sin, deta, sc);
-      else
-        hipLaunchKernelGGL((k_pc_rhs32<1, SinT, CT>), grd, blk, 0, st->stream, A, sin, deta, sc);
-    }
+constexpr int kLineMaxNz = 256;  // levels of k_line_step32's columns (taller ones: k_line_tall32)
+
+// f(W, NPL), the columns and levels per thread of a grid's line steps.  Eight
+// levels per thread up to 128 levels, 16 above (a block has at most 1024
+// threads).  Four columns per thread (16-byte loads, a quarter of the memory
+// instructions) pay where the tiles alone fill the chip: with bf16
+// coefficients 120 us against 125 at 256 x 256 x 128, but 30 against 28 at
+// 128 x 128 x 128 and 18 against 14 at 48 x 40 x 64, where the threads do.
+// The results do not depend on W.
+constexpr long long kLineWideCells = 4 << 20;
+template <class F>
+void with_line_shape(int nx, int ny, int nz, F&& f) {
+  using std::integral_constant;
+  if (nz > 128)
+    f(integral_constant<int, 1>{}, integral_constant<int, 16>{});
+  else if (nx % 4 == 0 && (long long)nx * ny * nz >= kLineWideCells)
+    f(integral_constant<int, 4>{}, integral_constant<int, 8>{});
+  else
+    f(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+}
+
+template <typename CT>
+LineArgs<CT> line_args(const MgLevel& L, const float* s, const float* e = nullptr, const MgLevel* C = nullptr) {
+  LineArgs<CT> A;
+  A.coefs = (const CT*)L.coefs;
+  A.factors = L.factors;
+  A.s = s;
+  A.nx = L.nx;
+  A.ny = L.ny;
+  A.nz = L.nz;
+  A.deta = L.deta;
+  A.e = e;
+  A.omega = kMgOmega;
+  A.sx = L.fx == 2;
+  A.sy = L.fy == 2;
+  A.cl = C ? (e ? correction_layout(L, *C) : lay_of(*C)) : Lay{1, 1, 1, false};
+  return A;
+}
+
+// One pseudo-time step of an x-fastest level: out = the line solve of
+// s + deta (H s - b), or of deta (0 - b) with FIRST; e (with the coarser
+// level C): s is s + omega P e.  out must differ from s.
+template <bool FIRST, typename BT, typename OutT>
+void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, OutT* out, const SolverScalars* sc,
+               const float* e = nullptr, const MgLevel* C = nullptr) {
+  ProfScope prof(st, FIRST ? PCF_K_PC_THOMAS : PCF_K_PC_RHS);
+  auto go = [&](auto ct, auto pro) {
+    constexpr bool PRO = decltype(pro)::value;
+    using CT = decltype(ct);
+    const LineArgs<CT> A = line_args<CT>(L, s, e, C);
+    const dim3 grd(line_tiles(L.nx, L.ny));
+    if (L.nz > kLineMaxNz)
+      hipLaunchKernelGGL((k_line_tall32<FIRST, PRO, CT, BT, OutT>), grd, dim3(kTileCols), 0, st->stream, A, b, out,
+                         L.col, sc);
+    else
+      with_line_shape(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
+        constexpr int W = decltype(w)::value, NPL = decltype(npl)::value;
+        const int threads = kTileCols / W * ((L.nz + NPL - 1) / NPL);
+        hipLaunchKernelGGL((k_line_step32<W, NPL, FIRST, PRO, CT, BT, OutT>), grd, dim3(threads),
+                           (line_lds<float, W>(threads)), st->stream, A, b, out, sc);
+      });
   };
-  if (a16 && bf16_storage(st)) {
-    PcArgs<uint16_t> A;
-    for (int t = 0; t < T_COUNT; ++t) A.a[t] = a16[t];
-    go(A);
+  if constexpr (FIRST) {
+    go(float{}, std::false_type{});
   } else {
-    PcArgs<float> A;
-    for (int t = 0; t < T_COUNT; ++t) A.a[t] = a32[t];
-    go(A);
+    auto pick = [&](auto ct) {
+      if (e) go(ct, std::true_type{});
+      else go(ct, std::false_type{});
+    };
+    if (bf16_storage(st)) pick(uint16_t{});
+    else pick(float{});
   }
 }
 
-__global__ void k_to_bf16(const float* a, uint16_t* b, size_t n) {
-  for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x) {
-    const unsigned u = __float_as_uint(a[q]);
-    b[q] = (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);  // round to nearest even
-  }
+// Pack a level's coefficients and factors for the line steps.
+template <typename SrcT>
+void line_pack(pcf_state* st, const MgLevel& L, const LineCoefs<SrcT>& A) {
+  const dim3 grd(line_tiles(L.nx, L.ny), blocks_for(L.nz, 4)), blk(kTileCols, 4);
+  if (bf16_storage(st))
+    hipLaunchKernelGGL((k_line_pack<SrcT, uint16_t, float>), grd, blk, 0, st->stream, A, (uint16_t*)L.coefs, L.factors,
+                       L.nx, L.ny, L.nz);
+  else
+    hipLaunchKernelGGL((k_line_pack<SrcT, float, float>), grd, blk, 0, st->stream, A, (float*)L.coefs, L.factors, L.nx,
+                       L.ny, L.nz);
 }
 
-// FP32 copies of the horizontal operator coefficients and of the line-solve
-// factors of the current operator.
+// The preconditioner's copies of the current operator: the packed
+// coefficients and line-solve factors of the levels smoothed by line steps,
+// and FP32 arrays of the multigrid's levels.
 int prepare_mixed(pcf_state* st) {
   if (st->t32_valid) return PCF_OK;
   int rc = pc_factors(st);
   if (rc) return rc;
   const size_t N = st->g.nv();
-  for (int t = 0; t < T_COUNT; ++t)
-    hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st->stream, st->T.a[t], st->T32[t], N);
-  if (bf16_storage(st))
+  const MgLevel& L0 = st->mg[0];
+  if (L0.coefs) {
+    LineCoefs<double> A;
+    for (int t = 0; t < T_COUNT; ++t) A.a[t] = st->T.a[t];
+    A.P = st->pc_P;
+    A.E = st->pc_E;
+    A.Q = st->pc_Q;
+    line_pack(st, L0, A);
+  }
+  if (L0.a[0]) {
     for (int t = 0; t < T_COUNT; ++t)
-      hipLaunchKernelGGL(k_to_bf16, dim3(1024), dim3(256), 0, st->stream, st->T32[t], st->T16[t], N);
-  hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st->stream, st->pc_P, st->pc32_P, N);
-  hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st->stream, st->pc_E, st->pc32_E, N);
-  hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st->stream, st->pc_Q, st->pc32_Q, N);
+      hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st->stream, st->T.a[t], L0.a[t], N);
+    hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st->stream, st->pc_P, L0.P, N);
+    hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st->stream, st->pc_E, L0.E, N);
+    hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, st->stream, st->pc_Q, L0.Q, N);
+  }
   // coarse operators and their line-solve factors
   for (size_t l = 1; l < st->mg.size(); ++l) {
     const MgLevel& F = st->mg[l - 1];
@@ -845,23 +701,25 @@ int prepare_mixed(pcf_state* st) {
       hipLaunchKernelGGL((k_mg_coarsen<1, 2>), grd, blk, 0, st->stream, fa, ca, fl, cl);
     hipLaunchKernelGGL(k_mg_factors, dim3(blocks_for((long long)C.nx * C.ny, 64)), dim3(64), 0, st->stream,
                        C.a[T_AC], C.a[T_AD], C.a[T_AU], C.P, C.E, C.Q, cl, C.deta);
-    if (C.a16[0])
-      for (int t = 0; t < T_COUNT; ++t)
-        hipLaunchKernelGGL(k_to_bf16, dim3(1024), dim3(256), 0, st->stream, C.a[t], C.a16[t], cl.count());
+    if (C.coefs) {
+      LineCoefs<float> A;
+      for (int t = 0; t < T_COUNT; ++t) A.a[t] = C.a[t];
+      A.P = C.P;
+      A.E = C.E;
+      A.Q = C.Q;
+      line_pack(st, C, A);
+    }
   }
   PCF_HIP(hipGetLastError());
   st->t32_valid = true;
   return PCF_OK;
 }
 
-// Level paths.  Levels with at most kColumnCols columns smooth with one
-// fused wavefront-per-column kernel per step; larger ones with the
-// row-parallel horizontal kernel and a line solve, the latter one wavefront
-// per column up to kScanCols columns and one thread per column beyond (where
-// the columns alone fill the chip).  The coarsest level runs all its steps
-// in one workgroup when it has at most 16 columns.
+// Level paths.  Levels with at most kColumnCols columns are stored z fastest
+// and smoothed one wavefront per column, larger ones x fastest by line steps.
+// The coarsest level runs all its steps in one workgroup when it has at most
+// 16 columns.
 constexpr size_t kColumnCols = 1024;
-constexpr size_t kScanCols = 4096;
 constexpr int kScanMaxNz = 512;
 constexpr size_t kCoarseLdsFloats = 16384;
 
@@ -886,26 +744,6 @@ MgCoefs coefs_of(const MgLevel& L) {
   return A;
 }
 
-// Line solve of a row-path level (FIRST: rhs = deta (0 - src)).
-template <bool FIRST, typename SrcT, typename OutT>
-void line_solve(pcf_state* st, const MgLevel& L, const SrcT* src, OutT* out, const SolverScalars* sc) {
-  ProfScope prof(st, PCF_K_PC_THOMAS);
-  const size_t nc = columns(L);
-  if (nc <= kScanCols && L.nz <= kScanMaxNz) {
-    with_npl(L.nz, [&](auto npl) {
-      hipLaunchKernelGGL((k_line_scan<decltype(npl)::value, FIRST, SrcT, OutT>), dim3(blocks_for(nc, 4)), dim3(256),
-                         0, st->stream, L.P, L.E, L.Q, src, out, (int)nc, L.nz, L.deta, sc);
-    });
-  } else {
-    if (nc >= kThomas32LdsColumns)
-      hipLaunchKernelGGL((k_pc_thomas32<FIRST, SrcT, OutT>), dim3(blocks_for(L.nx, 64), L.ny), dim3(64), 0,
-                         st->stream, L.P, L.E, L.Q, src, out, L.col, L.nx, L.ny, L.nz, L.deta, sc);
-    else
-      hipLaunchKernelGGL((k_pc_thomas32<FIRST, SrcT, OutT, 0>), dim3(blocks_for(L.nx, 64), L.ny), dim3(64), 0,
-                         st->stream, L.P, L.E, L.Q, src, out, L.col, L.nx, L.ny, L.nz, L.deta, sc);
-  }
-}
-
 // steps smoothing steps on level L.  s: the buffer holding the current
 // iterate, null to start from zero; e (with the coarser level C): the coarse
 // correction, s += omega P e before the first step.  The last step writes to
@@ -913,7 +751,7 @@ void line_solve(pcf_state* st, const MgLevel& L, const SrcT* src, OutT* out, con
 // the buffer holding the result.
 template <typename BT>
 float* mg_smooth(pcf_state* st, const MgLevel& L, const BT* b, float* s, const float* e, const MgLevel* C, int steps,
-                 double* out64, const SolverScalars* sc) {
+                 double* out64, const Lay& ol, const SolverScalars* sc) {
   const bool col = column_path(L);
   const size_t nc = columns(L);
   int step = 0;
@@ -926,24 +764,22 @@ float* mg_smooth(pcf_state* st, const MgLevel& L, const BT* b, float* s, const f
         const Lay l = lay_of(L);
         if (last && out64)
           hipLaunchKernelGGL((k_col_smooth<NPL, true, false, BT, double>), dim3(blocks_for(nc, 4)), dim3(256), 0,
-                             st->stream, coefs_of(L), L.P, L.E, L.Q, b, nullptr, nullptr, 0.0f, 0, 0, l, l, out64,
+                             st->stream, coefs_of(L), L.P, L.E, L.Q, b, nullptr, nullptr, 0.0f, 0, 0, l, l, out64, l,
                              L.deta, sc);
         else
           hipLaunchKernelGGL((k_col_smooth<NPL, true, false, BT, float>), dim3(blocks_for(nc, 4)), dim3(256), 0,
                              st->stream, coefs_of(L), L.P, L.E, L.Q, b, nullptr, nullptr, 0.0f, 0, 0, l, l, L.s,
-                             L.deta, sc);
+                             last ? ol : l, L.deta, sc);
       });
     } else {
       if (last && out64)
-        line_solve<true>(st, L, b, out64, sc);
+        line_step<true, BT, double>(st, L, b, nullptr, out64, sc);
       else
-        line_solve<true>(st, L, b, L.s, sc);
+        line_step<true, BT, float>(st, L, b, nullptr, L.s, sc);
     }
     s = L.s;
     step = 1;
   }
-  // the row path adds the coarse correction in its first horizontal kernel
-  const int first_post = step;
   for (; step < steps; ++step) {
     const bool last = step == steps - 1;
     if (col) {
@@ -953,34 +789,36 @@ float* mg_smooth(pcf_state* st, const MgLevel& L, const BT* b, float* s, const f
       with_npl(L.nz, [&](auto npl) {
         constexpr int NPL = decltype(npl)::value;
         const int sx = L.fx == 2, sy = L.fy == 2;
-        const Lay l = lay_of(L), cl = C ? lay_of(*C) : l;
+        const Lay l = lay_of(L), cl = C ? correction_layout(L, *C) : l;
         const dim3 g(blocks_for(nc, 4)), blk(256);
         if (last && out64) {
           if (pro)
             hipLaunchKernelGGL((k_col_smooth<NPL, false, true, BT, double>), g, blk, 0, st->stream, coefs_of(L), L.P,
-                               L.E, L.Q, b, s, e, kMgOmega, sx, sy, l, cl, out64, L.deta, sc);
+                               L.E, L.Q, b, s, e, kMgOmega, sx, sy, l, cl, out64, l, L.deta, sc);
           else
             hipLaunchKernelGGL((k_col_smooth<NPL, false, false, BT, double>), g, blk, 0, st->stream, coefs_of(L), L.P,
-                               L.E, L.Q, b, s, e, kMgOmega, sx, sy, l, cl, out64, L.deta, sc);
+                               L.E, L.Q, b, s, e, kMgOmega, sx, sy, l, cl, out64, l, L.deta, sc);
         } else {
           if (pro)
             hipLaunchKernelGGL((k_col_smooth<NPL, false, true, BT, float>), g, blk, 0, st->stream, coefs_of(L), L.P,
-                               L.E, L.Q, b, s, e, kMgOmega, sx, sy, l, cl, dst, L.deta, sc);
+                               L.E, L.Q, b, s, e, kMgOmega, sx, sy, l, cl, dst, last ? ol : l, L.deta,
+                               sc);
           else
             hipLaunchKernelGGL((k_col_smooth<NPL, false, false, BT, float>), g, blk, 0, st->stream, coefs_of(L), L.P,
-                               L.E, L.Q, b, s, e, kMgOmega, sx, sy, l, cl, dst, L.deta, sc);
+                               L.E, L.Q, b, s, e, kMgOmega, sx, sy, l, cl, dst, last ? ol : l, L.deta,
+                               sc);
         }
       });
       s = dst;
       continue;
     }
-    pc_rhs<BT>(st, L.a, L.a16[0] ? L.a16 : nullptr, s, L.rhs, b, L.nx, L.ny, L.nz, L.deta, sc,
-               step == first_post ? e : nullptr, &L, C);
+    const float* pro = step == 0 ? e : nullptr;
+    float* dst = s == L.s ? L.rhs : L.s;
     if (last && out64)
-      line_solve<false>(st, L, (const float*)L.rhs, out64, sc);
+      line_step<false, BT, double>(st, L, b, s, out64, sc, pro, C);
     else
-      line_solve<false>(st, L, (const float*)L.rhs, L.s, sc);
-    s = L.s;
+      line_step<false, BT, float>(st, L, b, s, dst, sc, pro, C);
+    s = dst;
   }
   return s;
 }
@@ -990,22 +828,21 @@ template <typename BT>
 void mg_restrict(pcf_state* st, const MgLevel& L, const MgLevel& C, const BT* b, const float* s,
                  const SolverScalars* sc) {
   ProfScope prof(st, PCF_K_PC_RHS);
-  const MgCoefs A = coefs_of(L);
-  if (!column_path(L) && L.fx == 2 && L.fy == 2 && L.nx % 4 == 0) {
-    const dim3 grd(blocks_for(L.nx, 64), blocks_for(L.ny, 16), L.nz), blk(16, 16);
-    if (L.a16[0] && bf16_storage(st)) {
-      Coefs<uint16_t> A16;
-      for (int t = 0; t < T_COUNT; ++t) A16.a[t] = L.a16[t];
-      hipLaunchKernelGGL((k_resid_restrict4<BT, uint16_t>), grd, blk, 0, st->stream, A16, b, s, C.b, L.nx, L.ny,
-                         L.nz, lay_of(C), sc);
-    } else {
-      Coefs<float> A32;
-      for (int t = 0; t < T_COUNT; ++t) A32.a[t] = L.a[t];
-      hipLaunchKernelGGL((k_resid_restrict4<BT, float>), grd, blk, 0, st->stream, A32, b, s, C.b, L.nx, L.ny, L.nz,
-                         lay_of(C), sc);
-    }
+  if (L.coefs && L.fx == 2 && L.fy == 2 && L.nz <= kLineMaxNz) {
+    auto go = [&](auto ct) {
+      using CT = decltype(ct);
+      with_line_shape(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
+        constexpr int W = decltype(w)::value, NPL = decltype(npl)::value;
+        hipLaunchKernelGGL((k_resid_restrict<W, NPL, BT, CT>), dim3(line_tiles(L.nx, L.ny)),
+                           dim3(kTileCols / W * ((L.nz + NPL - 1) / NPL)), 0, st->stream,
+                           line_args<CT>(L, s, nullptr, &C), b, C.b, sc);
+      });
+    };
+    if (bf16_storage(st)) go(uint16_t{});
+    else go(float{});
     return;
   }
+  const MgCoefs A = coefs_of(L);
   float* r = L.col;  // the line-solve scratch is free here
   const Lay fl = lay_of(L), cl = lay_of(C);
   hipLaunchKernelGGL((k_mg_resid<BT>), dim3(blocks_for(fl.count(), 256)), dim3(256), 0, st->stream, A, b, s, r, fl,
@@ -1021,7 +858,8 @@ void mg_restrict(pcf_state* st, const MgLevel& L, const MgLevel& C, const BT* b,
 
 // The coarsest level: mg_coarse_steps smoothing steps from zero.
 template <typename BT>
-float* mg_coarsest(pcf_state* st, const MgLevel& L, const BT* b, double* out64, const SolverScalars* sc) {
+float* mg_coarsest(pcf_state* st, const MgLevel& L, const BT* b, double* out64, const Lay& ol,
+                   const SolverScalars* sc) {
   const size_t nc = columns(L);
   const size_t n = nc * (size_t)L.nz;
   if (nc <= 16 && L.nz <= 256 && 2 * n <= kCoarseLdsFloats) {
@@ -1033,28 +871,30 @@ float* mg_coarsest(pcf_state* st, const MgLevel& L, const BT* b, double* out64, 
       if constexpr (NPL <= 4) {
         if (out64)
           hipLaunchKernelGGL((k_coarse_solve<NPL, BT, double>), dim3(1), blk, lds, st->stream, coefs_of(L), L.P, L.E,
-                             L.Q, b, out64, lay_of(L), L.deta, st->cfg.mg_coarse_steps, sc);
+                             L.Q, b, out64, lay_of(L), lay_of(L), L.deta, st->cfg.mg_coarse_steps, sc);
         else
           hipLaunchKernelGGL((k_coarse_solve<NPL, BT, float>), dim3(1), blk, lds, st->stream, coefs_of(L), L.P, L.E,
-                             L.Q, b, L.s, lay_of(L), L.deta, st->cfg.mg_coarse_steps, sc);
+                             L.Q, b, L.s, lay_of(L), ol, L.deta, st->cfg.mg_coarse_steps, sc);
       }
     });
     return L.s;
   }
-  return mg_smooth<BT>(st, L, b, nullptr, nullptr, nullptr, st->cfg.mg_coarse_steps, out64, sc);
+  return mg_smooth<BT>(st, L, b, nullptr, nullptr, nullptr, st->cfg.mg_coarse_steps, out64, ol, sc);
 }
 
 // One V-cycle on level l for the right-hand side b; the finest level writes
-// its result to out64; returns the buffer holding the level's result.
+// its result to out64; returns the buffer holding the level's result, in
+// layout ol.
 template <typename BT>
-float* mg_vcycle(pcf_state* st, size_t l, const BT* b, double* out64, const SolverScalars* sc) {
+float* mg_vcycle(pcf_state* st, size_t l, const BT* b, double* out64, const Lay& ol, const SolverScalars* sc) {
   const MgLevel& L = st->mg[l];
-  if (l + 1 == st->mg.size()) return mg_coarsest<BT>(st, L, b, out64, sc);
+  if (l + 1 == st->mg.size()) return mg_coarsest<BT>(st, L, b, out64, ol, sc);
   const MgLevel& C = st->mg[l + 1];
-  float* s = mg_smooth<BT>(st, L, b, nullptr, nullptr, nullptr, st->cfg.mg_smoothing_steps, nullptr, sc);
+  float* s = mg_smooth<BT>(st, L, b, nullptr, nullptr, nullptr, st->cfg.mg_smoothing_steps, nullptr, lay_of(L), sc);
   mg_restrict<BT>(st, L, C, b, s, sc);
-  const float* e = mg_vcycle<float>(st, l + 1, C.b, nullptr, sc);
-  return mg_smooth<BT>(st, L, b, s, e, &C, st->cfg.mg_smoothing_steps, out64, sc);
+  const Lay el = correction_layout(L, C);
+  const float* e = mg_vcycle<float>(st, l + 1, C.b, nullptr, el, sc);
+  return mg_smooth<BT>(st, L, b, s, e, &C, st->cfg.mg_smoothing_steps, out64, ol, sc);
 }
 
 }  // namespace
@@ -1064,39 +904,24 @@ int precondition_mixed(pcf_state* st, const double* sin, double* sout, const Sol
   int rc = prepare_mixed(st);
   if (rc) return rc;
   if (st->cfg.preconditioner_type == PCF_PC_MULTIGRID) {
-    mg_vcycle<double>(st, 0, sin, sout, sc);
+    mg_vcycle<double>(st, 0, sin, sout, lay_of(st->mg[0]), sc);
     PCF_HIP(hipGetLastError());
     return PCF_OK;
   }
-  const Geo& g = st->g;
-  const dim3 tgrd(blocks_for(g.nx, 64), g.ny), tblk(64);
-  const float deta = (float)st->deta;
+  const MgLevel& L = st->mg[0];
   const int iters = st->cfg.preconditioner_iterations;
-  float* col = st->m_pc_tmp;  // upward-sweep scratch of the line solves
-  float* cur = st->m_pc_cur;  // FP32 iterate between pseudo-time steps
-  float* rhs = st->m_pc_rhs;  // FP32 right-hand side of a later pseudo-time step
-  {
-    ProfScope prof(st, PCF_K_PC_THOMAS);
-    if (iters == 1)
-      hipLaunchKernelGGL((k_pc_thomas32<true, double, double>), tgrd, tblk, 0, st->stream, st->pc32_P, st->pc32_E,
-                         st->pc32_Q, sin, sout, col, g.nx, g.ny, g.nz, deta, sc);
-    else
-      hipLaunchKernelGGL((k_pc_thomas32<true, double, float>), tgrd, tblk, 0, st->stream, st->pc32_P, st->pc32_E,
-                         st->pc32_Q, sin, cur, col, g.nx, g.ny, g.nz, deta, sc);
-  }
-  for (int it = 2; it <= iters; ++it) {
-    {
-      ProfScope prof(st, PCF_K_PC_RHS);
-      pc_rhs<double>(st, st->T32, st->T16[0] ? st->T16 : nullptr, cur, rhs, sin, g.nx, g.ny, g.nz, deta, sc);
-    }
-    {
-      ProfScope prof(st, PCF_K_PC_THOMAS);
+  if (iters == 1) {
+    line_step<true, double, double>(st, L, sin, nullptr, sout, sc);
+  } else {
+    float* cur = L.s;  // FP32 iterate between pseudo-time steps
+    line_step<true, double, float>(st, L, sin, nullptr, cur, sc);
+    for (int it = 2; it <= iters; ++it) {
+      float* next = cur == L.s ? L.rhs : L.s;
       if (it == iters)
-        hipLaunchKernelGGL((k_pc_thomas32<false, float, double>), tgrd, tblk, 0, st->stream, st->pc32_P, st->pc32_E,
-                           st->pc32_Q, rhs, sout, col, g.nx, g.ny, g.nz, deta, sc);
+        line_step<false, double, double>(st, L, sin, cur, sout, sc);
       else
-        hipLaunchKernelGGL((k_pc_thomas32<false, float, float>), tgrd, tblk, 0, st->stream, st->pc32_P, st->pc32_E,
-                           st->pc32_Q, rhs, cur, col, g.nx, g.ny, g.nz, deta, sc);
+        line_step<false, double, float>(st, L, sin, cur, next, sc);
+      cur = next;
     }
   }
   PCF_HIP(hipGetLastError());
@@ -1156,8 +981,8 @@ int apply_bicgstab_mixed(pcf_state* st, double tolref, double dt, int* niter_out
 // ---------------------------------------------------------------------------
 // Ensemble batch: the FP32 line preconditioner over the solves of a batched
 // iteration (see the ensemble kernels of poisson.hip).  Each member runs the
-// blocks of its single solve's kernels (precondition_mixed; x_size a
-// multiple of 4).
+// line steps of its single solve (precondition_mixed), with the same segments
+// and so the same bits.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -1171,92 +996,85 @@ __device__ __forceinline__ int ens_member32(const int* start, int count, int b) 
   return lo;
 }
 
-// FIRST: from the FP64 vector v[in]; else from the member's FP32 rhs.
-// OutT double: to v[out]; float: to the member's FP32 iterate.
-template <bool FIRST, typename OutT>
-__global__ void __launch_bounds__(64) kEm_thomas(const EnsTable* __restrict__ E, const EnsList* __restrict__ L, int in,
-                                                 int out) {
-  const int a = ens_member32(L->thomas_start, L->count, blockIdx.x);
+// One pseudo-time step of every solve: from the FP64 vector v[in] (FIRST) or
+// the member's FP32 iterate `from` (0: cur32, 1: rhs32), to v[out] (OutT
+// double) or the other FP32 buffer.  The members' columns may have different
+// heights: the segments beyond a column's top are identity maps.
+template <bool FIRST, typename CT, typename OutT>
+__global__ void __launch_bounds__(1024) kEm_line(const EnsTable* __restrict__ E, const EnsList* __restrict__ L, int in,
+                                                 int from, int out) {
+  const int a = ens_member32(L->line_start, L->count, blockIdx.x);
   const EnsMember& M = E->m[L->member[a]];
   if (M.sc->done) return;
-  const int b = blockIdx.x - L->thomas_start[a];
-  const int gx = (M.nx + 63) / 64;
-  OutT* dst;
-  if constexpr (sizeof(OutT) == 8) dst = M.v[out];
-  else dst = M.cur32;
-  const float deta = (float)M.deta;
-  if constexpr (FIRST)
-    pc_thomas32<true, double, OutT>(M.P32, M.E32, M.Q32, (const double*)M.v[in], dst, M.col32, M.nx, M.ny, M.nz,
-                                    deta, b % gx, b / gx);
-  else
-    pc_thomas32<false, float, OutT>(M.P32, M.E32, M.Q32, (const float*)M.rhs32, dst, M.col32, M.nx, M.ny, M.nz,
-                                    deta, b % gx, b / gx);
-}
-
-// rhs32 = cur32 + deta (H cur32 - v[in]) with the coefficients in storage CT
-template <typename CT>
-__global__ void __launch_bounds__(256) kEm_rhs(const EnsTable* __restrict__ E, const EnsList* __restrict__ L, int in) {
-  const int a = ens_member32(L->rhs32_start, L->count, blockIdx.x);
-  const EnsMember& M = E->m[L->member[a]];
-  if (M.sc->done) return;
-  const int b = blockIdx.x - L->rhs32_start[a];
-  const int gx = (M.nx + 63) / 64, gy = (M.ny + 15) / 16;
-  PcArgs<CT> A;
-  for (int t = 0; t < T_COUNT; ++t) {
-    if constexpr (sizeof(CT) == 2) A.a[t] = M.T16[t];
-    else A.a[t] = M.T32[t];
-  }
-  A.s = M.cur32;
-  A.out = M.rhs32;
+  const int b = blockIdx.x - L->line_start[a];
+  LineArgs<CT> A;
+  A.coefs = (const CT*)M.coefs32;
+  A.factors = M.factors32;
+  A.s = from == 0 ? M.cur32 : M.rhs32;
   A.nx = M.nx;
   A.ny = M.ny;
   A.nz = M.nz;
+  A.deta = (float)M.deta;
   A.e = nullptr;
   A.omega = 0.0f;
   A.sx = A.sy = 0;
   A.cl = Lay{1, 1, 1, false};
-  pc_rhs32<4, double, CT>(A, (const double*)M.v[in], (float)M.deta, b % gx, (b / gx) % gy, b / (gx * gy));
+  OutT* dst;
+  if constexpr (sizeof(OutT) == 8) dst = M.v[out];
+  else dst = FIRST || from == 1 ? M.cur32 : M.rhs32;
+  const double* v = M.v[in];
+  if (M.nz > 128)
+    line_step32<1, 16, FIRST, false, CT, double, OutT>(A, v, dst, b);
+  else
+    line_step32<1, 8, FIRST, false, CT, double, OutT>(A, v, dst, b);
 }
 
 }  // namespace
 
-int ensemble_rhs32_blocks(const pcf_state* st) {
-  if (st->cfg.precision != PCF_PRECISION_MIXED) return 0;
-  const Geo& g = st->g;
-  return (int)(blocks_for(g.nx, 64) * blocks_for(g.ny, 16) * g.nz);
+// blocks and threads per block of a member's line steps
+int ensemble_line_blocks(const pcf_state* st) { return line_tiles(st->g.nx, st->g.ny); }
+int ensemble_line_threads(const pcf_state* st) {
+  const int npl = st->g.nz > 128 ? 16 : 8;
+  return kTileCols * ((st->g.nz + npl - 1) / npl);
 }
+bool ensemble_line_covers(const pcf_state* st) { return st->g.nz <= kLineMaxNz; }
 
 // M^-1 v[in] -> v[out] for every solve of the list (precondition_mixed's
-// line branch)
-void ensemble_precondition_mixed(hipStream_t s, const EnsTable* dT, const EnsList* dL, const EnsList& L, int iters,
-                                 bool bf16, int in, int out) {
-  const int tb = L.thomas_start[L.count], rb = L.rhs32_start[L.count];
+// line branch); threads: the largest of the members' blocks
+void ensemble_precondition_mixed(hipStream_t s, const EnsTable* dT, const EnsList* dL, const EnsList& L, int threads,
+                                 int iters, bool bf16, int in, int out) {
+  const dim3 grd(L.line_start[L.count]), blk(threads);
+  const unsigned lds = 4 * threads * sizeof(float);
   if (iters == 1) {
-    hipLaunchKernelGGL((kEm_thomas<true, double>), dim3(tb), dim3(64), 0, s, dT, dL, in, out);
+    hipLaunchKernelGGL((kEm_line<true, float, double>), grd, blk, lds, s, dT, dL, in, 0, out);
     return;
   }
-  hipLaunchKernelGGL((kEm_thomas<true, float>), dim3(tb), dim3(64), 0, s, dT, dL, in, out);
-  for (int it = 2; it <= iters; ++it) {
-    if (bf16) hipLaunchKernelGGL(kEm_rhs<uint16_t>, dim3(rb), dim3(16, 16), 0, s, dT, dL, in);
-    else hipLaunchKernelGGL(kEm_rhs<float>, dim3(rb), dim3(16, 16), 0, s, dT, dL, in);
-    if (it == iters) hipLaunchKernelGGL((kEm_thomas<false, double>), dim3(tb), dim3(64), 0, s, dT, dL, in, out);
-    else hipLaunchKernelGGL((kEm_thomas<false, float>), dim3(tb), dim3(64), 0, s, dT, dL, in, out);
+  hipLaunchKernelGGL((kEm_line<true, float, float>), grd, blk, lds, s, dT, dL, in, 0, out);
+  int from = 0;
+  for (int it = 2; it <= iters; ++it, from ^= 1) {
+    if (it == iters && bf16)
+      hipLaunchKernelGGL((kEm_line<false, uint16_t, double>), grd, blk, lds, s, dT, dL, in, from, out);
+    else if (it == iters)
+      hipLaunchKernelGGL((kEm_line<false, float, double>), grd, blk, lds, s, dT, dL, in, from, out);
+    else if (bf16)
+      hipLaunchKernelGGL((kEm_line<false, uint16_t, float>), grd, blk, lds, s, dT, dL, in, from, out);
+    else
+      hipLaunchKernelGGL((kEm_line<false, float, float>), grd, blk, lds, s, dT, dL, in, from, out);
   }
 }
 
 // Allocation of the mixed-precision buffers (pcf_create, precision MIXED).
 int alloc_mixed(pcf_state* st) {
   const size_t N = st->g.nv();
+  const bool multigrid = st->cfg.preconditioner_type == PCF_PC_MULTIGRID;
   auto af = [&](float** p) -> int { return device_alloc(st, p, N); };
+  // the packed arrays of a level smoothed by line steps
+  auto packed = [&](MgLevel& L) -> int {
+    const size_t n = (size_t)line_tiles(L.nx, L.ny) * kTileCols * L.nz;
+    int rc1 = device_alloc(st, &L.coefs, n * T_COUNT * (bf16_storage(st) ? 2 : 4));
+    return rc1 ? rc1 : device_alloc(st, &L.factors, 3 * n);
+  };
   int rc;
-  for (int t = 0; t < T_COUNT; ++t)
-    if ((rc = af(&st->T32[t]))) return rc;
-  if (st->cfg.preconditioner_storage == PCF_STORAGE_BF16)
-    for (int t = 0; t < T_COUNT; ++t)
-      if ((rc = device_alloc(st, &st->T16[t], N))) return rc;
-  float** fl[] = {&st->pc32_P, &st->pc32_E, &st->pc32_Q, &st->m_pc_tmp, &st->m_pc_cur, &st->m_pc_rhs};
-  for (float** p : fl)
-    if ((rc = af(p))) return rc;
   double** dl[] = {&st->bzpc, &st->m_prev[0], &st->m_prev[1]};
   for (double** p : dl)
     if ((rc = device_alloc(st, p, N))) return rc;
@@ -1265,26 +1083,26 @@ int alloc_mixed(pcf_state* st) {
     for (double** p : el)
       if ((rc = device_alloc(st, p, N))) return rc;
   }
-  if (st->cfg.preconditioner_type != PCF_PC_MULTIGRID) return PCF_OK;
-  // level 0 works on the buffers above; coarser levels get their own
+  // level 0, the only one of the line relaxation
   const Geo& g = st->g;
   MgLevel L0;
   L0.nx = g.nx;
   L0.ny = g.ny;
   L0.nz = g.nz;
   L0.deta = (float)st->deta;
-  for (int t = 0; t < T_COUNT; ++t) {
-    L0.a[t] = st->T32[t];
-    L0.a16[t] = st->T16[t];
+  for (float** p : {&L0.s, &L0.rhs, &L0.col})
+    if ((rc = af(p))) return rc;
+  if (!multigrid || !column_path(L0))
+    if ((rc = packed(L0))) return rc;
+  if (multigrid) {
+    for (int t = 0; t < T_COUNT; ++t)
+      if ((rc = af(&L0.a[t]))) return rc;
+    for (float** p : {&L0.P, &L0.E, &L0.Q})
+      if ((rc = af(p))) return rc;
   }
-  L0.P = st->pc32_P;
-  L0.E = st->pc32_E;
-  L0.Q = st->pc32_Q;
-  L0.s = st->m_pc_cur;
-  L0.rhs = st->m_pc_rhs;
-  L0.col = st->m_pc_tmp;
   st->mg.clear();
   st->mg.push_back(L0);
+  if (!multigrid) return PCF_OK;
   // the coarse levels' "grid spacings": Galerkin aggregation of fx x fy
   // columns multiplies the x couplings by fy and the y couplings by fx, which
   // sets the pseudo-time step of each level's smoother like the reference's
@@ -1312,9 +1130,7 @@ int alloc_mixed(pcf_state* st) {
     for (float** p : v)
       if ((rc = ac(p))) return rc;
     C.zf = column_path(C);  // coarse levels smoothed column by column: z fastest
-    if (!C.zf && st->cfg.preconditioner_storage == PCF_STORAGE_BF16)
-      for (int t = 0; t < T_COUNT; ++t)
-        if ((rc = device_alloc(st, &C.a16[t], Nc))) return rc;
+    if (!C.zf && (rc = packed(C))) return rc;
     st->mg.push_back(C);
   }
   return PCF_OK;

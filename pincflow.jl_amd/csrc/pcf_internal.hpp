@@ -82,7 +82,10 @@ struct MgLevel {
   bool zf = false;  // arrays stored z fastest (else x fastest)
   float deta = 0.0f;
   float* a[T_COUNT] = {};
-  uint16_t* a16[T_COUNT] = {};  // bf16 copies read by the row kernels (storage BF16)
+  // levels smoothed by line steps: packed coefficients (float or bf16 bits)
+  // and line-solve factors (k_line_pack)
+  char* coefs = nullptr;
+  float* factors = nullptr;
   float *P = nullptr, *E = nullptr, *Q = nullptr;
   float *b = nullptr, *s = nullptr, *rhs = nullptr, *col = nullptr;
 };
@@ -128,10 +131,9 @@ struct EnsMember {
   Tensor T;                         // FP64 operator
   double* v[EV_COUNT];
   const double *P, *E, *Q;          // FP64 line-solve factors
-  const float *P32, *E32, *Q32;     // mixed: FP32 factors, coefficients and work
-  const float* T32[T_COUNT];
-  const uint16_t* T16[T_COUNT];     // bf16 storage (else null)
-  float *col32, *cur32, *rhs32;
+  const char* coefs32;              // mixed: packed coefficients and factors, FP32 iterates
+  const float* factors32;
+  float *cur32, *rhs32;
   double* partials;
   SolverScalars* sc;
   size_t n;                         // cells
@@ -153,8 +155,7 @@ struct EnsList {
   int count;
   int member[kEnsMax];
   int pair_start[kEnsMax + 1];      // apply and pc-rhs grids
-  int thomas_start[kEnsMax + 1];    // line-solve grids
-  int rhs32_start[kEnsMax + 1];     // FP32 pc-rhs grid (mixed)
+  int line_start[kEnsMax + 1];      // line-solve grids
 };
 
 // ---------------------------------------------------------------------------
@@ -194,7 +195,7 @@ struct pcf_ensemble {
     std::vector<pcf_state*> active;      // solves in the batch
     pcf::EnsTable* table = nullptr;
     std::unique_ptr<pcf::EnsTable> host;
-    std::vector<int> pair_blocks, thomas_blocks, rhs32_blocks;
+    std::vector<int> pair_blocks, line_blocks, line_threads;
     pcf::EnsList* list_host = nullptr;   // pinned, two slots
     pcf::EnsList* list = nullptr;
   };
@@ -277,15 +278,10 @@ struct pcf_state {
   double *pc_P, *pc_E, *pc_Q;         // line-solve factors of the current operator
   bool pc_factors_valid = false;
   // mixed precision (allocated when cfg.precision == PCF_PRECISION_MIXED):
-  // FP32 copies of the 22 horizontal operator coefficients and of the
-  // line-solve factors, FP32 preconditioner work, and z = M^-1 s
-  float* T32[pcf::T_COUNT] = {};
-  uint16_t* T16[pcf::T_COUNT] = {};   // bf16 bits of T32 (preconditioner_storage BF16)
-  float *pc32_P = nullptr, *pc32_E = nullptr, *pc32_Q = nullptr;
-  float *m_pc_tmp = nullptr, *m_pc_cur = nullptr, *m_pc_rhs = nullptr;
+  // the preconditioner's levels (mg below) and z = M^-1 s
   double* bzpc = nullptr;
   bool t32_valid = false;
-  std::vector<pcf::MgLevel> mg;       // multigrid levels (level 0 aliases the buffers above)
+  std::vector<pcf::MgLevel> mg;       // the FP32 preconditioner's levels (one for line relaxation)
   // warm start of the mixed solve: solution / dt of each implicit stage of
   // the previous time step (slot 0: first stage, 1: second stage)
   double* m_prev[2] = {nullptr, nullptr};
@@ -418,10 +414,13 @@ int dot(pcf_state* st, const double* a, const double* b, double* out);
 // ---- mixed.hip -------------------------------------------------------------
 int apply_bicgstab_mixed(pcf_state* st, double tolref, double dt, int* niter);
 int precondition_mixed(pcf_state* st, const double* sin, double* sout, const SolverScalars* sc);
-// the ensemble batch's FP32 line preconditioner and its pc-rhs grid per member
-int ensemble_rhs32_blocks(const pcf_state* st);
-void ensemble_precondition_mixed(hipStream_t s, const EnsTable* dT, const EnsList* dL, const EnsList& L, int iters,
-                                 bool bf16, int in, int out);
+// the ensemble batch's FP32 line preconditioner: a member's grid, whether it
+// covers the member, and the launches over a list (threads: the largest block)
+int ensemble_line_blocks(const pcf_state* st);
+int ensemble_line_threads(const pcf_state* st);
+bool ensemble_line_covers(const pcf_state* st);
+void ensemble_precondition_mixed(hipStream_t s, const EnsTable* dT, const EnsList* dL, const EnsList& L, int threads,
+                                 int iters, bool bf16, int in, int out);
 int alloc_mixed(pcf_state* st);
 // Device buffer of `bytes` owned by the state (freed by pcf_destroy).  The
 // start of the n-th buffer is offset by (n mod 28) x 2304 B within its

@@ -8,6 +8,7 @@
 // one-block finalize kernel sums the partials in a fixed order and leaves the
 // BiCGSTAB scalars (alpha, omega, beta, residual, convergence flag) in device
 // memory, so an iteration needs no host round trip.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -1047,10 +1048,10 @@ __device__ __forceinline__ int ens_find(const int* start, int count, int b) {
 template <bool FIRST>
 __global__ void __launch_bounds__(64) kE_thomas(const EnsTable* __restrict__ E, const EnsList* __restrict__ L,
                                                 int src, int out) {
-  const int a = ens_find(L->thomas_start, L->count, blockIdx.x);
+  const int a = ens_find(L->line_start, L->count, blockIdx.x);
   const EnsMember& M = E->m[L->member[a]];
   if (M.sc->done) return;
-  const int b = blockIdx.x - L->thomas_start[a];
+  const int b = blockIdx.x - L->line_start[a];
   const int gx = (M.nx + 63) / 64;
   pc_thomas<FIRST, 64>(M.P, M.E, M.Q, M.v[src], M.v[out], M.nx, M.ny, M.nz, M.deta, b % gx, b / gx);
 }
@@ -1576,14 +1577,14 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
 // ---------------------------------------------------------------------------
 
 // The member table covers the line preconditioner (FP64, or FP32 in the
-// mixed solve) on grids with an even x_size (the two-cell apply kernels; a
-// multiple of 4 for the FP32 pc-rhs kernel).  Members with the same key
+// mixed solve) on grids with an even x_size (the two-cell apply kernels; in
+// the mixed solve columns the line steps cover).  Members with the same key
 // share a table; -1: not covered.
 int ensemble_key(const pcf_state* st) {
   const pcf_config& n = st->cfg;
   const bool mixed = n.precision == PCF_PRECISION_MIXED;
   if (n.preconditioner == 0 || !use_pairs(st->g)) return -1;
-  if (mixed && (n.preconditioner_type == PCF_PC_MULTIGRID || st->g.nx % 4 != 0)) return -1;
+  if (mixed && (n.preconditioner_type == PCF_PC_MULTIGRID || !ensemble_line_covers(st))) return -1;
   const int bf16 = mixed && n.preconditioner_storage == PCF_STORAGE_BF16 ? 1 : 0;
   return (mixed ? 1 : 0) | bf16 << 1 | n.preconditioner_iterations << 2;
 }
@@ -1598,7 +1599,7 @@ bool ensemble_batchable(const pcf_state* st, bool mixed, bool stage) {
 // preconditioner; the pseudo-time steps and buffers of precondition())
 static void ensemble_precondition(hipStream_t s, const EnsTable* dT, const EnsList* dL, const EnsList& L, int iters,
                                   int in, int out) {
-  const int tb = L.thomas_start[L.count], pb = L.pair_start[L.count];
+  const int tb = L.line_start[L.count], pb = L.pair_start[L.count];
   int cur = iters == 1 ? out : EV_PCTMP;
   hipLaunchKernelGGL(kE_thomas<true>, dim3(tb), dim3(64), 0, s, dT, dL, in, cur);
   for (int it = 2; it <= iters; ++it) {
@@ -1614,8 +1615,9 @@ static void ensemble_fill(pcf_ensemble::Group& grp) {
   const std::vector<pcf_state*>& mem = grp.slots;
   H.count = (int)mem.size();
   grp.pair_blocks.assign(H.count, 0);
-  grp.thomas_blocks.assign(H.count, 0);
-  grp.rhs32_blocks.assign(H.count, 0);
+  grp.line_blocks.assign(H.count, 0);
+  grp.line_threads.assign(H.count, 0);
+  const bool mixed = (grp.key & 1) != 0;
   for (int q = 0; q < H.count; ++q) {
     pcf_state* st = mem[q];
     const Geo& g = st->g;
@@ -1628,16 +1630,13 @@ static void ensemble_fill(pcf_ensemble::Group& grp) {
     M.P = st->pc_P;
     M.E = st->pc_E;
     M.Q = st->pc_Q;
-    M.P32 = st->pc32_P;
-    M.E32 = st->pc32_E;
-    M.Q32 = st->pc32_Q;
-    for (int t = 0; t < T_COUNT; ++t) {
-      M.T32[t] = st->T32[t];
-      M.T16[t] = st->T16[t];
+    if (mixed) {
+      const MgLevel& L0 = st->mg[0];
+      M.coefs32 = L0.coefs;
+      M.factors32 = L0.factors;
+      M.cur32 = L0.s;
+      M.rhs32 = L0.rhs;
     }
-    M.col32 = st->m_pc_tmp;
-    M.cur32 = st->m_pc_cur;
-    M.rhs32 = st->m_pc_rhs;
     M.partials = st->partials;
     M.sc = st->sc;
     M.n = g.nv();
@@ -1650,8 +1649,8 @@ static void ensemble_fill(pcf_ensemble::Group& grp) {
     M.maxit = st->cfg.poisson_iterations;
     const dim3 pg = pair_grid(g);
     grp.pair_blocks[q] = (int)(pg.x * pg.y * pg.z);
-    grp.thomas_blocks[q] = (int)(blocks_for(g.nx, 64) * g.ny);
-    grp.rhs32_blocks[q] = ensemble_rhs32_blocks(st);
+    grp.line_blocks[q] = mixed ? ensemble_line_blocks(st) : (int)(blocks_for(g.nx, 64) * g.ny);
+    grp.line_threads[q] = mixed ? ensemble_line_threads(st) : 64;
   }
 }
 
@@ -1687,26 +1686,24 @@ int ensemble_iterate(pcf_ensemble* e, pcf_ensemble::Group& grp, int parity, int3
   hipStream_t s = e->stream;
   EnsList& L = grp.list_host[parity];
   L.count = cnt;
-  int pb = 0, tb = 0, rb = 0;
+  int pb = 0, tb = 0, threads = 0;
   for (int a = 0; a < cnt; ++a) {
     const int m = grp.active[a]->ens_slot;
     L.member[a] = m;
     L.pair_start[a] = pb;
-    L.thomas_start[a] = tb;
-    L.rhs32_start[a] = rb;
+    L.line_start[a] = tb;
     pb += grp.pair_blocks[m];
-    tb += grp.thomas_blocks[m];
-    rb += grp.rhs32_blocks[m];
+    tb += grp.line_blocks[m];
+    threads = std::max(threads, grp.line_threads[m]);
   }
   L.pair_start[cnt] = pb;
-  L.thomas_start[cnt] = tb;
-  L.rhs32_start[cnt] = rb;
+  L.line_start[cnt] = tb;
   PCF_HIP(hipMemcpyAsync(grp.list, &L, sizeof(EnsList), hipMemcpyHostToDevice, s));
   const EnsTable* dT = grp.table;
   const EnsList* dL = grp.list;
   const int vb = cnt * kVecGrid;
   auto prec = [&](int in, int out) {
-    if (mixed) ensemble_precondition_mixed(s, dT, dL, L, iters, bf16, in, out);
+    if (mixed) ensemble_precondition_mixed(s, dT, dL, L, threads, iters, bf16, in, out);
     else ensemble_precondition(s, dT, dL, L, iters, in, out);
   };
   prec(EV_P, EV_Y);
