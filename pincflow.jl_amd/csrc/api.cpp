@@ -367,6 +367,7 @@ int pcf_create(const pcf_config* cfg, pcf_state** out) {
     if ((rc = alloc(st, p, NV > (size_t)g.nz ? NV : (size_t)g.nz))) return fail(rc);
   if ((rc = alloc(st, &st->partials, (size_t)kMaxDots * kPartialStride))) return fail(rc);
   if (cfg->precision == PCF_PRECISION_MIXED && (rc = alloc_mixed(st))) return fail(rc);
+  if ((rc = alloc_line64(st))) return fail(rc);
   if ((rc = alloc(st, &st->cfl_dev, 8))) return fail(rc);
   {
     void* p = nullptr;
@@ -712,8 +713,7 @@ int pcf_set_vector(pcf_state* st, int vec, const double* host_in) {
   if (!p) { set_error("unknown vector"); return PCF_E_ARG; }
   PCF_HIP(hipMemcpyAsync(p, host_in, st->g.nv() * sizeof(double), hipMemcpyHostToDevice, st->stream));
   PCF_HIP(hipStreamSynchronize(st->stream));
-  if (vec == PCF_V_AC || vec == PCF_V_AD || vec == PCF_V_AU) st->pc_factors_valid = false;
-  if (vec >= PCF_V_AC) st->t32_valid = false;
+  if (vec >= PCF_V_AC) st->pc_factors_valid = st->t32_valid = false;  // factors and packed coefficients
   return PCF_OK;
 }
 

@@ -12,16 +12,17 @@
 namespace pcf {
 namespace {
 
-// The grid is cut into tiles of 32 x 2 columns.  A tile's coefficients lie
-// together in memory, [tile][k][coefficient][64 columns], and so do its
-// line-solve factors, [tile][k][P, E, Q][64 columns] (k_line_pack): the 128
-// levels of a block's columns are then one contiguous stream.  With x-fastest
+// The grid is cut into tiles of columns (FP32: 32 x 2, whose bf16 rows fill a
+// 128-byte line; FP64: 16 x 1).  A tile's coefficients lie together in
+// memory, [tile][k][coefficient][column], and so do its line-solve factors,
+// [tile][k][P, E, Q][column] (k_line_pack): the levels of a block's columns
+// are then one contiguous stream.  With x-fastest
 // arrays every level and coefficient of a column lies on a page of its own,
 // and the same kernel took 234 us instead of 120 at 256 x 256 x 128 (bf16).
 //
 // A block takes one tile; thread (x, seg) owns the NPL consecutive levels
 // from seg NPL of W adjacent columns, so the block has CX ceil(nz / NPL)
-// threads, CX = 64 / W.  A thread evaluates the right-hand side of
+// threads, CX = the tile's columns / W.  A thread evaluates the right-hand side of
 // its levels in registers.  The two recurrences of the line solve,
 // s_k = (r_k + e_k s_(k-1)) p_k upwards and y_k = s_k + q_k y_(k+1)
 // downwards, are affine maps: a thread composes those of its levels, the
@@ -45,11 +46,34 @@ struct LineCoefs {
   const T *P, *E, *Q;
 };
 
-constexpr int kTileX = 32, kTileY = 2, kTileCols = kTileX * kTileY;
+template <typename R>
+struct LineTile {
+  static constexpr int X = sizeof(R) == 8 ? 16 : 32, Y = sizeof(R) == 8 ? 1 : 2, cols = X * Y;
+  static int count(int nx, int ny) { return ((nx + X - 1) / X) * ((ny + Y - 1) / Y); }
+};
 
-__host__ __device__ inline int line_tiles(int nx, int ny) {
-  return ((nx + kTileX - 1) / kTileX) * ((ny + kTileY - 1) / kTileY);
-}
+// The columns and levels of a thread of a tile.
+template <typename R, int W, int NPL>
+struct LineThread {
+  int tx, seg, i, j, k0;
+  bool act;
+  size_t o, c;  // the first cell in the x-fastest arrays; its level in the tile's arrays
+  __device__ __forceinline__ LineThread(int tile, int nx, int ny, int nz) {
+    using T = LineTile<R>;
+    constexpr int CX = T::cols / W;
+    const int tiles_x = (nx + T::X - 1) / T::X;
+    tx = threadIdx.x % CX;
+    seg = threadIdx.x / CX;
+    i = (tile % tiles_x) * T::X + (tx * W) % T::X;
+    j = (tile / tiles_x) * T::Y + (tx * W) / T::X;
+    act = i < nx && j < ny;
+    if (i >= nx) i = nx - W;  // idle threads read cells of the grid
+    if (j >= ny) j = ny - 1;
+    k0 = seg * NPL;
+    o = (size_t)i + (size_t)nx * (j + (size_t)ny * k0);
+    c = (size_t)tile * nz + k0;
+  }
+};
 
 // bytes of dynamic LDS of a block of `threads` threads
 template <typename R, int W>
@@ -110,7 +134,7 @@ struct LineCoef {
 template <typename R, int W, int NPL>
 __device__ __forceinline__ void line_solve_segments(const R* __restrict__ f, int k0, int nz, int tx, int seg, int nseg,
                                                     R (&r)[NPL][W], R* lds) {
-  constexpr int CX = kTileCols / W;
+  constexpr int cols = LineTile<R>::cols, CX = cols / W;
   R *la = lds, *lb = lds + CX * W * nseg, *lc = lb + CX * W * nseg, *ld = lc + CX * W * nseg;
   const int at = (seg * CX + tx) * W;
   R e[NPL][W], p[NPL][W], q[NPL][W];
@@ -122,10 +146,10 @@ __device__ __forceinline__ void line_solve_segments(const R* __restrict__ f, int
   }
 #pragma unroll
   for (int u = 0; u < NPL; ++u) {
-    const R* fu = f + 3 * kTileCols * (min(k0 + u, nz - 1) - k0);
+    const R* fu = f + 3 * cols * (min(k0 + u, nz - 1) - k0);
     line_load<W, true>(fu, p[u]);
-    line_load<W, true>(fu + kTileCols, e[u]);
-    line_load<W, true>(fu + 2 * kTileCols, q[u]);
+    line_load<W, true>(fu + cols, e[u]);
+    line_load<W, true>(fu + 2 * cols, q[u]);
   }
 #pragma unroll
   for (int u = 0; u < NPL; ++u) {
@@ -203,44 +227,52 @@ __device__ __forceinline__ void line_solve_segments(const R* __restrict__ f, int
 template <typename R, class Rhs, class Put>
 __device__ __forceinline__ void line_solve_column(const R* f, R* col, size_t c, size_t stride, int nz, Rhs rhs,
                                                   Put put) {
+  constexpr int cols = LineTile<R>::cols;
   R s = 0;
   for (int k = 0; k < nz; ++k) {
-    const R* fk = f + (size_t)3 * kTileCols * k;
-    s = k == 0 ? rhs(k) / fk[0] : (rhs(k) + fk[kTileCols] * s) * fk[0];
+    const R* fk = f + (size_t)3 * cols * k;
+    s = k == 0 ? rhs(k) / fk[0] : (rhs(k) + fk[cols] * s) * fk[0];
     col[c + stride * k] = s;
   }
   put(nz - 1, s);
   for (int k = nz - 2; k >= 0; --k) {
-    s = col[c + stride * k] + f[(size_t)3 * kTileCols * k + 2 * kTileCols] * s;
+    s = col[c + stride * k] + f[(size_t)3 * cols * k + 2 * cols] * s;
     put(k, s);
   }
 }
 
 // Pack a grid's x-fastest coefficients and factors (SrcT) into tiles: block
-// (tile, group of 4 levels) of 64 x 4 threads.  The columns beyond the grid
-// of a partial tile get zero coefficients and the identity's factors.
+// (tile, group of levels) of cols x 256 / cols threads.  The columns beyond
+// the grid of a partial tile get zero coefficients and the identity's factors.
 template <typename SrcT, typename CT, typename R>
 __global__ void __launch_bounds__(256) k_line_pack(LineCoefs<SrcT> A, CT* __restrict__ coefs, R* __restrict__ factors,
                                                    int nx, int ny, int nz) {
-  const int lane = threadIdx.x, k = blockIdx.y * 4 + threadIdx.y, tile = blockIdx.x;
+  using L = LineTile<R>;
+  const int lane = threadIdx.x, k = blockIdx.y * blockDim.y + threadIdx.y, tile = blockIdx.x;
   if (k >= nz) return;
-  const int tx = (nx + kTileX - 1) / kTileX;
-  const int i = (tile % tx) * kTileX + lane % kTileX, j = (tile / tx) * kTileY + lane / kTileX;
+  const int tx = (nx + L::X - 1) / L::X;
+  const int i = (tile % tx) * L::X + lane % L::X, j = (tile / tx) * L::Y + lane / L::X;
   const bool in = i < nx && j < ny;
   const size_t o = in ? (size_t)i + (size_t)nx * (j + (size_t)ny * k) : 0;
-  CT* c = coefs + ((size_t)tile * nz + k) * T_COUNT * kTileCols + lane;
-  R* f = factors + ((size_t)tile * nz + k) * 3 * kTileCols + lane;
+  CT* c = coefs + ((size_t)tile * nz + k) * T_COUNT * L::cols + lane;
+  R* f = factors + ((size_t)tile * nz + k) * 3 * L::cols + lane;
   for (int t = 0; t < T_COUNT; ++t) {
     if constexpr (sizeof(CT) == 2) {
       const unsigned u = in ? __float_as_uint((float)A.a[t][o]) : 0u;
-      c[t * kTileCols] = (CT)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);  // round to nearest even
+      c[t * L::cols] = (CT)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);  // round to nearest even
     } else {
-      c[t * kTileCols] = in ? (CT)A.a[t][o] : (CT)0;
+      c[t * L::cols] = in ? (CT)A.a[t][o] : (CT)0;
     }
   }
   f[0] = in ? (R)A.P[o] : (R)1;
-  f[kTileCols] = in ? (R)A.E[o] : (R)0;
-  f[2 * kTileCols] = in ? (R)A.Q[o] : (R)0;
+  f[L::cols] = in ? (R)A.E[o] : (R)0;
+  f[2 * L::cols] = in ? (R)A.Q[o] : (R)0;
+}
+template <typename SrcT, typename CT, typename R>
+void launch_line_pack(hipStream_t s, const LineCoefs<SrcT>& A, CT* coefs, R* factors, int nx, int ny, int nz) {
+  constexpr int cols = LineTile<R>::cols, rows = 256 / cols;
+  hipLaunchKernelGGL((k_line_pack<SrcT, CT, R>), dim3(LineTile<R>::count(nx, ny), (nz + rows - 1) / rows),
+                     dim3(cols, rows), 0, s, A, coefs, factors, nx, ny, nz);
 }
 
 // The block a launch's b-th workgroup takes: consecutive workgroups go to
@@ -271,6 +303,7 @@ __device__ __forceinline__ void line_rhs(const CT* __restrict__ a, Rd rd, const 
   // evaluated and those beyond it after, which a compiler barrier at the
   // level's result keeps (without it the loads are hoisted until the registers
   // spill); DEPTH < 0 leaves the order to the compiler.
+  constexpr int cols = LineTile<R>::cols;
   constexpr int LAG = DEPTH < 0 ? 0 : DEPTH, AHEAD = 4 + LAG;  // levels of s loaded before the first is evaluated
   R C[NPL + 4][W + 2], F[NPL + 4][W], B[NPL + 4][W];  // C with its x neighbours
   auto level = [&](int w) {
@@ -288,10 +321,10 @@ __device__ __forceinline__ void line_rhs(const CT* __restrict__ a, Rd rd, const 
   BT bv[LAG + 1][W];
   auto coefs = [&](int u) {
     const int d = u % (LAG + 1), v = min(k0 + u, nz - 1) - k0;  // v < 0 only for idle segments
-    const CT* av = a + T_COUNT * kTileCols * v;
+    const CT* av = a + T_COUNT * cols * v;
 #pragma unroll
     for (int t = 0; t < T_COUNT; ++t)
-      if (RESID || (t != T_AC && t != T_AD && t != T_AU)) T[d][t].load(av + t * kTileCols);
+      if (RESID || (t != T_AC && t != T_AD && t != T_AU)) T[d][t].load(av + t * cols);
     line_load<W, true>(b + ((size_t)i + (size_t)nx * j + sxy * (size_t)(k0 + v)), bv[d]);
   };
 #pragma unroll

@@ -106,27 +106,7 @@ struct LineRead {
   }
 };
 
-// The columns and levels of a thread of tile `tile` (line_step.hpp).
-template <int W, int NPL>
-struct LineThread {
-  int tx, seg, i, j, k0;
-  bool act;
-  size_t o, c;  // the first cell in the x-fastest arrays; its column in the tile's arrays
-  __device__ __forceinline__ LineThread(int tile, int nx, int ny, int nz) {
-    constexpr int CX = kTileCols / W;
-    const int tiles_x = (nx + kTileX - 1) / kTileX;
-    tx = threadIdx.x % CX;
-    seg = threadIdx.x / CX;
-    i = (tile % tiles_x) * kTileX + (tx * W) % kTileX;
-    j = (tile / tiles_x) * kTileY + (tx * W) / kTileX;
-    act = i < nx && j < ny;
-    if (i >= nx) i = nx - W;  // idle threads read cells of the grid
-    if (j >= ny) j = ny - 1;
-    k0 = seg * NPL;
-    o = (size_t)i + (size_t)nx * (j + (size_t)ny * k0);
-    c = (size_t)tile * nz + k0;
-  }
-};
+constexpr int kTileCols = LineTile<float>::cols, kTileX = LineTile<float>::X;
 
 // One pseudo-time step in FP32 of a tile (line_step.hpp); s and out must
 // differ.
@@ -135,7 +115,7 @@ __device__ __forceinline__ void line_step32(const LineArgs<CT>& A, const BT* __r
                                             int tile) {
   extern __shared__ float line_shared[];
   const int nx = A.nx, ny = A.ny, nz = A.nz;
-  const LineThread<W, NPL> t(tile, nx, ny, nz);
+  const LineThread<float, W, NPL> t(tile, nx, ny, nz);
   const size_t sxy = (size_t)nx * ny;
   float r[NPL][W];
   if constexpr (FIRST) {
@@ -174,7 +154,7 @@ __global__ void __launch_bounds__(kTileCols) k_line_tall32(LineArgs<CT> A, const
                                                            OutT* __restrict__ out, float* col,
                                                            const SolverScalars* sc) {
   if (sc && sc->done) return;
-  const LineThread<1, 1> t(blockIdx.x, A.nx, A.ny, A.nz);
+  const LineThread<float, 1, 1> t(blockIdx.x, A.nx, A.ny, A.nz);
   if (!t.act) return;
   const size_t sxy = (size_t)A.nx * A.ny;
   auto rhs = [&](int k) -> float {
@@ -347,7 +327,7 @@ __global__ void __launch_bounds__(W == 4 ? 512 : 1024)
   if (sc && sc->done) return;
   const int nx = A.nx, ny = A.ny, nz = A.nz;
   const int tile = xcd_block(blockIdx.x, gridDim.x);
-  const LineThread<W, NPL> t(tile, nx, ny, nz);
+  const LineThread<float, W, NPL> t(tile, nx, ny, nz);
   float r[NPL][W];
   line_rhs<float, W, NPL, W == 1 && NPL == 8 ? 1 : 0, true, CT, BT>(A.coefs + t.c * T_COUNT * kTileCols + t.tx * W, LineRead<W, false, CT>{A}, b,
                                         nx, ny, nz, A.deta, t.i, t.j, t.k0, r);
@@ -622,7 +602,7 @@ void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, Out
     constexpr bool PRO = decltype(pro)::value;
     using CT = decltype(ct);
     const LineArgs<CT> A = line_args<CT>(L, s, e, C);
-    const dim3 grd(line_tiles(L.nx, L.ny));
+    const dim3 grd(LineTile<float>::count(L.nx, L.ny));
     if (L.nz > kLineMaxNz)
       hipLaunchKernelGGL((k_line_tall32<FIRST, PRO, CT, BT, OutT>), grd, dim3(kTileCols), 0, st->stream, A, b, out,
                          L.col, sc);
@@ -649,13 +629,8 @@ void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, Out
 // Pack a level's coefficients and factors for the line steps.
 template <typename SrcT>
 void line_pack(pcf_state* st, const MgLevel& L, const LineCoefs<SrcT>& A) {
-  const dim3 grd(line_tiles(L.nx, L.ny), blocks_for(L.nz, 4)), blk(kTileCols, 4);
-  if (bf16_storage(st))
-    hipLaunchKernelGGL((k_line_pack<SrcT, uint16_t, float>), grd, blk, 0, st->stream, A, (uint16_t*)L.coefs, L.factors,
-                       L.nx, L.ny, L.nz);
-  else
-    hipLaunchKernelGGL((k_line_pack<SrcT, float, float>), grd, blk, 0, st->stream, A, (float*)L.coefs, L.factors, L.nx,
-                       L.ny, L.nz);
+  if (bf16_storage(st)) launch_line_pack(st->stream, A, (uint16_t*)L.coefs, L.factors, L.nx, L.ny, L.nz);
+  else launch_line_pack(st->stream, A, (float*)L.coefs, L.factors, L.nx, L.ny, L.nz);
 }
 
 // The preconditioner's copies of the current operator: the packed
@@ -833,7 +808,7 @@ void mg_restrict(pcf_state* st, const MgLevel& L, const MgLevel& C, const BT* b,
       using CT = decltype(ct);
       with_line_shape(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
         constexpr int W = decltype(w)::value, NPL = decltype(npl)::value;
-        hipLaunchKernelGGL((k_resid_restrict<W, NPL, BT, CT>), dim3(line_tiles(L.nx, L.ny)),
+        hipLaunchKernelGGL((k_resid_restrict<W, NPL, BT, CT>), dim3(LineTile<float>::count(L.nx, L.ny)),
                            dim3(kTileCols / W * ((L.nz + NPL - 1) / NPL)), 0, st->stream,
                            line_args<CT>(L, s, nullptr, &C), b, C.b, sc);
       });
@@ -1032,7 +1007,7 @@ __global__ void __launch_bounds__(1024) kEm_line(const EnsTable* __restrict__ E,
 }  // namespace
 
 // blocks and threads per block of a member's line steps
-int ensemble_line_blocks(const pcf_state* st) { return line_tiles(st->g.nx, st->g.ny); }
+int ensemble_line_blocks(const pcf_state* st) { return LineTile<float>::count(st->g.nx, st->g.ny); }
 int ensemble_line_threads(const pcf_state* st) {
   const int npl = st->g.nz > 128 ? 16 : 8;
   return kTileCols * ((st->g.nz + npl - 1) / npl);
@@ -1070,7 +1045,7 @@ int alloc_mixed(pcf_state* st) {
   auto af = [&](float** p) -> int { return device_alloc(st, p, N); };
   // the packed arrays of a level smoothed by line steps
   auto packed = [&](MgLevel& L) -> int {
-    const size_t n = (size_t)line_tiles(L.nx, L.ny) * kTileCols * L.nz;
+    const size_t n = (size_t)LineTile<float>::count(L.nx, L.ny) * kTileCols * L.nz;
     int rc1 = device_alloc(st, &L.coefs, n * T_COUNT * (bf16_storage(st) ? 2 : 4));
     return rc1 ? rc1 : device_alloc(st, &L.factors, 3 * n);
   };

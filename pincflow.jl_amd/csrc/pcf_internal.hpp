@@ -277,6 +277,7 @@ struct pcf_state {
   double *pc_rhs, *pc_q, *pc_tmp;     // preconditioner work (pc_q: also scratch of the sponge)
   double *pc_P, *pc_E, *pc_Q;         // line-solve factors of the current operator
   bool pc_factors_valid = false;
+  double *pc_coefs = nullptr, *pc_factors = nullptr;  // packed for the line steps (line_step.hpp)
   // mixed precision (allocated when cfg.precision == PCF_PRECISION_MIXED):
   // the preconditioner's levels (mg below) and z = M^-1 s
   double* bzpc = nullptr;
@@ -397,6 +398,7 @@ int apply_bicgstab(pcf_state* st, double tolref, int* niter);
 int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess, double guess_scale, int* niter);
 int solve(pcf_state* st, double tolref, double dt, int* niter);  // apply_bicgstab, configured precision
 int pc_factors(pcf_state* st);
+int alloc_line64(pcf_state* st);
 // ensemble (poisson.hip): the solve kind of a member (-1: the member table
 // does not cover it), whether this solve joins the batch, the table upload,
 // one batched iteration of a group's active solves (list slot `parity`,

@@ -1,6 +1,6 @@
 """The fused line step of the preconditioner (csrc/line_step.hpp) at the edges
-of its tiles (32 x 2 columns), of its segments (8 or 16 levels per thread) and
-of its launch rule, against the FP64 oracle's preconditioner."""
+of its tiles (FP32: 32 x 2 columns, FP64: 16 x 1), of its segments (4, 8 or 16
+levels per thread) and of its launch rules, against the FP64 oracle's preconditioner."""
 import numpy as np
 import pytest
 
@@ -45,3 +45,13 @@ def test_fp32_line_step_matches_the_oracle(pcf, abi, oracle_mod, shape, storage,
     err = preconditioned(pcf, abi, oracle_mod, shape, "mixed", storage, iterations)
     print(shape, storage, iterations, err)
     assert err <= 1e-4, err
+
+
+@pytest.mark.parametrize("shape,iterations", [
+    ((16, 4, 4), 2), ((17, 1, 5), 2), ((15, 3, 129), 2), ((33, 5, 128), 3), ((20, 3, 256), 2), ((20, 3, 257), 2),
+    ((120, 50, 100), 2), ((120, 51, 100), 2), ((31, 7, 9), 1)])
+def test_fp64_line_step_matches_the_oracle(pcf, abi, oracle_mod, shape, iterations):
+    """FP64, both sides of the launch rule (256 levels, 600000 cells), the
+    same operations in the same order as the oracle: 1e-13."""
+    err = preconditioned(pcf, abi, oracle_mod, shape, "fp64", iterations=iterations)
+    assert err <= 1e-13, err
