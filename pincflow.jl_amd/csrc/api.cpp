@@ -128,14 +128,25 @@ int predictand_slots(pcf_state* st, double* out[7]) {
   return st->compressible ? 7 : 6;
 }
 
+// fields to copy in one launch
+struct Copies {
+  double *dst[8], *src[8];
+  int n = 0;
+  void add(double* d, double* s) {
+    dst[n] = d;
+    src[n] = s;
+    n += 1;
+  }
+};
+
 int save_backups(pcf_state* st, bool rho, bool rhop, bool u, bool v, bool w) {  // save_backups!.jl
-  int rc = PCF_OK;
-  if (rho && (rc = copy_field(st, st->rhoold, st->rho))) return rc;
-  if (rhop && (rc = copy_field(st, st->rhopold, st->rhop))) return rc;
-  if (u && (rc = copy_field(st, st->uold, st->u))) return rc;
-  if (v && (rc = copy_field(st, st->vold, st->v))) return rc;
-  if (w && (rc = copy_field(st, st->wold, st->w))) return rc;
-  return rc;
+  Copies c;
+  if (rho) c.add(st->rhoold, st->rho);
+  if (rhop) c.add(st->rhopold, st->rhop);
+  if (u) c.add(st->uold, st->u);
+  if (v) c.add(st->vold, st->v);
+  if (w) c.add(st->wold, st->w);
+  return copy_fields(st, c.dst, c.src, c.n);
 }
 
 #define TRY(x)            \
@@ -204,11 +215,6 @@ int implicit(pcf_state* st, double dt, double time, double rf, int* niter) {
   TRY(apply_corrector(st, dt, rf, niter));
   TRY(modify_compressible_wind(st, false));
   return set_boundaries_predictands(st);
-}
-
-int copy_set(pcf_state* st, double* const* dst, double* const* src, int n) {
-  for (int q = 0; q < n; ++q) TRY(copy_field(st, dst[q], src[q]));
-  return PCF_OK;
 }
 
 // compute_time_step.jl:46-153 (NoWKB)
@@ -465,9 +471,10 @@ int pcf_backup_predictands(pcf_state* st) {
   if (!st) return PCF_E_ARG;
   double* cur[7];
   const int np = predictand_slots(st, cur);
-  TRY(copy_set(st, st->p0, cur, np));
-  if (st->tracer) TRY(copy_field(st, st->chi0, st->chi));  // backup_predictands.jl:18
-  return PCF_OK;
+  Copies c;
+  for (int q = 0; q < np; ++q) c.add(st->p0[q], cur[q]);
+  if (st->tracer) c.add(st->chi0, st->chi);  // backup_predictands.jl:18
+  return copy_fields(st, c.dst, c.src, c.n);
 }
 
 int pcf_explicit_integration_lhs(pcf_state* st, double dt, double time) {
@@ -509,8 +516,7 @@ int pcf_step(pcf_state* st, pcf_step_info* info) {
   TRY(set_boundaries_predictands(st));
   double* cur[7];
   const int np = predictand_slots(st, cur);
-  TRY(copy_set(st, st->p0, cur, np));  // backup_predictands
-  if (st->tracer) TRY(copy_field(st, st->chi0, st->chi));
+  TRY(pcf_backup_predictands(st));
   TRY(compute_theta_fluxes(st));                              // integrate.jl:277
   TRY(explicit_lhs(st, 0.5 * dt, time));                      // (1)
   int it1 = 0, it2 = 0;
@@ -519,22 +525,19 @@ int pcf_step(pcf_state* st, pcf_step_info* info) {
   st->solve_slot = -1;
   info->niter[0] = it1;
   if (rc) return rc;
-  TRY(copy_set(st, st->p1, cur, np));                         // p1 = predictands
+  TRY(copy_fields(st, st->p1, cur, np));                      // p1 = predictands
   // reset_predictands! (reset_predictands!.jl:71-118): rho (PI and
   // compressible), rhop, u, v, w; pip and p too in the compressible model,
   // else pip keeps its new value
-  if (n.model != PCF_BOUSSINESQ) TRY(copy_field(st, st->rho, st->p0[0]));
-  TRY(copy_field(st, st->rhop, st->p0[1]));
-  TRY(copy_field(st, st->u, st->p0[2]));
-  TRY(copy_field(st, st->v, st->p0[3]));
-  TRY(copy_field(st, st->w, st->p0[4]));
-  if (st->compressible) {
-    TRY(copy_field(st, st->pip, st->p0[5]));
-    TRY(copy_field(st, st->p, st->p0[6]));
-  }
-  if (st->tracer) TRY(copy_field(st, st->chi, st->chi0));     // reset_predictands!.jl:63-67
+  Copies reset;
+  if (n.model != PCF_BOUSSINESQ) reset.add(st->rho, st->p0[0]);
+  for (int q = 1; q <= 4; ++q) reset.add(cur[q], st->p0[q]);  // rhop, u, v, w
+  if (st->compressible)
+    for (int q = 5; q <= 6; ++q) reset.add(cur[q], st->p0[q]);  // pip, p
+  if (st->tracer) reset.add(st->chi, st->chi0);               // reset_predictands!.jl:63-67
+  TRY(copy_fields(st, reset.dst, reset.src, reset.n));
   TRY(explicit_rhs(st, 0.5 * dt, time));                      // (3)
-  TRY(copy_set(st, st->p0, st->p1, np));                      // p0 = p1
+  TRY(copy_fields(st, st->p0, st->p1, np));                   // p0 = p1
   TRY(synchronize_compressible_atmosphere(st, st->p0[6]));   // pbar = p1.p
   TRY(explicit_lhs(st, dt, time));                            // (4)
   st->solve_slot = 1;

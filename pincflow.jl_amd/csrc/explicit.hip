@@ -11,6 +11,7 @@
 // halo position gives the same bits.  Only fluxes the updates consume are
 // computed; the wall faces that set_boundaries!(state, BoundaryFluxes()) zeroes
 // are written as zeros.
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <type_traits>
@@ -1186,16 +1187,22 @@ __global__ void k_cfl(const double* u, const double* v, const double* w, Geo g, 
     }
 }
 
+// one wavefront per component (one thread alone took 130 us for 3 x 512 maxima)
 __global__ void k_cfl_final(const double* partials, int nparts, double* out) {
-  if (threadIdx.x != 0) return;
-  for (int d = 0; d < 3; ++d) {
-    double x = 0.0;
-    for (int q = 0; q < nparts; ++q) x = dmax(x, partials[d * nparts + q]);
-    out[d] = x;
-  }
+  const int d = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double x = 0.0;
+  for (int q = lane; q < nparts; q += 64) x = dmax(x, partials[d * nparts + q]);
+  for (int off = 32; off > 0; off >>= 1) x = dmax(x, __shfl_down(x, off, 64));
+  if (lane == 0) out[d] = x;
 }
 
-__global__ void k_copy_field(double* dst, const double* src, size_t n) {
+struct CopyList {
+  double* dst[kMaxCopies];
+  const double* src[kMaxCopies];
+};
+__global__ void k_copy_fields(CopyList cl, size_t n) {
+  double* dst = cl.dst[blockIdx.y];
+  const double* src = cl.src[blockIdx.y];
   for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x)
     dst[q] = src[q];
 }
@@ -1473,7 +1480,7 @@ int refresh_fcscal(pcf_state* st) {
 
 int synchronize_density_fluctuations(pcf_state* st) {
   ProfScope prof(st, PCF_K_UPDATES);
-  if (st->cfg.model == PCF_PSEUDO_INCOMPRESSIBLE) return copy_field(st, st->rhop, st->rho);
+  if (st->cfg.model == PCF_PSEUDO_INCOMPRESSIBLE) return copy_fields(st, &st->rhop, &st->rho, 1);
   if (st->cfg.model == PCF_COMPRESSIBLE) {
     hipLaunchKernelGGL(k_sync_rhop, dim3(2048), dim3(256), 0, st->stream, st->rhop, st->rho, st->rhobar, st->pbar,
                        st->thetabar, st->g.nh());
@@ -1861,7 +1868,7 @@ int compute_sponges(pcf_state* st, double dt, double time) {
 int cfl_maxima(pcf_state* st, double out[3]) {
   const int nb = 512;
   hipLaunchKernelGGL(k_cfl, dim3(nb), dim3(256), 0, st->stream, st->u, st->v, st->w, st->g, st->partials);
-  hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(64), 0, st->stream, st->partials, nb, st->cfl_dev);
+  hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(192), 0, st->stream, st->partials, nb, st->cfl_dev);
   PCF_HIP(hipGetLastError());
   PCF_HIP(hipMemcpyAsync(st->cfl_host, st->cfl_dev, 3 * sizeof(double), hipMemcpyDeviceToHost, st->stream));
   PCF_HIP(hipStreamSynchronize(st->stream));
@@ -1869,9 +1876,18 @@ int cfl_maxima(pcf_state* st, double out[3]) {
   return PCF_OK;
 }
 
-int copy_field(pcf_state* st, double* dst, const double* src) {
+int copy_fields(pcf_state* st, double* const* dst, double* const* src, int n) {
   ProfScope prof(st, PCF_K_UPDATES);
-  hipLaunchKernelGGL(k_copy_field, dim3(2048), dim3(256), 0, st->stream, dst, src, st->g.nh());
+  const unsigned blocks = std::min(2048u, blocks_for((long long)st->g.nh(), 256));
+  for (int off = 0; off < n; off += kMaxCopies) {
+    CopyList cl{};
+    const int m = std::min(n - off, kMaxCopies);
+    for (int q = 0; q < m; ++q) {
+      cl.dst[q] = dst[off + q];
+      cl.src[q] = src[off + q];
+    }
+    hipLaunchKernelGGL(k_copy_fields, dim3(blocks, m), dim3(256), 0, st->stream, cl, st->g.nh());
+  }
   PCF_HIP(hipGetLastError());
   return PCF_OK;
 }

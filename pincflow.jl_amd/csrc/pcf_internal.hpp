@@ -455,7 +455,8 @@ int update_rhs(pcf_state* st, double dt, int var, bool implicit, double rf);
 int apply_lhs_sponge(pcf_state* st, double dt, double time, int var);
 int compute_sponges(pcf_state* st, double dt, double time);
 int cfl_maxima(pcf_state* st, double out[3]);
-int copy_field(pcf_state* st, double* dst, const double* src);
+constexpr int kMaxCopies = 8;
+int copy_fields(pcf_state* st, double* const* dst, double* const* src, int n);  // one launch per kMaxCopies
 int compute_theta_fluxes(pcf_state* st);
 int modify_compressible_wind(pcf_state* st, bool multiply);
 int synchronize_compressible_atmosphere(pcf_state* st, const double* p);
