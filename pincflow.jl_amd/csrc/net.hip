@@ -8,15 +8,16 @@
 // in LDS (k_brick); weights and activations are bf16, the network's input is
 // rounded to bf16 on staging.  The backward pass reuses the 32 -> 32 kernel
 // for the input gradient (transposed, tap-flipped weights) and has its own
-// MFMA kernel for the weight gradient (a GEMM over the voxels, split into
-// chunks whose partial sums are added in a fixed order); the weight
-// gradients of the first and last layers and the last layer's input
-// gradient run on the vector units from the FP32 master weights.
+// MFMA kernels for the weight gradients (GEMMs over the voxels, split into
+// groups of bricks whose partial sums are added in a fixed order; FP32 MFMA
+// in the first and last layers); the last layer's input gradient runs on the
+// vector units from the FP32 master weights.
 //
 // Layout: activations are channels-last [voxel][channel] with voxel =
 // i + nx (j + ny k); parameters are one FP32 vector, layer by layer W[27][cout][cin]
 // then b[cout], tap t = (dx + 1) + 3 (dy + 1) + 9 (dz + 1) weighing the input
 // at (i + dx, j + dy, k + dz).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -35,7 +36,6 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 
 constexpr int kC = 32;        // hidden channels
 constexpr int kLayers = 6;
-constexpr int kChunk = 4096;  // voxels per partial sum of a weight gradient
 constexpr int kCin[kLayers] = {3, 32, 32, 32, 32, 32};
 constexpr int kCout[kLayers] = {32, 32, 32, 32, 32, 1};
 
@@ -353,200 +353,267 @@ __global__ void k_last_data(Dims d, const float* dout, const float* W, float* g)
   for (int c = 0; c < kC; ++c) g[p * kC + c] = acc[c];
 }
 
-// ---- layer 6 weight gradient: per chunk of voxels, W[t][c] += dout(p) in(p + tap_t)[c], b += dout(p).
-// Thread (t, 4 channels) of 216, thread 216 the bias; the chunk's dout in LDS.
-constexpr int kLastWThreads = 27 * kC / 4 + 1;
-__global__ void __launch_bounds__(256) k_last_weights(Dims d, const float* dout, const bf16* in, float* partials) {
-  __shared__ float ld[256];
-  const int slot = threadIdx.x;
-  const size_t p0 = (size_t)blockIdx.x * kChunk, p1 = p0 + kChunk < d.n ? p0 + kChunk : d.n;
-  const int t = slot / (kC / 4), c0 = 4 * (slot % (kC / 4));
-  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (size_t pb = p0; pb < p1; pb += 256) {
-    const size_t pl = pb + threadIdx.x;
-    ld[threadIdx.x] = pl < p1 ? dout[pl] : 0.0f;
-    __syncthreads();
-    const int m = (int)(p1 - pb < 256 ? p1 - pb : 256);
-    if (slot < kLastWThreads - 1) {
-      for (int v = 0; v < m; ++v) {
-        const size_t p = pb + v;
-        int i, j, k;
-        coords(d, p, i, j, k);
-        const long long q = neighbour(d, i, j, k, t);
-        if (q < 0) continue;
-        const float dv = ld[v];
-        typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
-        const bf4 x = *(const bf4*)(in + (size_t)q * kC + c0);
+// ---- weight gradients, over the bricks of the forward pass.  A workgroup
+// takes `per` consecutive bricks of 32 x 4 x 4 voxels, stages each with its
+// halo in LDS once for all 27 taps, and keeps its sums in the matrix cores'
+// accumulators; its partial sums are added in a fixed order afterwards
+// (sum_chunks).  The first and last layers' sums have FP32 factors and run on
+// v_mfma_f32_32x32x2_f32 (FP32 products and sums): lane l holds A[l % 32][l / 32]
+// and B[l / 32][l % 32], two voxels a step.  Before, these sums walked chunks
+// of 4096 voxels one voxel at a time on the vector units, or one tap per
+// wavefront: at 128 x 128 x 64 the first, a middle and the last layer took
+// 639, 327 and 1598 us, now 102, 83 and 56.
+constexpr int kBricksPer = 8;  // most bricks per workgroup
+
+// Brick coordinates and LDS staging shared by the first and last layers:
+// NC floats per voxel of the brick with its halo (zero beyond the walls).
+template <int NC>
+__device__ __forceinline__ void stage_brick(const Dims& d, const float* __restrict__ src, int x0, int y0, int z0,
+                                            float* brick) {
+  for (int v = threadIdx.x; v < kBrickVox; v += 256) {
+    const int bx = v % kBX, byz = v / kBX, by = byz % kBY, bz = byz / kBY;
+    const int gz = z0 + bz - 1;
+    float x[NC] = {};
+    if (gz >= 0 && gz < d.nz) {
+      const size_t q = (size_t)wrap(x0 + bx - 1, d.nx) + (size_t)d.nx * (wrap(y0 + by - 1, d.ny) + (size_t)d.ny * gz);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] += dv * (float)x[e];
-      }
-    } else if (slot == kLastWThreads - 1) {
-      for (int v = 0; v < m; ++v) s[0] += ld[v];
+      for (int c = 0; c < NC; ++c) x[c] = src[NC * q + c];
     }
-    __syncthreads();
-  }
-  float* out = partials + (size_t)blockIdx.x * (27 * kC + 1);
-  if (slot < kLastWThreads - 1) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) out[t * kC + c0 + e] = s[e];
-  } else if (slot == kLastWThreads - 1) {
-    out[27 * kC] = s[0];
+    for (int c = 0; c < NC; ++c) brick[NC * v + c] = x[c];
   }
+}
+// brick voxel offset of tap t
+__device__ __forceinline__ int tap_offset(int t) { return (t % 3 - 1) + kBX * ((t / 3) % 3 - 1) + kBX * kBY * (t / 9 - 1); }
+
+// ---- layer 6: W[t][c] = sum_q in(q)[c] dout(q - tap_t), b = sum dout.  A: the
+// 32 channels of two voxels, B: their 27 shifted dout.  Wavefront w takes
+// the rows (y, z) = 4 w ... 4 w + 3 of each brick and has its own partial sums.
+__global__ void __launch_bounds__(256) k_last_weights(Dims d, BrickGrid bg, int per, const float* __restrict__ dout,
+                                                      const bf16* __restrict__ in, float* partials) {
+  __shared__ float brick[kBrickVox];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, col = lane & 31, half = lane >> 5;
+  const int off = col < 27 ? -tap_offset(col) : 0;
+  const int bricks = bg.tiles_x * bg.tiles_y * bg.tiles_z;
+  f16v acc = {};
+  float bias = 0.0f;
+  for (int b = blockIdx.x * per; b < min(bricks, ((int)blockIdx.x + 1) * per); ++b) {
+    const int tx = b % bg.tiles_x, tyz = b / bg.tiles_x;
+    const int x0 = 32 * tx, y0 = 4 * (tyz % bg.tiles_y), z0 = 4 * (tyz / bg.tiles_y);
+    __syncthreads();  // the previous brick's readers
+    stage_brick<1>(d, dout, x0, y0, z0, brick);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int y = y0 + r, z = z0 + wv;
+      if (y >= d.ny || z >= d.nz) continue;  // uniform over the wavefront
+      const bf16* row = in + ((size_t)x0 + (size_t)d.nx * (y + (size_t)d.ny * z)) * kC + col;
+      const int v0 = 1 + kBX * ((r + 1) + kBY * (wv + 1));
+      float a[16];
+#pragma unroll
+      for (int s = 0; s < 16; ++s) a[s] = (float)row[(2 * s + half) * kC];
+#pragma unroll
+      for (int s = 0; s < 16; ++s) {
+        const float x = brick[v0 + 2 * s + half + off];
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], col < 27 ? x : 0.0f, acc, 0, 0, 0);
+      }
+      if (half == 0) bias += brick[v0 + col];
+    }
+  }
+  float* out = partials + (size_t)(4 * blockIdx.x + wv) * (27 * kC + 1);
+  if (col < 27) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) out[col * kC + 8 * (q / 4) + 4 * half + q % 4] = acc[q];
+  }
+  for (int o = 32; o > 0; o >>= 1) bias += __shfl_down(bias, o, 64);
+  if (lane == 0) out[27 * kC] = bias;
 }
 
 // ---- GELU backward: dz = g * gelu'(z) (bf16 for the matrix cores), and per
-// block partial sums of dz per channel (the bias gradient, FP32)
-__global__ void k_gelu_back(Dims d, const float* g, const float* z, bf16* dz, float* bias_partials) {
-  __shared__ float red[256];
-  const size_t p0 = (size_t)blockIdx.x * kChunk, p1 = p0 + kChunk < d.n ? p0 + kChunk : d.n;
-  const int c = threadIdx.x % kC, lane_group = threadIdx.x / kC;  // 8 groups of 32
-  float s = 0.0f;
-  for (size_t p = p0 + lane_group; p < p1; p += 8) {
-    const float v = g[p * kC + c] * gelu_grad(z[p * kC + c]);
-    dz[p * kC + c] = (bf16)v;
-    s += v;
+// block of kGeluChunk voxels partial sums of dz per channel (the bias
+// gradient, FP32); four channels per thread.  300 -> 66 us at 128 x 128 x 64
+// (335 MB), where blocks of 4096 voxels left one workgroup per CU.
+constexpr int kGeluChunk = 512;
+__global__ void __launch_bounds__(256) k_gelu_back(Dims d, const float* __restrict__ g, const float* __restrict__ z,
+                                                   bf16* __restrict__ dz, float* bias_partials) {
+  __shared__ float red[32][kC];
+  const size_t p0 = (size_t)blockIdx.x * kGeluChunk;
+  const int c = 4 * (threadIdx.x & 7), v = threadIdx.x >> 3;  // 32 voxels of 8 quads
+  float s[4] = {};
+#pragma unroll 4
+  for (int u = 0; u < kGeluChunk / 32; ++u) {
+    const size_t p = p0 + v + 32 * u;
+    if (p < d.n) {
+      const float4 gv = *(const float4*)(g + p * kC + c), zv = *(const float4*)(z + p * kC + c);
+      const float x[4] = {gv.x * gelu_grad(zv.x), gv.y * gelu_grad(zv.y), gv.z * gelu_grad(zv.z),
+                          gv.w * gelu_grad(zv.w)};
+      *(uint2*)(dz + p * kC + c) = pack4(x[0], x[1], x[2], x[3]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] += x[e];
+    }
   }
-  red[threadIdx.x] = s;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) red[v][c + e] = s[e];
   __syncthreads();
   if (threadIdx.x < kC) {
     float t = 0.0f;
-    for (int q = 0; q < 8; ++q) t += red[q * kC + threadIdx.x];
+    for (int q = 0; q < 32; ++q) t += red[q][threadIdx.x];
     bias_partials[(size_t)blockIdx.x * kC + threadIdx.x] = t;
   }
 }
 
-// ---- weight gradient of a 32 -> 32 layer on the matrix cores: for tap t and
-// a chunk of voxels, dW[t] (32 co x 32 ci) += sum_p dz(p)[co] in(p + tap_t)[ci],
-// with 16 voxels per MFMA step.  A workgroup of four wavefronts takes a chunk
-// and four taps (blockIdx.y = tap group, wavefront w: tap 4 y + w, the last
-// group has three): batches of 64 voxels are staged in LDS, dz once for the
-// four taps and each tap's neighbours apart, and the next batch's global
-// loads are issued before the current batch's MFMAs.  Each tap's MFMAs run
-// over the chunk's 16-voxel steps in order.
-constexpr int kWBatch = 64;  // voxels per staged batch
+// ---- 32 -> 32 layers: dW[t] (32 co x 32 ci) = sum_p dz(p)[co] in(p + tap_t)[ci]
+// on v_mfma_f32_32x32x16_bf16, K = 16 voxels consecutive in x.  Nine
+// wavefronts, one per (dy, dz), each with the accumulators of its three dx.
+// The brick is stored channel by channel, so that a lane reads its channel's
+// 8 consecutive voxels in one access and the window of 10 serves the three
+// dx by shifts; channel strides of 2896 and 1040 bytes put the lanes of an
+// access on distinct banks.  The next brick's loads are in flight during the
+// current brick's MFMAs.  327 -> 83 us per layer at 128 x 128 x 64.
+constexpr int kWThreads = 576;
+constexpr int kInRow = 40, kInChan = 36 * kInRow + 8;  // elements per row of 34 voxels, per channel
+constexpr int kDzChan = 16 * 32 + 8;
+constexpr int kInItems = 36 * 17 * 4, kDzItems = 16 * 16 * 4;  // (row, voxel pair, 8 channels)
+constexpr int kInPer = (kInItems + kWThreads - 1) / kWThreads, kDzPer = (kDzItems + kWThreads - 1) / kWThreads;
 
-__global__ void __launch_bounds__(256) k_mid_weights(Dims d, const bf16* __restrict__ dz, const bf16* __restrict__ in,
-                                                     float* partials) {
-  __shared__ bf16 ld[kWBatch][kC];
-  __shared__ bf16 la[4][kWBatch][kC];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int t = 4 * (int)blockIdx.y + w;  // 27: no tap (the wavefront only stages)
-  const int col = lane & 31, half = lane >> 5;
-  const size_t p0 = (size_t)blockIdx.x * kChunk, p1 = p0 + kChunk < d.n ? p0 + kChunk : d.n;
-  // staging: thread T loads dz of voxel T / 4 (8 channels 8 (T % 4)); lane L
-  // of wavefront w loads its tap's neighbour of voxels L / 4 + 16 u, u < 4
-  const int vd = (int)threadIdx.x >> 2, cd = 8 * (threadIdx.x & 3);
-  const int va = lane >> 2, ca = 8 * (lane & 3);
-  auto load = [&](size_t pb, bf8& dv, bf8 (&av)[4]) {
+__global__ void __launch_bounds__(kWThreads) k_mid_weights(Dims d, BrickGrid bg, int per, const bf16* __restrict__ dz,
+                                                           const bf16* __restrict__ in, float* partials) {
+  extern __shared__ uint4 wlds[];
+  uint16_t* li = (uint16_t*)wlds;
+  uint16_t* ld = li + kC * kInChan;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, col = lane & 31, half = lane >> 5;
+  const int ty = wv % 3, tz = wv / 3;  // dy + 1, dz + 1
+  const int bricks = bg.tiles_x * bg.tiles_y * bg.tiles_z;
+  const int b0 = (int)blockIdx.x * per, b1 = min(bricks, b0 + per);
+  uint4 iv[kInPer][2], dv[kDzPer][2];
+  auto load = [&](int b) {
+    const int tx = b % bg.tiles_x, tyz = b / bg.tiles_x;
+    const int x0 = 32 * tx, y0 = 4 * (tyz % bg.tiles_y), z0 = 4 * (tyz / bg.tiles_y);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) dv[e] = (bf16)0.0f;
-    const size_t p = pb + vd;
-    if (p < p1) dv = *(const bf8*)(dz + p * kC + cd);
+    for (int u = 0; u < kInPer; ++u) {
+      const int e = threadIdx.x + kWThreads * u;
+      iv[u][0] = iv[u][1] = uint4{0u, 0u, 0u, 0u};
+      const int c = e & 3, pr = (e >> 2) % 17, row = (e >> 2) / 17;
+      const int gz = z0 + row / kBY - 1;
+      if (e < kInItems && gz >= 0 && gz < d.nz) {
+        const size_t r = (size_t)d.nx * (wrap(y0 + row % kBY - 1, d.ny) + (size_t)d.ny * gz);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+        for (int h = 0; h < 2; ++h)
+          iv[u][h] = *(const uint4*)(in + (r + wrap(x0 + 2 * pr + h - 1, d.nx)) * kC + 8 * c);
+      }
+    }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) av[u][e] = (bf16)0.0f;
-      const size_t q = pb + va + 16 * u;
-      if (t < 27 && q < p1) {
-        int i, j, k;
-        coords(d, q, i, j, k);
-        const long long nq = neighbour(d, i, j, k, t);
-        if (nq >= 0) av[u] = *(const bf8*)(in + (size_t)nq * kC + ca);
+    for (int u = 0; u < kDzPer; ++u) {
+      const int e = threadIdx.x + kWThreads * u;
+      dv[u][0] = dv[u][1] = uint4{0u, 0u, 0u, 0u};
+      const int c = e & 3, pr = (e >> 2) & 15, row = e >> 6;
+      const int y = y0 + (row & 3), z = z0 + (row >> 2);
+      if (e < kDzItems && y < d.ny && z < d.nz) {
+        const size_t p = (size_t)(x0 + 2 * pr) + (size_t)d.nx * (y + (size_t)d.ny * z);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) dv[u][h] = *(const uint4*)(dz + (p + h) * kC + 8 * c);
       }
     }
   };
-  f16v acc = {};
-  bf8 dv, av[4];
-  load(p0, dv, av);
-  for (size_t pb = p0; pb < p1; pb += kWBatch) {
+  // two voxels' 8 channels -> one 4-byte store per channel
+  auto put = [&](uint16_t* base, int stride, const uint4 (&v)[2]) {
+    const unsigned a[4] = {v[0].x, v[0].y, v[0].z, v[0].w}, b[4] = {v[1].x, v[1].y, v[1].z, v[1].w};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ld[vd][cd + e] = dv[e];
+    for (int q = 0; q < 4; ++q) {
+      *(unsigned*)(base + (2 * q) * stride) = (a[q] & 0xffffu) | (b[q] << 16);
+      *(unsigned*)(base + (2 * q + 1) * stride) = (a[q] >> 16) | (b[q] & 0xffff0000u);
+    }
+  };
+  f16v acc[3] = {};
+  if (b0 < b1) load(b0);
+  for (int b = b0; b < b1; ++b) {
+    __syncthreads();  // the previous brick's readers
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < kInPer; ++u) {
+      const int e = threadIdx.x + kWThreads * u;
+      const int c = e & 3, pr = (e >> 2) % 17, row = (e >> 2) / 17;
+      if (e < kInItems) put(li + 8 * c * kInChan + row * kInRow + 2 * pr, kInChan, iv[u]);
+    }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) la[w][va + 16 * u][ca + e] = av[u][e];
-    __syncthreads();
-    if (pb + kWBatch < p1) load(pb + kWBatch, dv, av);  // in flight during the MFMAs
-    if (t < 27) {
-#pragma unroll
-      for (int s = 0; s < kWBatch / 16; ++s) {
-        if (pb + 16 * s >= p1) break;
-        bf8 A, B;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          A[e] = ld[16 * s + 8 * half + e][col];     // A[co][k = voxel]
-          B[e] = la[w][16 * s + 8 * half + e][col];  // B[k = voxel][ci]
-        }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, B, acc, 0, 0, 0);
-      }
+    for (int u = 0; u < kDzPer; ++u) {
+      const int e = threadIdx.x + kWThreads * u;
+      const int c = e & 3, pr = (e >> 2) & 15, row = e >> 6;
+      if (e < kDzItems) put(ld + 8 * c * kDzChan + row * 32 + 2 * pr, kDzChan, dv[u]);
     }
     __syncthreads();
-  }
-  if (t >= 27) return;
-  float* out = partials + ((size_t)blockIdx.x * 27 + t) * kC * kC;
+    if (b + 1 < b1) load(b + 1);
+#pragma unroll 4
+    for (int row = 0; row < 16; ++row) {
+      const uint16_t* ir = li + col * kInChan + ((row & 3) + ty + kBY * ((row >> 2) + tz)) * kInRow;
+      const uint16_t* dr = ld + col * kDzChan + row * 32;
 #pragma unroll
-  for (int qi = 0; qi < 16; ++qi) {
-    const int co = 8 * (qi / 4) + 4 * half + (qi % 4);
-    out[co * kC + col] = acc[qi];
+      for (int s = 0; s < 2; ++s) {
+        const uint4 A = *(const uint4*)(dr + 16 * s + 8 * half);
+        const uint4 w = *(const uint4*)(ir + 16 * s + 8 * half);
+        const unsigned w4 = *(const unsigned*)(ir + 16 * s + 8 * half + 8);
+        const uint4 w1{__builtin_amdgcn_alignbit(w.y, w.x, 16), __builtin_amdgcn_alignbit(w.z, w.y, 16),
+                       __builtin_amdgcn_alignbit(w.w, w.z, 16), __builtin_amdgcn_alignbit(w4, w.w, 16)};
+        const uint4 w2{w.y, w.z, w.w, w4};
+        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(A), as_bf8(w), acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(A), as_bf8(w1), acc[1], 0, 0, 0);
+        acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(A), as_bf8(w2), acc[2], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int dx = 0; dx < 3; ++dx) {
+    float* out = partials + ((size_t)blockIdx.x * 27 + dx + 3 * ty + 9 * tz) * kC * kC;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) out[(8 * (q / 4) + 4 * half + q % 4) * kC + col] = acc[dx][q];
   }
 }
+constexpr unsigned kMidWeightsLds = (unsigned)((kC * kInChan + kC * kDzChan) * sizeof(uint16_t));
 
-// ---- layer 1 weight gradient: W[t][co][ci] += dz(p)[co] x(p + tap_t)[ci].
-// A batch of 64 voxels of the chunk is staged in LDS (dz and the 27 x 3
-// neighbour inputs); thread (t, 4 output channels) of 216 accumulates 12
-// weights over the batch, voxel by voxel in order.
-constexpr int kFirstWBatch = 64;
-__global__ void __launch_bounds__(256) k_first_weights(Dims d, const bf16* dz, const float* x, float* partials) {
-  __shared__ float ldz[kFirstWBatch][kC];
-  __shared__ float lx[kFirstWBatch][27 * 3];
-  const size_t p0 = (size_t)blockIdx.x * kChunk, p1 = p0 + kChunk < d.n ? p0 + kChunk : d.n;
-  const int slot = threadIdx.x;
-  const int t = slot / (kC / 4), co0 = 4 * (slot % (kC / 4));
-  float s[4][3] = {};
-  for (size_t pb = p0; pb < p1; pb += kFirstWBatch) {
-    const int m = (int)(p1 - pb < kFirstWBatch ? p1 - pb : kFirstWBatch);
-    for (int e = threadIdx.x; e < kFirstWBatch * kC; e += blockDim.x) {
-      const int v = e / kC, c = e % kC;
-      ldz[v][c] = v < m ? (float)dz[(pb + v) * kC + c] : 0.0f;
-    }
-    for (int e = threadIdx.x; e < kFirstWBatch * 27; e += blockDim.x) {
-      const int v = e / 27, tt = e % 27;
-      float x0 = 0.0f, x1 = 0.0f, x2 = 0.0f;
-      if (v < m) {
-        int i, j, k;
-        coords(d, pb + v, i, j, k);
-        const long long q = neighbour(d, i, j, k, tt);
-        if (q >= 0) {
-          x0 = x[3 * q];
-          x1 = x[3 * q + 1];
-          x2 = x[3 * q + 2];
-        }
-      }
-      lx[v][3 * tt] = x0;
-      lx[v][3 * tt + 1] = x1;
-      lx[v][3 * tt + 2] = x2;
-    }
-    __syncthreads();
-    if (slot < 27 * kC / 4) {
-      for (int v = 0; v < m; ++v) {
-        const float x0 = lx[v][3 * t], x1 = lx[v][3 * t + 1], x2 = lx[v][3 * t + 2];
+// ---- layer 1: W[t][co][ci] = sum_p dz(p)[co] x(p + tap_t)[ci].  A: the 32
+// output channels of two voxels, B: three groups of 32 of their 27 x 3 inputs.
+__global__ void __launch_bounds__(256) k_first_weights(Dims d, BrickGrid bg, int per, const bf16* __restrict__ dz,
+                                                       const float* __restrict__ x, float* partials) {
+  __shared__ float brick[3 * kBrickVox];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, col = lane & 31, half = lane >> 5;
+  int off[3];  // of column n = 32 m + col: tap n / 3, channel n % 3
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const float dv = ldz[v][co0 + c];
-          s[c][0] += dv * x0;
-          s[c][1] += dv * x1;
-          s[c][2] += dv * x2;
-        }
-      }
-    }
-    __syncthreads();
+  for (int m = 0; m < 3; ++m) {
+    const int n = 32 * m + col;
+    off[m] = n < 81 ? 3 * tap_offset(n / 3) + n % 3 : 0;
   }
-  if (slot < 27 * kC / 4) {
-    float* out = partials + (size_t)blockIdx.x * (27 * kC * 3) + (size_t)t * kC * 3;
+  const int bricks = bg.tiles_x * bg.tiles_y * bg.tiles_z;
+  f16v acc[3] = {};
+  for (int b = blockIdx.x * per; b < min(bricks, ((int)blockIdx.x + 1) * per); ++b) {
+    const int tx = b % bg.tiles_x, tyz = b / bg.tiles_x;
+    const int x0 = 32 * tx, y0 = 4 * (tyz % bg.tiles_y), z0 = 4 * (tyz / bg.tiles_y);
+    __syncthreads();  // the previous brick's readers
+    stage_brick<3>(d, x, x0, y0, z0, brick);
+    __syncthreads();
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int r = 0; r < 4; ++r) {
+      const int y = y0 + r, z = z0 + wv;
+      if (y >= d.ny || z >= d.nz) continue;  // uniform over the wavefront
+      const bf16* row = dz + ((size_t)x0 + (size_t)d.nx * (y + (size_t)d.ny * z)) * kC + col;
+      const int v0 = 1 + kBX * ((r + 1) + kBY * (wv + 1));
+      float a[16];
 #pragma unroll
-      for (int ci = 0; ci < 3; ++ci) out[(co0 + c) * 3 + ci] = s[c][ci];
+      for (int s = 0; s < 16; ++s) a[s] = (float)row[(2 * s + half) * kC];
+#pragma unroll
+      for (int s = 0; s < 16; ++s)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+          const float v = brick[3 * (v0 + 2 * s + half) + off[m]];
+          acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], 32 * m + col < 81 ? v : 0.0f, acc[m], 0, 0, 0);
+        }
+    }
+  }
+  float* out = partials + (size_t)(4 * blockIdx.x + wv) * (27 * kC * 3);
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    const int n = 32 * m + col;
+    if (n >= 81) continue;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) out[((n / 3) * kC + 8 * (q / 4) + 4 * half + q % 4) * 3 + n % 3] = acc[m][q];
   }
 }
 
@@ -719,13 +786,19 @@ int net_alloc(pcf_net* net, void** p, size_t bytes) {
   return PCF_OK;
 }
 
-int nchunks(const pcf_net* net) { return (int)((net->d.n + kChunk - 1) / kChunk); }
-
 // blocks of the k_brick launches
 BrickGrid brick_grid(const Dims& d) {
   return BrickGrid{d.nx / 32, (d.ny + 3) / 4, (d.nz + 3) / 4};
 }
 unsigned brick_blocks(const BrickGrid& bg) { return (unsigned)(bg.tiles_x * bg.tiles_y * bg.tiles_z); }
+// The weight gradients' bricks per workgroup: enough workgroups for the 256
+// CUs, then up to kBricksPer bricks each, which keeps the partial sums (108
+// KB per workgroup of a middle layer) small against the activations read.
+int weight_per(const BrickGrid& bg) {
+  return std::min(kBricksPer, std::max(1, (int)brick_blocks(bg) / 256));
+}
+int weight_blocks(const BrickGrid& bg) { return ((int)brick_blocks(bg) + weight_per(bg) - 1) / weight_per(bg); }
+int gelu_blocks(const Dims& d) { return (int)((d.n + kGeluChunk - 1) / kGeluChunk); }
 
 // out[0..size) = sum over the nc chunk partials (fixed order, two levels)
 void sum_chunks(pcf_net* net, int nc, int size, float* out) {
@@ -764,28 +837,29 @@ int net_backward_dout(pcf_net* net, const float* input) {
   hipStream_t s = net->stream;
   const unsigned vb = 256, vg = (unsigned)((d.n + vb - 1) / vb);
   const BrickGrid bg = brick_grid(d);
-  const int nc = nchunks(net);
+  const int per = weight_per(bg), wb = weight_blocks(bg), gb = gelu_blocks(d);
   const float* P = net->params;
   float* G = net->grads;
   // layer 6
-  hipLaunchKernelGGL(k_last_weights, dim3(nc), dim3(256), 0, s, d, net->dout, net->a[4], net->partials);
-  sum_chunks(net, nc, 27 * kC + 1, G + layer_offset(5));
+  hipLaunchKernelGGL(k_last_weights, dim3(wb), dim3(256), 0, s, d, bg, per, net->dout, net->a[4], net->partials);
+  sum_chunks(net, 4 * wb, 27 * kC + 1, G + layer_offset(5));
   hipLaunchKernelGGL(k_last_data, dim3(vg), dim3(vb), 0, s, d, net->dout, P + layer_offset(5), net->g);
   // layers 5..2
   for (int l = 4; l >= 1; --l) {
-    hipLaunchKernelGGL(k_gelu_back, dim3(nc), dim3(256), 0, s, d, net->g, net->z[l], net->dzb, net->partials);
-    sum_chunks(net, nc, kC, G + layer_offset(l) + 27 * kC * kC);
-    hipLaunchKernelGGL(k_mid_weights, dim3(nc, 7), dim3(256), 0, s, d, net->dzb, net->a[l - 1], net->partials);
-    sum_chunks(net, nc, 27 * kC * kC, G + layer_offset(l));
+    hipLaunchKernelGGL(k_gelu_back, dim3(gb), dim3(256), 0, s, d, net->g, net->z[l], net->dzb, net->partials);
+    sum_chunks(net, gb, kC, G + layer_offset(l) + 27 * kC * kC);
+    hipLaunchKernelGGL(k_mid_weights, dim3(wb), dim3(kWThreads), kMidWeightsLds, s, d, bg, per, net->dzb, net->a[l - 1],
+                       net->partials);
+    sum_chunks(net, wb, 27 * kC * kC, G + layer_offset(l));
     hipLaunchKernelGGL((k_brick<KIND_MID, MID_DATA>), dim3(brick_blocks(bg)), dim3(256), 0, s, d, bg,
                        (const void*)net->dzb, net->wt16 + (size_t)(l - 1) * 27 * kC * kC, nullptr, nullptr, nullptr,
                        net->g);
   }
   // layer 1
-  hipLaunchKernelGGL(k_gelu_back, dim3(nc), dim3(256), 0, s, d, net->g, net->z[0], net->dzb, net->partials);
-  sum_chunks(net, nc, kC, G + layer_offset(0) + 27 * kC * 3);
-  hipLaunchKernelGGL(k_first_weights, dim3(nc), dim3(256), 0, s, d, net->dzb, input, net->partials);
-  sum_chunks(net, nc, 27 * kC * 3, G + layer_offset(0));
+  hipLaunchKernelGGL(k_gelu_back, dim3(gb), dim3(256), 0, s, d, net->g, net->z[0], net->dzb, net->partials);
+  sum_chunks(net, gb, kC, G + layer_offset(0) + 27 * kC * 3);
+  hipLaunchKernelGGL(k_first_weights, dim3(wb), dim3(256), 0, s, d, bg, per, net->dzb, input, net->partials);
+  sum_chunks(net, 4 * wb, 27 * kC * 3, G + layer_offset(0));
   PCF_HIP(hipGetLastError());
   return PCF_OK;
 }
@@ -983,10 +1057,19 @@ int pcf_net_create(int32_t nx, int32_t ny, int32_t nz, int32_t training, pcf_net
     if ((rc = net_alloc(net, (void**)&net->dout, N * sizeof(float)))) return fail(rc);
     if ((rc = net_alloc(net, (void**)&net->g, N * kC * sizeof(float)))) return fail(rc);
     if ((rc = net_alloc(net, (void**)&net->dzb, N * kC * sizeof(bf16)))) return fail(rc);
-    const size_t part = (size_t)nchunks(net) * 27 * kC * kC;
+    // the partial sums of each use (sum_chunks: chunks, values per chunk)
+    const size_t wb = (size_t)weight_blocks(brick_grid(net->d)), gb = (size_t)gelu_blocks(net->d);
+    const size_t uses[4][2] = {{wb, 27 * kC * kC}, {4 * wb, 27 * kC * 3}, {4 * wb, 27 * kC + 1}, {gb, kC}};
+    size_t part = 0, groups = 0;
+    for (const auto& u : uses) {
+      part = std::max(part, u[0] * u[1]);
+      groups = std::max(groups, (u[0] + kSumGroup - 1) / kSumGroup * u[1]);
+    }
     if ((rc = net_alloc(net, (void**)&net->partials, part * sizeof(float)))) return fail(rc);
-    const size_t ngroups = (size_t)(nchunks(net) + kSumGroup - 1) / kSumGroup;
-    if ((rc = net_alloc(net, (void**)&net->groups, ngroups * 27 * kC * kC * sizeof(float)))) return fail(rc);
+    if ((rc = net_alloc(net, (void**)&net->groups, groups * sizeof(float)))) return fail(rc);
+    if (hipFuncSetAttribute((const void*)k_mid_weights, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)kMidWeightsLds) != hipSuccess)
+      return fail(PCF_E_HIP);
     if ((rc = net_alloc(net, (void**)&net->loss_partials, 1024 * sizeof(double)))) return fail(rc);
     if (hipMemsetAsync(net->adam_m, 0, kParams * sizeof(float), net->stream) != hipSuccess) return fail(PCF_E_HIP);
     if (hipMemsetAsync(net->adam_v, 0, kParams * sizeof(float), net->stream) != hipSuccess) return fail(PCF_E_HIP);
