@@ -140,11 +140,51 @@ __device__ __forceinline__ void line_step32(const LineArgs<CT>& A, const BT* __r
       if (t.k0 + u < nz) line_store<W>(out + t.o + sxy * u, r[u]);
   }
 }
+// commit: the kernel before was a FUSE_P one
 template <int W, int NPL, bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
 __global__ void __launch_bounds__(W == 4 ? 512 : 1024) __attribute__((amdgpu_waves_per_eu(W == 4 ? 2 : 4, W == 4 ? 2 : 4)))
-    k_line_step32(LineArgs<CT> A, const BT* __restrict__ b, OutT* __restrict__ out, const SolverScalars* sc) {
-  if (sc && sc->done) return;
+    k_line_step32(LineArgs<CT> A, const BT* __restrict__ b, OutT* __restrict__ out, const SolverScalars* sc,
+                  SolverScalars* commit) {
+  if (!FIRST && commit) {
+    if (!fuse_commit(commit)) return;
+  } else if (sc && sc->done) {
+    return;
+  }
   line_step32<W, NPL, FIRST, PRO, CT, BT, OutT>(A, b, out, xcd_block(blockIdx.x, gridDim.x));
+}
+
+// The first pseudo-time step of the vector that a fused BiCGSTAB step updates
+// first.
+template <int NPL, int FUSE>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)))
+    k_line_fuse32(LineArgs<float> A, BicgFuse F, float* __restrict__ out) {
+  extern __shared__ float line_shared[];
+  const LineThread<float, 1, NPL> t(xcd_block(blockIdx.x, gridDim.x), A.nx, A.ny, A.nz);
+  const size_t sxy = (size_t)A.nx * A.ny;
+  FuseOperands<FUSE, NPL> X;
+  if (t.act) {
+#pragma unroll
+    for (int u = 0; u < NPL; ++u) X.load(F, u, t.o + sxy * (ptrdiff_t)(min(t.k0 + u, A.nz - 1) - t.k0));
+  }
+  FuseScalars S;
+  if (!fuse_scalars<FUSE>(F, S)) return;
+  float r[NPL][1];
+#pragma unroll
+  for (int u = 0; u < NPL; ++u) {
+    r[u][0] = 0.0f;
+    if (t.act && t.k0 + u < A.nz) {
+      const double x = fuse_value(X, S, u);
+      F.dst[t.o + sxy * u] = x;
+      r[u][0] = A.deta * (0.0f - (float)x);
+    }
+  }
+  line_solve_segments<float, 1, NPL>(A.factors + t.c * 3 * kTileCols + t.tx, t.k0, A.nz, t.tx, t.seg,
+                                     blockDim.x / kTileCols, r, line_shared);
+  if (t.act) {
+#pragma unroll
+    for (int u = 0; u < NPL; ++u)
+      if (t.k0 + u < A.nz) out[t.o + sxy * u] = r[u][0];
+  }
 }
 
 // The same step for columns of more than kLineMaxNz levels, one thread per
@@ -596,7 +636,7 @@ LineArgs<CT> line_args(const MgLevel& L, const float* s, const float* e = nullpt
 // level C): s is s + omega P e.  out must differ from s.
 template <bool FIRST, typename BT, typename OutT>
 void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, OutT* out, const SolverScalars* sc,
-               const float* e = nullptr, const MgLevel* C = nullptr) {
+               const float* e = nullptr, const MgLevel* C = nullptr, SolverScalars* commit = nullptr) {
   ProfScope prof(st, FIRST ? PCF_K_PC_THOMAS : PCF_K_PC_RHS);
   auto go = [&](auto ct, auto pro) {
     constexpr bool PRO = decltype(pro)::value;
@@ -611,7 +651,7 @@ void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, Out
         constexpr int W = decltype(w)::value, NPL = decltype(npl)::value;
         const int threads = kTileCols / W * ((L.nz + NPL - 1) / NPL);
         hipLaunchKernelGGL((k_line_step32<W, NPL, FIRST, PRO, CT, BT, OutT>), grd, dim3(threads),
-                           (line_lds<float, W>(threads)), st->stream, A, b, out, sc);
+                           (line_lds<float, W>(threads)), st->stream, A, b, out, sc, commit);
       });
   };
   if constexpr (FIRST) {
@@ -624,6 +664,21 @@ void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, Out
     if (bf16_storage(st)) pick(uint16_t{});
     else pick(float{});
   }
+}
+
+// The first pseudo-time step of the finest level with a fused BiCGSTAB step.
+void line_fuse(pcf_state* st, const MgLevel& L, const BicgFuse& F, int fuse, float* out) {
+  ProfScope prof(st, PCF_K_PC_THOMAS);
+  const LineArgs<float> A = line_args<float>(L, nullptr);
+  auto go = [&](auto npl) {
+    constexpr int NPL = decltype(npl)::value;
+    const dim3 grd(LineTile<float>::count(L.nx, L.ny)), blk(kTileCols * ((L.nz + NPL - 1) / NPL));
+    const unsigned lds = line_lds<float, 1>((int)blk.x);
+    if (fuse == FUSE_P) hipLaunchKernelGGL((k_line_fuse32<NPL, FUSE_P>), grd, blk, lds, st->stream, A, F, out);
+    else hipLaunchKernelGGL((k_line_fuse32<NPL, FUSE_S>), grd, blk, lds, st->stream, A, F, out);
+  };
+  if (L.nz > 128) go(std::integral_constant<int, 16>{});
+  else go(std::integral_constant<int, 8>{});
 }
 
 // Pack a level's coefficients and factors for the line steps.
@@ -726,7 +781,8 @@ MgCoefs coefs_of(const MgLevel& L) {
 // the buffer holding the result.
 template <typename BT>
 float* mg_smooth(pcf_state* st, const MgLevel& L, const BT* b, float* s, const float* e, const MgLevel* C, int steps,
-                 double* out64, const Lay& ol, const SolverScalars* sc) {
+                 double* out64, const Lay& ol, const SolverScalars* sc, const BicgFuse* F = nullptr,
+                 int fuse = FUSE_NONE) {
   const bool col = column_path(L);
   const size_t nc = columns(L);
   int step = 0;
@@ -746,6 +802,8 @@ float* mg_smooth(pcf_state* st, const MgLevel& L, const BT* b, float* s, const f
                              st->stream, coefs_of(L), L.P, L.E, L.Q, b, nullptr, nullptr, 0.0f, 0, 0, l, l, L.s,
                              last ? ol : l, L.deta, sc);
       });
+    } else if (fuse != FUSE_NONE) {
+      line_fuse(st, L, *F, fuse, L.s);
     } else {
       if (last && out64)
         line_step<true, BT, double>(st, L, b, nullptr, out64, sc);
@@ -789,10 +847,11 @@ float* mg_smooth(pcf_state* st, const MgLevel& L, const BT* b, float* s, const f
     }
     const float* pro = step == 0 ? e : nullptr;
     float* dst = s == L.s ? L.rhs : L.s;
+    SolverScalars* commit = fuse == FUSE_P && step == 1 ? F->sc : nullptr;
     if (last && out64)
-      line_step<false, BT, double>(st, L, b, s, out64, sc, pro, C);
+      line_step<false, BT, double>(st, L, b, s, out64, sc, pro, C, commit);
     else
-      line_step<false, BT, float>(st, L, b, s, dst, sc, pro, C);
+      line_step<false, BT, float>(st, L, b, s, dst, sc, pro, C, commit);
     s = dst;
   }
   return s;
@@ -861,11 +920,13 @@ float* mg_coarsest(pcf_state* st, const MgLevel& L, const BT* b, double* out64, 
 // its result to out64; returns the buffer holding the level's result, in
 // layout ol.
 template <typename BT>
-float* mg_vcycle(pcf_state* st, size_t l, const BT* b, double* out64, const Lay& ol, const SolverScalars* sc) {
+float* mg_vcycle(pcf_state* st, size_t l, const BT* b, double* out64, const Lay& ol, const SolverScalars* sc,
+                 const BicgFuse* F = nullptr, int fuse = FUSE_NONE) {
   const MgLevel& L = st->mg[l];
   if (l + 1 == st->mg.size()) return mg_coarsest<BT>(st, L, b, out64, ol, sc);
   const MgLevel& C = st->mg[l + 1];
-  float* s = mg_smooth<BT>(st, L, b, nullptr, nullptr, nullptr, st->cfg.mg_smoothing_steps, nullptr, lay_of(L), sc);
+  float* s =
+      mg_smooth<BT>(st, L, b, nullptr, nullptr, nullptr, st->cfg.mg_smoothing_steps, nullptr, lay_of(L), sc, F, fuse);
   mg_restrict<BT>(st, L, C, b, s, sc);
   const Lay el = correction_layout(L, C);
   const float* e = mg_vcycle<float>(st, l + 1, C.b, nullptr, el, sc);
@@ -874,12 +935,21 @@ float* mg_vcycle(pcf_state* st, size_t l, const BT* b, double* out64, const Lay&
 
 }  // namespace
 
+// Whether the solve's first two kernels are line steps of the finest level.
+bool fusable_mixed(const pcf_state* st) {
+  const MgLevel& L = st->mg[0];
+  if (!L.coefs || L.nz > kLineMaxNz) return false;
+  if (st->cfg.preconditioner_type == PCF_PC_MULTIGRID) return st->mg.size() > 1 && st->cfg.mg_smoothing_steps >= 2;
+  return st->cfg.preconditioner_iterations >= 2;
+}
+
 // M^-1 sin -> sout (FP64 in and out, FP32 inside); sout must not alias sin.
-int precondition_mixed(pcf_state* st, const double* sin, double* sout, const SolverScalars* sc) {
+int precondition_mixed(pcf_state* st, const double* sin, double* sout, const SolverScalars* sc, const BicgFuse* F,
+                       int fuse) {
   int rc = prepare_mixed(st);
   if (rc) return rc;
   if (st->cfg.preconditioner_type == PCF_PC_MULTIGRID) {
-    mg_vcycle<double>(st, 0, sin, sout, lay_of(st->mg[0]), sc);
+    mg_vcycle<double>(st, 0, sin, sout, lay_of(st->mg[0]), sc, F, fuse);
     PCF_HIP(hipGetLastError());
     return PCF_OK;
   }
@@ -889,13 +959,15 @@ int precondition_mixed(pcf_state* st, const double* sin, double* sout, const Sol
     line_step<true, double, double>(st, L, sin, nullptr, sout, sc);
   } else {
     float* cur = L.s;  // FP32 iterate between pseudo-time steps
-    line_step<true, double, float>(st, L, sin, nullptr, cur, sc);
+    if (fuse != FUSE_NONE) line_fuse(st, L, *F, fuse, cur);
+    else line_step<true, double, float>(st, L, sin, nullptr, cur, sc);
     for (int it = 2; it <= iters; ++it) {
       float* next = cur == L.s ? L.rhs : L.s;
+      SolverScalars* commit = fuse == FUSE_P && it == 2 ? F->sc : nullptr;
       if (it == iters)
-        line_step<false, double, double>(st, L, sin, cur, sout, sc);
+        line_step<false, double, double>(st, L, sin, cur, sout, sc, nullptr, nullptr, commit);
       else
-        line_step<false, double, float>(st, L, sin, cur, next, sc);
+        line_step<false, double, float>(st, L, sin, cur, next, sc, nullptr, nullptr, commit);
       cur = next;
     }
   }

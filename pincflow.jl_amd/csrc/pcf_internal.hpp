@@ -107,7 +107,26 @@ struct SolverScalars {
   double divl2, divl2_norm;
   int32_t done;    // 1 once res / b_norm <= tol; 2: stopped at the ensemble solve's maxit
   int32_t niter;
-  int32_t pad[2];
+  int32_t fresh;   // 1 until the first iteration has begun (fused iterations)
+  int32_t pad;
+  // the last iteration's check, found by the kernel that begins the next one
+  // while others still read the fields above; the kernel after it moves them
+  // over (fused iterations)
+  struct {
+    double rr, res, beta, rr0;
+    int32_t done, niter;
+  } next;
+};
+
+// A BiCGSTAB step fused into the preconditioner's first kernel
+// (solver_common.hpp).
+struct BicgFuse {
+  const double *r, *v;
+  double* dst;  // p or s, the vector being preconditioned
+  const double* partials;
+  int nparts;
+  double nxyz;
+  SolverScalars* sc;
 };
 
 constexpr int kReduceBlock = 256;     // threads per reduction block
@@ -415,7 +434,10 @@ int dot(pcf_state* st, const double* a, const double* b, double* out);
 
 // ---- mixed.hip -------------------------------------------------------------
 int apply_bicgstab_mixed(pcf_state* st, double tolref, double dt, int* niter);
-int precondition_mixed(pcf_state* st, const double* sin, double* sout, const SolverScalars* sc);
+// F, fuse: the BiCGSTAB step that the first kernel does before (solver_common.hpp), for the solves of fusable_mixed
+int precondition_mixed(pcf_state* st, const double* sin, double* sout, const SolverScalars* sc, const BicgFuse* F,
+                       int fuse);
+bool fusable_mixed(const pcf_state* st);
 // the ensemble batch's FP32 line preconditioner: a member's grid, whether it
 // covers the member, and the launches over a list (threads: the largest block)
 int ensemble_line_blocks(const pcf_state* st);

@@ -672,9 +672,11 @@ struct LineRead64 {
 constexpr int kLine64MaxNz = 256;
 inline unsigned line64_lds(int nz) { return (unsigned)(4 * nz * LineTile<double>::cols * sizeof(double)); }
 
-// b_at(o): the vector being preconditioned at cell o
-template <int NPL, bool FIRST, class B>
-__device__ __forceinline__ void line_step64(const LineArgs64& A, B b_at, double* __restrict__ out, int tile) {
+// FIRST: from s = 0, b updated by F's BiCGSTAB step first (FUSE); false if
+// that ended the solve.
+template <int NPL, int DEPTH, bool FIRST, int FUSE>
+__device__ __forceinline__ bool line_step64(const LineArgs64& A, const double* __restrict__ b, const BicgFuse& F,
+                                            double* __restrict__ out, int tile) {
   extern __shared__ double line_shared64[];
   constexpr int cols = LineTile<double>::cols;
   const int nx = A.nx, ny = A.ny, nz = A.nz;
@@ -691,14 +693,36 @@ __device__ __forceinline__ void line_step64(const LineArgs64& A, B b_at, double*
     q[u] = fu[2 * cols];
   }
   if constexpr (FIRST) {
+    FuseOperands<FUSE, NPL> X;
+    // (idle threads of a partial tile read no vector that others write)
+    if (t.act) {
 #pragma unroll
-    for (int u = 0; u < NPL; ++u)  // idle threads repeat a cell of the grid
-      r[u][0] = b_at(t.o + sxy * (ptrdiff_t)(min(t.k0 + u, nz - 1) - t.k0), t.act && t.k0 + u < nz);
+      for (int u = 0; u < NPL; ++u) {
+        const size_t o = t.o + sxy * (ptrdiff_t)(min(t.k0 + u, nz - 1) - t.k0);
+        if constexpr (FUSE == FUSE_NONE) X.p[u] = b[o];
+        else X.load(F, u, o);
+      }
+    }
+    FuseScalars S;
+    if constexpr (FUSE != FUSE_NONE)
+      if (!fuse_scalars<FUSE>(F, S)) return false;
 #pragma unroll
-    for (int u = 0; u < NPL; ++u) r[u][0] = 0.0 + A.deta * (0.0 - r[u][0]);
+    for (int u = 0; u < NPL; ++u) {
+      r[u][0] = 0.0;
+      if (t.act && t.k0 + u < nz) {
+        double x;
+        if constexpr (FUSE == FUSE_NONE) {
+          x = X.p[u];
+        } else {
+          x = fuse_value(X, S, u);
+          F.dst[t.o + sxy * u] = x;
+        }
+        r[u][0] = 0.0 + A.deta * (0.0 - x);
+      }
+    }
   } else {
-    line_rhs<double, 1, NPL, NPL == 4 ? 1 : 0, false, double, double>(A.coefs + t.c * T_COUNT * cols + t.tx,
-                                                                      LineRead64{A}, b_at, nx, ny, nz, A.deta, t.i, t.j,
+    line_rhs<double, 1, NPL, DEPTH, false, double, double>(A.coefs + t.c * T_COUNT * cols + t.tx,
+                                                                      LineRead64{A}, b, nx, ny, nz, A.deta, t.i, t.j,
                                                                       t.k0, r);
   }
 #pragma unroll
@@ -764,18 +788,28 @@ __device__ __forceinline__ void line_step64(const LineArgs64& A, B b_at, double*
     for (int u = 0; u < NPL; ++u)
       if (t.k0 + u < nz) out[t.o + sxy * u] = lr[(t.k0 + u) * cols + t.tx];
   }
+  return true;
 }
+// The first pseudo-time step of b (FUSE_NONE), or of the vector that a fused
+// BiCGSTAB step updates first.
+template <int NPL, int FUSE>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    k_line_first64(LineArgs64 A, const double* __restrict__ b, BicgFuse F, double* __restrict__ out,
+                   const SolverScalars* sc) {
+  if (FUSE == FUSE_NONE && sc && sc->done) return;
+  line_step64<NPL, 0, true, FUSE>(A, b, F, out, xcd_block(blockIdx.x, gridDim.x));
+}
+// commit: the kernel before was a FUSE_P one
 template <int NPL>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-    k_line_first64(LineArgs64 A, const double* __restrict__ b, double* __restrict__ out, const SolverScalars* sc) {
-  if (sc && sc->done) return;
-  line_step64<NPL, true>(A, [&](size_t o, bool) { return b[o]; }, out, xcd_block(blockIdx.x, gridDim.x));
-}
-template <int NPL>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-    k_line_step64(LineArgs64 A, const double* __restrict__ b, double* __restrict__ out, const SolverScalars* sc) {
-  if (sc && sc->done) return;
-  line_step64<NPL, false>(A, b, out, xcd_block(blockIdx.x, gridDim.x));
+    k_line_step64(LineArgs64 A, const double* __restrict__ b, double* __restrict__ out, const SolverScalars* sc,
+                  SolverScalars* commit) {
+  if (commit) {
+    if (!fuse_commit(commit)) return;
+  } else if (sc && sc->done) {
+    return;
+  }
+  line_step64<NPL, NPL <= 4 ? 1 : 0, false, FUSE_NONE>(A, b, BicgFuse{}, out, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // rhs of a later pseudo-time step: s + deta (L_h s - sin) (apply_preconditioner!.jl:62-63)
@@ -1475,31 +1509,56 @@ static void launch_thomas(pcf_state* st, const double* src, double* out, const S
                        g.nx, g.ny, g.nz, st->deta, sc);
 }
 
-// f(NPL), the levels per thread of the FP64 line steps
+// f(NPL), the levels per thread of the FP64 line steps.  Two on a handful of
+// tiles, where a thread's own loads set the time (40 x 1 x 40: 7.3 ms per
+// time step against 8.0), four where the tiles share the memory system
+// (75 x 53 x 41: 15 us against 18 per step).
+constexpr int kLine64FewTiles = 64;
 template <class F>
-static void with_line64(int nz, F&& f) {
-  if (nz <= 128) f(std::integral_constant<int, 4>{});
-  else f(std::integral_constant<int, 8>{});
+static void with_line64(const Geo& g, F&& f) {
+  using std::integral_constant;
+  if (g.nz > 128) f(integral_constant<int, 8>{});
+  else if (g.nz <= 64 && LineTile<double>::count(g.nx, g.ny) <= kLine64FewTiles) f(integral_constant<int, 2>{});
+  else f(integral_constant<int, 4>{});
 }
 static LineArgs64 line_args64(pcf_state* st, const double* s) {
   return LineArgs64{st->pc_coefs, st->pc_factors, s, st->g.nx, st->g.ny, st->g.nz, st->deta};
 }
-template <bool FIRST>
-static void line_step(pcf_state* st, const double* b, const double* s, double* out, const SolverScalars* sc) {
+static dim3 line_block64(const Geo& g, int npl) {
+  return dim3((LineTile<double>::cols * ((g.nz + npl - 1) / npl) + 63) / 64 * 64);
+}
+static void line_first(pcf_state* st, const double* b, double* out, const SolverScalars* sc, const BicgFuse* F,
+                       int fuse) {
   const Geo& g = st->g;
-  with_line64(g.nz, [&](auto npl) {
+  with_line64(g, [&](auto npl) {
     constexpr int NPL = decltype(npl)::value;
-    const dim3 grd(LineTile<double>::count(g.nx, g.ny)), blk(LineTile<double>::cols * ((g.nz + NPL - 1) / NPL));
-    if constexpr (FIRST)
-      hipLaunchKernelGGL(k_line_first64<NPL>, grd, blk, line64_lds(g.nz), st->stream, line_args64(st, s), b, out, sc);
+    const dim3 grd(LineTile<double>::count(g.nx, g.ny)), blk = line_block64(g, NPL);
+    const unsigned lds = line64_lds(g.nz);
+    const LineArgs64 A = line_args64(st, nullptr);
+    if (fuse == FUSE_P)
+      hipLaunchKernelGGL((k_line_first64<NPL, FUSE_P>), grd, blk, lds, st->stream, A, b, *F, out, sc);
+    else if (fuse == FUSE_S)
+      hipLaunchKernelGGL((k_line_first64<NPL, FUSE_S>), grd, blk, lds, st->stream, A, b, *F, out, sc);
     else
-      hipLaunchKernelGGL(k_line_step64<NPL>, grd, blk, line64_lds(g.nz), st->stream, line_args64(st, s), b, out, sc);
+      hipLaunchKernelGGL((k_line_first64<NPL, FUSE_NONE>), grd, blk, lds, st->stream, A, b, BicgFuse{}, out, sc);
+  });
+}
+static void line_step(pcf_state* st, const double* b, const double* s, double* out, const SolverScalars* sc,
+                      SolverScalars* commit) {
+  const Geo& g = st->g;
+  with_line64(g, [&](auto npl) {
+    constexpr int NPL = decltype(npl)::value;
+    hipLaunchKernelGGL(k_line_step64<NPL>, dim3(LineTile<double>::count(g.nx, g.ny)), line_block64(g, NPL),
+                       line64_lds(g.nz), st->stream, line_args64(st, s), b, out, sc, commit);
   });
 }
 
 // M^-1 sin -> sout with preconditioner_iterations pseudo-time steps.  sout
 // must not alias sin.  `sc` (may be null) lets a converged solve skip it.
-static int precondition(pcf_state* st, const double* sin, double* sout, const SolverScalars* sc) {
+// fuse != FUSE_NONE (line steps, two pseudo-time steps or more): F's BiCGSTAB
+// step runs in the first kernel, sin being the vector it updates.
+static int precondition(pcf_state* st, const double* sin, double* sout, const SolverScalars* sc,
+                        const BicgFuse* F = nullptr, int fuse = FUSE_NONE) {
   const Geo& g = st->g;
   int rc = pc_factors(st);
   if (rc) return rc;
@@ -1508,12 +1567,12 @@ static int precondition(pcf_state* st, const double* sin, double* sout, const So
     double* cur = iters == 1 ? sout : st->pc_tmp;
     {
       ProfScope prof(st, PCF_K_PC_THOMAS);
-      line_step<true>(st, sin, nullptr, cur, sc);
+      line_first(st, sin, cur, sc, F, fuse);
     }
     for (int it = 2; it <= iters; ++it) {
       ProfScope prof(st, PCF_K_PC_RHS);
       double* next = it == iters ? sout : (cur == st->pc_tmp ? st->pc_rhs : st->pc_tmp);
-      line_step<false>(st, sin, cur, next, sc);
+      line_step(st, sin, cur, next, sc, fuse == FUSE_P && it == 2 ? F->sc : nullptr);
       cur = next;
     }
     PCF_HIP(hipGetLastError());
@@ -1549,7 +1608,7 @@ static int precondition(pcf_state* st, const double* sin, double* sout, const So
 // apply_preconditioner! in the configured precision (and, for the mixed
 // solve, the configured preconditioner).
 int apply_preconditioner(pcf_state* st, const double* sin, double* sout) {
-  if (st->cfg.precision == PCF_PRECISION_MIXED) return precondition_mixed(st, sin, sout, nullptr);
+  if (st->cfg.precision == PCF_PRECISION_MIXED) return precondition_mixed(st, sin, sout, nullptr, nullptr, FUSE_NONE);
   return precondition(st, sin, sout, nullptr);
 }
 
@@ -1573,6 +1632,13 @@ int dot(pcf_state* st, const double* a, const double* b, double* out) {
 // keeps it consistent with the FP64 residual recurrence; guess (may be null):
 // the solve starts from x0 = guess_scale * guess instead of 0, unless x0
 // leaves a residual no smaller than |b|, in which case it starts from 0.
+//
+// Most partials of an apply that the blocks of a fused iteration sum again
+// each, and the solves that run fused iterations: those whose preconditioner
+// is line steps of two pseudo-time steps or more.
+constexpr int kFusePartials = 2048;
+static bool fusable(const pcf_state* st) { return st->pc_coefs && st->cfg.preconditioner_iterations >= 2; }
+
 int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess, double guess_scale,
                   int* niter_out) {
   const Geo& g = st->g;
@@ -1586,8 +1652,9 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
   // stage_iterations iterations (flexible BiCGSTAB: the textbook update below
   // keeps x consistent with the residual recurrence whatever M^-1 does)
   const bool stage = mixed && pc && st->stage_net && st->stage_iterations > 0;
-  auto prec = [&](const double* in, double* out, const SolverScalars* s, int iter) -> int {
-    int rc0 = mixed ? precondition_mixed(st, in, out, s) : precondition(st, in, out, s);
+  auto prec = [&](const double* in, double* out, const SolverScalars* s, int iter, const BicgFuse* F,
+                  int fuse) -> int {
+    int rc0 = mixed ? precondition_mixed(st, in, out, s, F, fuse) : precondition(st, in, out, s, F, fuse);
     if (rc0 == PCF_OK && stage && iter <= st->stage_iterations) rc0 = learned_stage(st, in, out, s);
     return rc0;
   };
@@ -1665,6 +1732,13 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
   PCF_HIP(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
   int converged_at = -1, last_seen = 0;
   int rc = PCF_OK;
+  // On small grids the vector and scalar steps run inside the kernels around
+  // them; the check of an iteration is then made by the next one's first
+  // kernel, and the host sees it one iteration later.
+  const bool fused = pc && !stage && (mixed ? fusable_mixed(st) : fusable(st)) && aparts <= kFusePartials;
+  const int vgrid = fused ? std::min(kVecGrid, (int)blocks_for((long long)N, kReduceBlock)) : kVecGrid;
+  const BicgFuse fuse_p{st->br, st->bv, st->bp, st->partials, vgrid, nxyz, sc};
+  const BicgFuse fuse_s{st->br, st->bv, st->bs, st->partials, aparts, nxyz, sc};
   // One BiCGSTAB iteration's launches.  Every argument is fixed for the
   // state (the scalars live in device memory), so the sequence is captured
   // once into a hipGraph and replayed as one launch per iteration; the
@@ -1672,19 +1746,19 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
   auto iteration = [&](int jb) -> int {
     int rc1 = PCF_OK;
     // v = A M^-1 p, <v, r0>
-    if ((rc1 = pc ? prec(st->bp, ybuf, sc, jb) : PCF_OK)) return rc1;
+    if ((rc1 = pc ? prec(st->bp, ybuf, sc, jb, &fuse_p, fused ? FUSE_P : FUSE_NONE) : PCF_OK)) return rc1;
     const double* vin = pc ? ybuf : st->bp;
     {
       ProfScope prof(st, PCF_K_APPLY_TOTAL_DOT);
       launch_total<1>(st, vin, st->bv, st->br0, sc);
     }
-    {
+    if (!fused) {
       ProfScope prof(st, PCF_K_BICG_VECTOR);
       hipLaunchKernelGGL(k_bicg_alpha, dim3(1), dim3(1024), 0, st->stream, st->partials, aparts, sc);
       hipLaunchKernelGGL(k_bicg_s, dim3(kVecGrid), dim3(256), 0, st->stream, st->br, st->bv, st->bs, N, sc);
     }
     // t = A M^-1 s, <t, s>, <t, t>
-    if ((rc1 = pc ? prec(st->bs, zbuf, sc, jb) : PCF_OK)) return rc1;
+    if ((rc1 = pc ? prec(st->bs, zbuf, sc, jb, &fuse_s, fused ? FUSE_S : FUSE_NONE) : PCF_OK)) return rc1;
     const double* sin2 = pc ? zbuf : st->bs;
     {
       ProfScope prof(st, PCF_K_APPLY_TOTAL_DOT);
@@ -1694,13 +1768,15 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
       ProfScope prof(st, PCF_K_BICG_VECTOR);
       hipLaunchKernelGGL(k_bicg_omega, dim3(1), dim3(1024), 0, st->stream, st->partials, aparts, sc);
       if (yz)
-        hipLaunchKernelGGL(k_bicg_xr_yz, dim3(kVecGrid), dim3(kReduceBlock), 0, st->stream, st->solution, ybuf, zbuf,
+        hipLaunchKernelGGL(k_bicg_xr_yz, dim3(vgrid), dim3(kReduceBlock), 0, st->stream, st->solution, ybuf, zbuf,
                            st->bs, st->bt, st->br, st->br0, N, st->partials, sc);
       else
-        hipLaunchKernelGGL(k_bicg_xr, dim3(kVecGrid), dim3(kReduceBlock), 0, st->stream, st->solution, st->bp,
+        hipLaunchKernelGGL(k_bicg_xr, dim3(vgrid), dim3(kReduceBlock), 0, st->stream, st->solution, st->bp,
                            st->bs, st->bt, st->br, st->br0, N, st->partials, sc);
-      hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(1024), 0, st->stream, st->partials, kVecGrid, sc, nxyz);
-      hipLaunchKernelGGL(k_bicg_p, dim3(kVecGrid), dim3(256), 0, st->stream, st->bp, st->br, st->bv, N, sc);
+      if (!fused) {
+        hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(1024), 0, st->stream, st->partials, kVecGrid, sc, nxyz);
+        hipLaunchKernelGGL(k_bicg_p, dim3(kVecGrid), dim3(256), 0, st->stream, st->bp, st->br, st->bv, N, sc);
+      }
     }
     PCF_HIP(hipGetLastError());
     return PCF_OK;
@@ -1742,6 +1818,10 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
     }
   }
   if (rc == PCF_OK && converged_at < 0) {
+    if (fused) {  // the last iteration's check
+      hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(1024), 0, st->stream, st->partials, vgrid, sc, nxyz);
+      PCF_HIP(hipMemcpyAsync(hs + (last_seen & 1), sc, sizeof(SolverScalars), hipMemcpyDeviceToHost, st->stream));
+    }
     PCF_HIP(hipStreamSynchronize(st->stream));
     int slot = (last_seen + 1) & 1;
     // the newest copy holds the final state
