@@ -314,47 +314,44 @@ __global__ void __launch_bounds__(64) k_mg_factors(const float* ac, const float*
   }
 }
 
-// r = b - A s on one level, one thread per cell in memory order.
-template <typename BT>
-__global__ void __launch_bounds__(256) k_mg_resid(MgCoefs A, const BT* __restrict__ b, const float* __restrict__ s,
-                                                  float* __restrict__ r, Lay l, const SolverScalars* sc) {
+// b_coarse = R (b - A s) on a level of any layout: block (64, FX FY) of 64
+// levels of one coarse column, one thread per fine cell, whose residuals are
+// summed in LDS in the order of the fine columns.
+template <int FX, int FY, typename BT>
+__global__ void __launch_bounds__(256) k_resid_restrict_any(MgCoefs A, const BT* __restrict__ b,
+                                                            const float* __restrict__ s, float* __restrict__ bc,
+                                                            Lay l, Lay cl, const SolverScalars* sc) {
   if (sc && sc->done) return;
-  const size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (o >= l.count()) return;
-  int i, j, k;
-  l.cell(o, i, j, k);
+  __shared__ float part[FX * FY][64];
+  const int nz = l.nz, nkb = (nz + 63) / 64;
+  const int col = blockIdx.x / nkb, k = 64 * (blockIdx.x % nkb) + threadIdx.x;
+  const int I = col % cl.nx, J = col / cl.nx, n = threadIdx.y;
+  const int i = FX * I + n % FX, j = FY * J + n / FX;
   constexpr int oi[T_COUNT] = {0, -1, 1, 0, 0, 0, 0, -1, -1, 1, 1, 0, 0, 0, 0, 0, 0, -1, -1, 1, 1, 0, 0, 0, 0};
   constexpr int oj[T_COUNT] = {0, 0, 0, -1, 1, 0, 0, 0, 0, 0, 0, -1, -1, 1, 1, 0, 0, 0, 0, 0, 0, -1, -1, 1, 1};
   constexpr int ok[T_COUNT] = {0, 0, 0, 0, 0, -1, 1, -1, 1, -1, 1, -1, 1, -1, 1, -2, 2, -2, 2, -2, 2, -2, 2, -2, 2};
-  float v = 0.0f;
+  const int kc = min(k, nz - 1);
+  const size_t o = l.at(i, j, kc);
+  float a[T_COUNT], x[T_COUNT];
 #pragma unroll
   for (int t = 0; t < T_COUNT; ++t) {
-    const int kk = k + ok[t];
-    if (kk < 0 || kk >= l.nz) continue;
     int ii = i + oi[t], jj = j + oj[t];
     ii = ii < 0 ? ii + l.nx : (ii >= l.nx ? ii - l.nx : ii);
     jj = jj < 0 ? jj + l.ny : (jj >= l.ny ? jj - l.ny : jj);
-    v += A.a[t][o] * s[l.at(ii, jj, kk)];
+    a[t] = A.a[t][o];
+    x[t] = s[l.at(ii, jj, min(max(kc + ok[t], 0), nz - 1))];
   }
-  r[o] = (float)b[o] - v;
-}
-
-// b_coarse = R r: one thread per coarse cell (coarse memory order) sums its
-// fx x fy fine cells.
-template <int FX, int FY>
-__global__ void k_mg_sum(const float* __restrict__ r, float* __restrict__ bc, Lay fl, Lay cl,
-                         const SolverScalars* sc) {
-  if (sc && sc->done) return;
-  const size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (t >= cl.count()) return;
-  int I, J, k;
-  cl.cell(t, I, J, k);
-  float sum = 0.0f;
+  float v = 0.0f;
 #pragma unroll
-  for (int bb = 0; bb < FY; ++bb)
+  for (int t = 0; t < T_COUNT; ++t) v += a[t] * ((unsigned)(kc + ok[t]) < (unsigned)nz ? x[t] : 0.0f);
+  part[n][threadIdx.x] = (float)b[o] - v;
+  __syncthreads();
+  if (n == 0 && k < nz) {
+    float sum = 0.0f;
 #pragma unroll
-    for (int a = 0; a < FX; ++a) sum += r[fl.at(FX * I + a, FY * J + bb, k)];
-  bc[t] = sum;
+    for (int q = 0; q < FX * FY; ++q) sum += part[q][threadIdx.x];
+    bc[cl.at(I, J, k)] = sum;
+  }
 }
 
 // b_coarse = R (b - A s) for 2 x 2 aggregation: a block per tile as in the
@@ -449,26 +446,16 @@ __device__ __forceinline__ void scan_line(const float (&fa)[NPL], const float (&
   }
 }
 
-// The forward map of level k of a column from its line-solve factors and
-// right-hand side r (k = 0: P holds the pivot itself); identity maps above nz.
-template <typename IdxT>
-__device__ __forceinline__ void line_maps(const float* P, const float* E, const float* Q, IdxT o, int k, int nz,
-                                          float r, float& fa, float& fb, float& q) {
-  if (k >= nz) {
-    fa = 0.0f;
-    fb = 1.0f;
-    q = 1.0f;
-    return;
-  }
-  const float p = P[o];
-  if (k == 0) {
-    fa = r / p;
-    fb = 0.0f;
-  } else {
-    fa = r * p;
-    fb = E[o] * p;
-  }
-  q = k == nz - 1 ? 0.0f : Q[o];
+// The forward map of level k of a column from its line-solve factors p, e, q
+// (those of a level inside the column) and right-hand side r (k = 0: p holds
+// the pivot itself); identity maps above nz.
+__device__ __forceinline__ void line_maps(float p, float e, float qv, int k, int nz, float r, float& fa, float& fb,
+                                          float& q) {
+  const bool in = k < nz;
+  const float a = k == 0 ? r / p : r * p, b = k == 0 ? 0.0f : e * p;
+  fa = in ? a : 0.0f;
+  fb = in ? b : 1.0f;
+  q = in ? (k == nz - 1 ? 0.0f : qv) : 1.0f;
 }
 
 // One pseudo-time step of column (i, j): the right-hand side
@@ -484,28 +471,46 @@ __device__ __forceinline__ void column_step(const MgCoefs& A, const float* P, co
   const int im = i == 0 ? nx - 1 : i - 1, ip = i + 1 == nx ? 0 : i + 1;
   const int jm = j == 0 ? ny - 1 : j - 1, jp = j + 1 == ny ? 0 : j + 1;
   float fa[NPL], fb[NPL], q[NPL];
+  // every load is unconditional, at a level inside the column (zeroed beyond
+  // the walls where it is used): a branch per neighbour made each load wait
+  // for the one before (14 us against 7 for a first post-smoothing step at
+  // 32 x 32 x 128)
 #pragma unroll
   for (int u = 0; u < NPL; ++u) {
     const int k = NPL * lane + u;
-    const int o = l.at32(i, j, k < nz ? k : nz - 1);
-    float r = 0.0f;
-    if (k < nz) {
-      if (FIRST) {
-        r = deta * (0.0f - (float)b[o]);
-      } else {
-        auto S = [&](int ii, int jj, int kk) -> float { return kk < 0 || kk >= nz ? 0.0f : rd(ii, jj, kk); };
-        auto T = [&](int t) -> float { return A.a[t][o]; };
-        float v = T(T_AL) * S(im, j, k) + T(T_AR) * S(ip, j, k) + T(T_AF) * S(i, jp, k) + T(T_AB) * S(i, jm, k);
-        v += T(T_ARU) * S(ip, j, k + 1) + T(T_ARD) * S(ip, j, k - 1) + T(T_ALU) * S(im, j, k + 1) +
-             T(T_ALD) * S(im, j, k - 1) + T(T_AFU) * S(i, jp, k + 1) + T(T_AFD) * S(i, jp, k - 1) +
-             T(T_ABU) * S(i, jm, k + 1) + T(T_ABD) * S(i, jm, k - 1) + T(T_AUU) * S(i, j, k + 2) +
-             T(T_ADD) * S(i, j, k - 2) + T(T_ARUU) * S(ip, j, k + 2) + T(T_ARDD) * S(ip, j, k - 2) +
-             T(T_ALUU) * S(im, j, k + 2) + T(T_ALDD) * S(im, j, k - 2) + T(T_AFUU) * S(i, jp, k + 2) +
-             T(T_AFDD) * S(i, jp, k - 2) + T(T_ABUU) * S(i, jm, k + 2) + T(T_ABDD) * S(i, jm, k - 2);
-        r = S(i, j, k) + deta * (v - (float)b[o]);
+    const int kc = k < nz ? k : nz - 1;
+    const int o = l.at32(i, j, kc);
+    const float p = P[o], e = E[o], qv = Q[o];
+    float r;
+    if constexpr (FIRST) {
+      r = deta * (0.0f - (float)b[o]);
+    } else {
+      float a[T_COUNT], s[5][5];  // s: the column and its x and y neighbours on levels k - 2 ... k + 2
+#pragma unroll
+      for (int t = 0; t < T_COUNT; ++t)
+        if (t != T_AC && t != T_AD && t != T_AU) a[t] = A.a[t][o];
+#pragma unroll
+      for (int w = 0; w < 5; ++w) {
+        const int kk = min(max(kc - 2 + w, 0), nz - 1);
+        s[0][w] = rd(i, j, kk);
+        s[1][w] = rd(im, j, kk);
+        s[2][w] = rd(ip, j, kk);
+        s[3][w] = rd(i, jm, kk);
+        s[4][w] = rd(i, jp, kk);
       }
+      const float bv = (float)b[o];
+#pragma unroll
+      for (int w = 0; w < 5; ++w)
+#pragma unroll
+        for (int n = 0; n < 5; ++n) s[n][w] = (unsigned)(kc - 2 + w) < (unsigned)nz ? s[n][w] : 0.0f;
+      float v = a[T_AL] * s[1][2] + a[T_AR] * s[2][2] + a[T_AF] * s[4][2] + a[T_AB] * s[3][2];
+      v += a[T_ARU] * s[2][3] + a[T_ARD] * s[2][1] + a[T_ALU] * s[1][3] + a[T_ALD] * s[1][1] + a[T_AFU] * s[4][3] +
+           a[T_AFD] * s[4][1] + a[T_ABU] * s[3][3] + a[T_ABD] * s[3][1] + a[T_AUU] * s[0][4] + a[T_ADD] * s[0][0] +
+           a[T_ARUU] * s[2][4] + a[T_ARDD] * s[2][0] + a[T_ALUU] * s[1][4] + a[T_ALDD] * s[1][0] +
+           a[T_AFUU] * s[4][4] + a[T_AFDD] * s[4][0] + a[T_ABUU] * s[3][4] + a[T_ABDD] * s[3][0];
+      r = s[0][2] + deta * (v - bv);
     }
-    line_maps(P, E, Q, o, k, nz, r, fa[u], fb[u], q[u]);
+    line_maps(p, e, qv, k, nz, r, fa[u], fb[u], q[u]);
   }
   scan_line<NPL>(fa, fb, q, nz, y);
 }
@@ -688,6 +693,34 @@ void line_pack(pcf_state* st, const MgLevel& L, const LineCoefs<SrcT>& A) {
   else launch_line_pack(st->stream, A, (float*)L.coefs, L.factors, L.nx, L.ny, L.nz);
 }
 
+// Level paths.  Coarse levels of at most kCoarseColumnCols columns are stored
+// z fastest and smoothed one wavefront per column, larger ones x fastest by
+// line steps (48 x 40 x 64: 5 us per step against 11, where a tile per
+// workgroup leaves the chip empty; 64 x 64 x 128 keeps line steps).  A finest
+// level, always x fastest, is smoothed column by column up to kColumnCols.
+// The coarsest level runs all its steps in one workgroup when it has at most
+// 16 columns.
+constexpr size_t kColumnCols = 1024, kCoarseColumnCols = 2048;
+constexpr int kScanMaxNz = 512;
+constexpr size_t kCoarseLdsFloats = 16384;
+
+size_t columns(const MgLevel& L) { return (size_t)L.nx * L.ny; }
+bool column_path(const MgLevel& L) { return (L.zf || columns(L) <= kColumnCols) && L.nz <= kScanMaxNz; }
+
+MgCoefs coefs_of(const MgLevel& L) {
+  MgCoefs A;
+  for (int t = 0; t < T_COUNT; ++t) A.a[t] = L.a[t];
+  return A;
+}
+
+__global__ void k_round_bf16(MgCoefs A, size_t n) {
+  float* a = A.a[blockIdx.y];
+  for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x) {
+    const unsigned u = __float_as_uint(a[q]);
+    a[q] = __uint_as_float((u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u);  // round to nearest even
+  }
+}
+
 // The preconditioner's copies of the current operator: the packed
 // coefficients and line-solve factors of the levels smoothed by line steps,
 // and FP32 arrays of the multigrid's levels.
@@ -740,21 +773,19 @@ int prepare_mixed(pcf_state* st) {
       line_pack(st, C, A);
     }
   }
+  // bf16 storage covers the levels of more than kColumnCols columns; those
+  // smoothed column by column keep the rounded values in FP32 arrays (after
+  // the coarser levels have been formed from the unrounded ones)
+  if (bf16_storage(st))
+    for (size_t l = 1; l < st->mg.size(); ++l) {
+      const MgLevel& C = st->mg[l];
+      if (C.zf && columns(C) > kColumnCols)
+        hipLaunchKernelGGL(k_round_bf16, dim3(64, T_COUNT), dim3(256), 0, st->stream, coefs_of(C), lay_of(C).count());
+    }
   PCF_HIP(hipGetLastError());
   st->t32_valid = true;
   return PCF_OK;
 }
-
-// Level paths.  Levels with at most kColumnCols columns are stored z fastest
-// and smoothed one wavefront per column, larger ones x fastest by line steps.
-// The coarsest level runs all its steps in one workgroup when it has at most
-// 16 columns.
-constexpr size_t kColumnCols = 1024;
-constexpr int kScanMaxNz = 512;
-constexpr size_t kCoarseLdsFloats = 16384;
-
-size_t columns(const MgLevel& L) { return (size_t)L.nx * L.ny; }
-bool column_path(const MgLevel& L) { return columns(L) <= kColumnCols && L.nz <= kScanMaxNz; }
 
 template <class F>
 void with_npl(int nz, F&& f) {
@@ -766,12 +797,6 @@ void with_npl(int nz, F&& f) {
     f(std::integral_constant<int, 4>{});
   else
     f(std::integral_constant<int, 8>{});
-}
-
-MgCoefs coefs_of(const MgLevel& L) {
-  MgCoefs A;
-  for (int t = 0; t < T_COUNT; ++t) A.a[t] = L.a[t];
-  return A;
 }
 
 // steps smoothing steps on level L.  s: the buffer holding the current
@@ -877,17 +902,14 @@ void mg_restrict(pcf_state* st, const MgLevel& L, const MgLevel& C, const BT* b,
     return;
   }
   const MgCoefs A = coefs_of(L);
-  float* r = L.col;  // the line-solve scratch is free here
   const Lay fl = lay_of(L), cl = lay_of(C);
-  hipLaunchKernelGGL((k_mg_resid<BT>), dim3(blocks_for(fl.count(), 256)), dim3(256), 0, st->stream, A, b, s, r, fl,
-                     sc);
-  const dim3 cgrd(blocks_for(cl.count(), 256)), blk(256);
+  const dim3 grd((unsigned)columns(C) * blocks_for(L.nz, 64)), blk(64, L.fx * L.fy);
   if (L.fx == 2 && L.fy == 2)
-    hipLaunchKernelGGL((k_mg_sum<2, 2>), cgrd, blk, 0, st->stream, r, C.b, fl, cl, sc);
+    hipLaunchKernelGGL((k_resid_restrict_any<2, 2, BT>), grd, blk, 0, st->stream, A, b, s, C.b, fl, cl, sc);
   else if (L.fx == 2)
-    hipLaunchKernelGGL((k_mg_sum<2, 1>), cgrd, blk, 0, st->stream, r, C.b, fl, cl, sc);
+    hipLaunchKernelGGL((k_resid_restrict_any<2, 1, BT>), grd, blk, 0, st->stream, A, b, s, C.b, fl, cl, sc);
   else
-    hipLaunchKernelGGL((k_mg_sum<1, 2>), cgrd, blk, 0, st->stream, r, C.b, fl, cl, sc);
+    hipLaunchKernelGGL((k_resid_restrict_any<1, 2, BT>), grd, blk, 0, st->stream, A, b, s, C.b, fl, cl, sc);
 }
 
 // The coarsest level: mg_coarse_steps smoothing steps from zero.
@@ -1176,7 +1198,7 @@ int alloc_mixed(pcf_state* st) {
     float** v[] = {&C.P, &C.E, &C.Q, &C.b, &C.s, &C.rhs, &C.col};
     for (float** p : v)
       if ((rc = ac(p))) return rc;
-    C.zf = column_path(C);  // coarse levels smoothed column by column: z fastest
+    C.zf = columns(C) <= kCoarseColumnCols && C.nz <= kScanMaxNz;  // smoothed column by column
     if (!C.zf && (rc = packed(C))) return rc;
     st->mg.push_back(C);
   }
