@@ -263,8 +263,11 @@ struct MgCoefs {
 };
 
 // R A P: one thread per coarse cell, in the coarse level's memory order.
-template <int FX, int FY>
-__global__ void k_mg_coarsen(MgCoefs fine, MgCoefs coarse, Lay fl, Lay cl) {
+// FT: the fine coefficients, FP32, or the finest level's in FP64, each rounded
+// to FP32 where it is added: the same sums as from FP32 copies, without the 28
+// conversions a solve (23 us each at 256 x 256 x 128) and the arrays' memory.
+template <int FX, int FY, typename FT>
+__global__ void k_mg_coarsen(LineCoefs<FT> fine, MgCoefs coarse, Lay fl, Lay cl) {
   const size_t t0 = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   if (t0 >= cl.count()) return;
   int I, J, k;
@@ -283,7 +286,7 @@ __global__ void k_mg_coarsen(MgCoefs fine, MgCoefs coarse, Lay fl, Lay cl) {
 #pragma unroll
       for (int t = 0; t < T_COUNT; ++t) {
         const int target = coef_of(floor_div(a + oi[t], FX), floor_div(b + oj[t], FY), ok[t]);
-        acc[target] += fine.a[t][o];
+        acc[target] += (float)fine.a[t][o];
       }
     }
 #pragma unroll
@@ -749,19 +752,22 @@ int prepare_mixed(pcf_state* st) {
   for (size_t l = 1; l < st->mg.size(); ++l) {
     const MgLevel& F = st->mg[l - 1];
     const MgLevel& C = st->mg[l];
-    MgCoefs fa, ca;
-    for (int t = 0; t < T_COUNT; ++t) {
-      fa.a[t] = F.a[t];
-      ca.a[t] = C.a[t];
-    }
+    const MgCoefs ca = coefs_of(C);
     const Lay fl = lay_of(F), cl = lay_of(C);
     const dim3 grd(blocks_for(cl.count(), 256)), blk(256);
-    if (F.fx == 2 && F.fy == 2)
-      hipLaunchKernelGGL((k_mg_coarsen<2, 2>), grd, blk, 0, st->stream, fa, ca, fl, cl);
-    else if (F.fx == 2)
-      hipLaunchKernelGGL((k_mg_coarsen<2, 1>), grd, blk, 0, st->stream, fa, ca, fl, cl);
-    else
-      hipLaunchKernelGGL((k_mg_coarsen<1, 2>), grd, blk, 0, st->stream, fa, ca, fl, cl);
+    auto coarsen = [&](auto ft, auto* const* src) {
+      using FT = decltype(ft);
+      LineCoefs<FT> fa{};
+      for (int t = 0; t < T_COUNT; ++t) fa.a[t] = src[t];
+      if (F.fx == 2 && F.fy == 2)
+        hipLaunchKernelGGL((k_mg_coarsen<2, 2, FT>), grd, blk, 0, st->stream, fa, ca, fl, cl);
+      else if (F.fx == 2)
+        hipLaunchKernelGGL((k_mg_coarsen<2, 1, FT>), grd, blk, 0, st->stream, fa, ca, fl, cl);
+      else
+        hipLaunchKernelGGL((k_mg_coarsen<1, 2, FT>), grd, blk, 0, st->stream, fa, ca, fl, cl);
+    };
+    if (l == 1) coarsen(double{}, st->T.a);
+    else coarsen(float{}, F.a);
     hipLaunchKernelGGL(k_mg_factors, dim3(blocks_for((long long)C.nx * C.ny, 64)), dim3(64), 0, st->stream,
                        C.a[T_AC], C.a[T_AD], C.a[T_AU], C.P, C.E, C.Q, cl, C.deta);
     if (C.coefs) {
@@ -1163,7 +1169,10 @@ int alloc_mixed(pcf_state* st) {
     if ((rc = af(p))) return rc;
   if (!multigrid || !column_path(L0))
     if ((rc = packed(L0))) return rc;
-  if (multigrid) {
+  // FP32 arrays of the finest level where the column kernels or the general
+  // residual read them; the line steps read the packed ones
+  const bool pair = g.nx % 2 == 0 && g.nx >= kMgMinSize && g.ny % 2 == 0 && g.ny >= kMgMinSize;
+  if (multigrid && (!L0.coefs || !pair || g.nz > kLineMaxNz)) {
     for (int t = 0; t < T_COUNT; ++t)
       if ((rc = af(&L0.a[t]))) return rc;
     for (float** p : {&L0.P, &L0.E, &L0.Q})
