@@ -164,7 +164,8 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)
   FuseOperands<FUSE, NPL> X;
   if (t.act) {
 #pragma unroll
-    for (int u = 0; u < NPL; ++u) X.load(F, u, t.o + sxy * (ptrdiff_t)(min(t.k0 + u, A.nz - 1) - t.k0));
+    for (int u = 0; u < NPL; ++u)
+      X.load(F, u, t.o + sxy * (ptrdiff_t)(min(t.k0 + u, A.nz - 1) - t.k0), t.k0 + u < A.nz);
   }
   FuseScalars S;
   if (!fuse_scalars<FUSE>(F, S)) return;

@@ -694,13 +694,12 @@ __device__ __forceinline__ bool line_step64(const LineArgs64& A, const double* _
   }
   if constexpr (FIRST) {
     FuseOperands<FUSE, NPL> X;
-    // (idle threads of a partial tile read no vector that others write)
     if (t.act) {
 #pragma unroll
       for (int u = 0; u < NPL; ++u) {
         const size_t o = t.o + sxy * (ptrdiff_t)(min(t.k0 + u, nz - 1) - t.k0);
         if constexpr (FUSE == FUSE_NONE) X.p[u] = b[o];
-        else X.load(F, u, o);
+        else X.load(F, u, o, t.k0 + u < nz);
       }
     }
     FuseScalars S;

@@ -201,14 +201,18 @@ __device__ __forceinline__ void block_sums(const double* partials, int nparts, d
 enum { FUSE_NONE = 0, FUSE_P = 1, FUSE_S = 2 };
 // The operands of a fused step at a thread's N cells.  They, the partials and
 // the scalars are loaded together, before anything waits for one of them: a
-// load that follows another costs a round trip of 1 us here.
+// load that follows another costs a round trip of 1 us here.  own: cell o is
+// the thread's own; threads beyond a column's top load another's, of vectors
+// that the kernel does not write (dst is stored by the cell's own thread
+// while others still load).
 template <int FUSE, int N>
 struct FuseOperands {
   double r[N], v[N], p[N];
-  __device__ __forceinline__ void load(const BicgFuse& F, int u, size_t o) {
+  __device__ __forceinline__ void load(const BicgFuse& F, int u, size_t o, bool own) {
+    const double* p_or_r = own ? F.dst : F.r;
     r[u] = F.r[o];
     v[u] = F.v[o];
-    p[u] = FUSE == FUSE_P ? F.dst[o] : 0.0;
+    p[u] = FUSE == FUSE_P ? p_or_r[o] : 0.0;
   }
 };
 struct FuseScalars {

@@ -116,6 +116,29 @@ def test_batched_solves_give_each_member_its_standalone_bits(pcf, tmp_path, prec
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("x_size,z_size", [(16, 9), (18, 41), (34, 131)])
+def test_fused_iterations_give_the_batched_bits_at_ragged_heights(pcf, precision, x_size, z_size):
+    """A standalone solve on a small grid updates p and s inside the
+    preconditioner's first kernel; the batch updates them in kernels of their
+    own.  Heights that are no multiple of the levels per thread (2, 4, 8 or
+    16) leave threads beyond the top of a column, which must read no vector
+    that the others write: the bits are the batch's."""
+    sim = lambda: pcf.examples.bubble_member(seed=1, x_size=x_size, z_size=z_size, iterations=2, precision=precision)
+    alone, batched, batch = pcf.State(sim()), pcf.State(sim()), pcf.SolveBatch()
+    batch.attach(batched)
+    for a, b in ((alone.initial_cleaning(), batched.initial_cleaning()), (alone.step().niter, batched.step().niter)):
+        assert np.array_equal(a, b), (a, b)
+    assert batch.stats()["member_solves"] > 0
+    for f in ("RHOP", "U", "V", "W", "PIP", "RHO"):
+        assert np.array_equal(alone.get(f), batched.get(f)), f
+    batch.detach(batched)
+    alone.close()
+    batched.close()
+    batch.close()
+
+
+@pytest.mark.gpu
 def test_batched_solve_that_fails_stops_at_its_own_limit(pcf, abi, tmp_path):
     """A member whose poisson_iterations no solve can meet fails with the
     reference's non-convergence error after exactly that many iterations,
