@@ -408,8 +408,9 @@ int pcf_destroy(pcf_state* st) {
   if (st->stream) (void)hipStreamSynchronize(st->stream);
   if (st->ens_ready) (void)hipEventDestroy(st->ens_ready);
   prof_release(st);
-  for (hipGraphExec_t& e : st->iter_graph)
-    if (e) (void)hipGraphExecDestroy(e);
+  for (auto& by_form : st->iter_graph)
+    for (hipGraphExec_t& e : by_form)
+      if (e) (void)hipGraphExecDestroy(e);
   for (void* p : st->allocations) (void)hipFree(p);
   if (st->sc_host) (void)hipHostFree(st->sc_host);
   if (st->cfl_host) (void)hipHostFree(st->cfl_host);

@@ -328,10 +328,11 @@ struct pcf_state {
   double* stage_norm = nullptr;
   int stage_fallbacks = 0;            // solves rerun without the stage after it failed to converge
   double* train_buf[3] = {};          // network training work: x, A x - v, A^T (A x - v)
-  // the BiCGSTAB iteration captured as a hipGraph (FP64 / mixed solve),
-  // instantiated on first use and replayed once per iteration (when
-  // solver_graphs is set: pcf_set_solver_graphs)
-  hipGraphExec_t iter_graph[2] = {nullptr, nullptr};
+  // the BiCGSTAB iteration captured as a hipGraph ([mixed solve][fused
+  // iteration]: whether a solve's iterations are fused depends on the learned
+  // stage, which comes and goes), instantiated on first use and replayed once
+  // per iteration (when solver_graphs is set: pcf_set_solver_graphs)
+  hipGraphExec_t iter_graph[2][2] = {};
   bool solver_graphs = false;
   // ensemble membership (pcf_ensemble_attach): the ensemble, the member's
   // group (-1: its solves run on their own) and slot in the group's table,

@@ -1739,9 +1739,10 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
   const BicgFuse fuse_p{st->br, st->bv, st->bp, st->partials, vgrid, nxyz, sc};
   const BicgFuse fuse_s{st->br, st->bv, st->bs, st->partials, aparts, nxyz, sc};
   // One BiCGSTAB iteration's launches.  Every argument is fixed for the
-  // state (the scalars live in device memory), so the sequence is captured
-  // once into a hipGraph and replayed as one launch per iteration; the
-  // learned stage's iterations and profiled runs launch it directly.
+  // state and the form of the iteration, fused or not (the scalars live in
+  // device memory), so each form's sequence is captured once into a hipGraph
+  // and replayed as one launch per iteration; the learned stage's iterations
+  // and profiled runs launch it directly.
   auto iteration = [&](int jb) -> int {
     int rc1 = PCF_OK;
     // v = A M^-1 p, <v, r0>
@@ -1786,7 +1787,7 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
     const bool graphed =
         st->solver_graphs && !st->ens && !st->prof_on && !(stage && jb <= st->stage_iterations);
     if (graphed) {
-      hipGraphExec_t& exec = st->iter_graph[mixed ? 1 : 0];
+      hipGraphExec_t& exec = st->iter_graph[mixed ? 1 : 0][fused ? 1 : 0];
       if (!exec) {
         hipGraph_t graph = nullptr;
         PCF_HIP(hipStreamBeginCapture(st->stream, hipStreamCaptureModeThreadLocal));

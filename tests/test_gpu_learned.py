@@ -6,6 +6,7 @@ stopping test is unchanged (|r| / |b| against the reference tolerance), so
 what the network does can change the iteration count, never the accuracy;
 a solve that fails with the stage is rerun without it."""
 import ctypes
+import zlib
 
 import hipmem
 import numpy as np
@@ -200,3 +201,43 @@ def test_stage_fallback_keeps_the_error_code(pcf, abi):
     fb = ctypes.c_int32(0)
     assert st.lib.pcf_stage_fallbacks(st.h, ctypes.byref(fb)) == 0
     assert fb.value == 1
+
+
+@pytest.mark.parametrize("short", [0, 1])
+@pytest.mark.parametrize("order", [(0, 1, 0), (1, 0, 1)])
+def test_solver_graphs_follow_the_stage(pcf, order, short):
+    """Solves without (0) and with (1) a stage network, one after the other
+    on one state: the stage changes the launches of an iteration (on a small
+    grid a plain solve's are fused), so each form replays its own captured
+    graph and every solve gives the eager launches' return code, iteration
+    count, residual and bits.  poisson_iterations is what the plain solve
+    needs, where the last permitted iteration converges, and one less, where
+    no solve does (the stage network's last layer is zero: it needs the same)."""
+    def solves(graphs, limit, order):
+        nl = namelists(pcf, 21, "zero", 2)
+        nl.poisson.preconditioner_type = "line_relaxation"
+        nl.poisson.poisson_iterations = limit
+        st = pcf.State(nl)
+        assert st.lib.pcf_set_solver_graphs(st.h, int(graphs)) == 0
+        net = pcf.learned.GuessNetwork(32, 32, 16, training=False, params=pcf.learned.init_params(2))
+        st.compute_sponges(0.8, 3.0)
+        tolref = st.compute_lhs()
+        st.compute_operator(0.8, 1.0)
+        out = []
+        for stage in order:
+            if stage:
+                pcf.learned.attach_stage(st, net, 1)
+            else:
+                assert st.lib.pcf_set_stage_network(st.h, None, 0) == 0
+            n = ctypes.c_int32(0)
+            rc = st.lib.pcf_apply_bicgstab(st.h, tolref, ctypes.byref(n))
+            out.append((rc, n.value, st.last_residual(), zlib.crc32(st.get_vector("SOLUTION").tobytes())))
+        st.close()
+        return out
+
+    rc, needed, _, _ = solves(False, 1000, (0,))[0]
+    assert rc == 0 and needed > 2
+    eager, graphed = solves(False, needed - short, order), solves(True, needed - short, order)
+    print(needed, eager, graphed)
+    assert all((s[0] == 0) == (short == 0) for s in eager)
+    assert graphed == eager
