@@ -1818,7 +1818,7 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
     }
   }
   if (rc == PCF_OK && converged_at < 0) {
-    if (fused) {  // the last iteration's check
+    if (fused && maxit > 0) {  // the last iteration's check
       hipLaunchKernelGGL(k_bicg_check, dim3(1), dim3(1024), 0, st->stream, st->partials, vgrid, sc, nxyz);
       PCF_HIP(hipMemcpyAsync(hs + (last_seen & 1), sc, sizeof(SolverScalars), hipMemcpyDeviceToHost, st->stream));
     }

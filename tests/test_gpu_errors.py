@@ -61,6 +61,23 @@ def test_iteration_limit_is_noconv(pcf, abi, oracle_mod, precision):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_no_permitted_iteration_is_noconv_after_none(pcf, abi, oracle_mod, precision):
+    """poisson_iterations = 0 on a grid whose iterations are fused (each
+    makes the check of the one before)."""
+    nls = [pcf.examples.mountain_wave(x_size=12, y_size=10, z_size=9) for _ in range(2)]
+    for nl in nls:
+        nl.poisson.poisson_iterations = 0
+    nls[0].poisson.precision = precision
+    gpu = pcf.State(nls[0])
+    orc = oracle_mod.Oracle(pcf.to_config(nls[1]), abi)
+    divergent_winds(gpu, orc)
+    for s in (gpu, orc):
+        s.set_boundaries(abi.BOUNDARY_PREDICTANDS)
+    assert orc.apply_corrector(1.0, 1.0) == (abi.E_NOCONV, 0)
+    assert corrector(gpu) == (abi.E_NOCONV, 0)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_nan_right_hand_side_stops_at_the_limit(pcf, abi, oracle_mod, precision):
     limit = 12
     nls = []
