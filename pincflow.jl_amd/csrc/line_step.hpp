@@ -336,6 +336,10 @@ __device__ __forceinline__ void line_rhs(const CT* __restrict__ a, Rd rd, const 
     const int m = u + 2, d = u % (LAG + 1);
     if (AHEAD + u < NPL + 4) level(AHEAD + u);
     if (u + LAG < NPL) coefs(u + LAG);
+    // (without it the 16-level kernel's bf16 loads sink to their uses, one
+    // round trip each: 152 us against 42 at 64 x 64 x 160, 650 against 204 at
+    // 256 x 256 x 160)
+    if constexpr (DEPTH == 0 && sizeof(CT) == 2) asm volatile("" ::: "memory");
     const int k = k0 + u;
 #pragma unroll
     for (int c = 0; c < W; ++c) {
