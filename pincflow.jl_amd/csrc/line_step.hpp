@@ -220,24 +220,91 @@ __device__ __forceinline__ void line_solve_segments(const R* __restrict__ f, int
     }
 }
 
-// The same line solve for a column of any height in one thread: rhs(k) gives
-// the right-hand sides in ascending order, f points to the packed factors,
-// col[c + stride k] keeps the upward sweep, put(k, y) takes the solution from
-// the top down.
-template <typename R, class Rhs, class Put>
-__device__ __forceinline__ void line_solve_column(const R* f, R* col, size_t c, size_t stride, int nz, Rhs rhs,
-                                                  Put put) {
+// The same line solve for columns of any height, one column wide (W = 1): the
+// block's first `own` segments take the levels in chunks of own NPL, upwards
+// and then downwards, the value at a chunk's edge going on to the next one in
+// LDS; idle threads of a wider block run identity maps.  rhs(k0, r): the
+// right-hand sides of the NPL levels from k0; f: the tile's packed factors at
+// the thread's column; keep(k, s) and kept(k): a thread's own scratch for the
+// upward sweep of all chunks but the last, inside the column; put(k, y): the
+// solution at a level inside it.  lds: 2 blockDim.x + cols values.
+template <typename R, int NPL, class Rhs, class Keep, class Kept, class Put>
+__device__ __forceinline__ void line_solve_chunks(const R* __restrict__ f, int nz, int own, int tx, int seg, Rhs rhs,
+                                                  Keep keep, Kept kept, Put put, R* lds) {
   constexpr int cols = LineTile<R>::cols;
-  R s = 0;
-  for (int k = 0; k < nz; ++k) {
-    const R* fk = f + (size_t)3 * cols * k;
-    s = k == 0 ? rhs(k) / fk[0] : (rhs(k) + fk[cols] * s) * fk[0];
-    col[c + stride * k] = s;
+  R *la = lds, *lb = la + blockDim.x, *edge = lb + blockDim.x;
+  const int chunk = own * NPL, chunks = (nz + chunk - 1) / chunk;
+  R r[NPL][1], in = 0;
+  for (int ch = 0; ch < chunks; ++ch) {
+    const int k0 = seg < own ? ch * chunk + seg * NPL : nz;
+    rhs(k0, r);
+    R p[NPL], e[NPL], A = 0, B = 1;
+#pragma unroll
+    for (int u = 0; u < NPL; ++u) {
+      const R* fu = f + (size_t)3 * cols * min(k0 + u, nz - 1);
+      p[u] = __builtin_nontemporal_load(fu);
+      e[u] = __builtin_nontemporal_load(fu + cols);
+    }
+#pragma unroll
+    for (int u = 0; u < NPL; ++u) {
+      const bool lev = k0 + u < nz, bottom = u == 0 && k0 == 0;  // the lowest level's P is the pivot itself
+      const R rr = bottom ? r[u][0] / p[u] : r[u][0];
+      r[u][0] = lev ? rr : (R)0;
+      p[u] = lev && !bottom ? p[u] : (R)1;
+      e[u] = bottom ? (R)0 : (lev ? e[u] : (R)1);
+      A = (r[u][0] + e[u] * A) * p[u];
+      B = e[u] * B * p[u];
+    }
+    la[threadIdx.x] = A;
+    lb[threadIdx.x] = B;
+    __syncthreads();
+    R s = in;
+#pragma unroll 4
+    for (int t = 0; t < seg; ++t) s = la[t * cols + tx] + lb[t * cols + tx] * s;
+#pragma unroll
+    for (int u = 0; u < NPL; ++u) {
+      s = (r[u][0] + e[u] * s) * p[u];
+      r[u][0] = k0 + u < nz ? s : (R)0;
+    }
+    if (seg == own - 1) edge[tx] = s;
+    if (ch + 1 < chunks)
+#pragma unroll
+      for (int u = 0; u < NPL; ++u)
+        if (k0 + u < nz) keep(k0 + u, r[u][0]);
+    __syncthreads();  // the readers of la, lb; edge
+    in = edge[tx];
   }
-  put(nz - 1, s);
-  for (int k = nz - 2; k >= 0; --k) {
-    s = col[c + stride * k] + f[(size_t)3 * cols * k + 2 * cols] * s;
-    put(k, s);
+  in = 0;
+  for (int ch = chunks - 1; ch >= 0; --ch) {
+    const int k0 = seg < own ? ch * chunk + seg * NPL : nz;
+    R q[NPL], A = 0, B = 1;
+    if (ch + 1 < chunks)
+#pragma unroll
+      for (int u = 0; u < NPL; ++u) r[u][0] = k0 + u < nz ? kept(k0 + u) : (R)0;
+#pragma unroll
+    for (int u = 0; u < NPL; ++u)
+      q[u] = __builtin_nontemporal_load(f + (size_t)3 * cols * min(k0 + u, nz - 1) + 2 * cols);
+#pragma unroll
+    for (int u = NPL - 1; u >= 0; --u) {
+      const int k = k0 + u;
+      q[u] = k == nz - 1 ? (R)0 : (k < nz ? q[u] : (R)1);
+      A = r[u][0] + q[u] * A;
+      B = q[u] * B;
+    }
+    la[threadIdx.x] = A;
+    lb[threadIdx.x] = B;
+    __syncthreads();
+    R y = in;
+#pragma unroll 4
+    for (int t = own - 1; t > seg; --t) y = la[t * cols + tx] + lb[t * cols + tx] * y;
+#pragma unroll
+    for (int u = NPL - 1; u >= 0; --u) {
+      y = r[u][0] + q[u] * y;
+      if (k0 + u < nz) put(k0 + u, y);
+    }
+    if (seg == 0) edge[tx] = y;
+    __syncthreads();
+    in = edge[tx];
   }
 }
 

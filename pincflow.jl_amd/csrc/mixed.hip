@@ -188,28 +188,54 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)
   }
 }
 
-// The same step for columns of more than kLineMaxNz levels, one thread per
-// column; col: FP32 scratch of the grid's size.
+constexpr int kLineMaxNz = 256;  // levels of k_line_step32's columns (taller ones: k_line_tall32)
+constexpr int kTallNpl = 16;     // levels per thread of a chunk of a taller column
+
+// segments of a tall column's chunks: the fewest chunks of at most kLineMaxNz
+// levels, and the levels spread over them
+inline __host__ __device__ int tall_segments(int nz) {
+  const int chunks = (nz + kLineMaxNz - 1) / kLineMaxNz, levels = (nz + chunks - 1) / chunks;
+  return (levels + kTallNpl - 1) / kTallNpl;
+}
+
+// The same step for columns of more than kLineMaxNz levels, chunk by chunk;
+// col: FP32 scratch of the grid's size, which keeps the upward sweep.  Like
+// the shorter columns it is bound by memory on a large grid and by the round
+// trips of a chunk on a small one.  One application of two steps, FP32 / bf16
+// storage, with a horizontal kernel and a line solve apart, with a thread per
+// column for both, and chunk by chunk:
+//   64 x 64 x 300    145 / 138   632 / 614    92 /  77 us
+//   256 x 128 x 320  382 / 307   836 / 802   307 / 231 us
 template <bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
-__global__ void __launch_bounds__(kTileCols) k_line_tall32(LineArgs<CT> A, const BT* __restrict__ b,
-                                                           OutT* __restrict__ out, float* col,
-                                                           const SolverScalars* sc) {
-  if (sc && sc->done) return;
-  const LineThread<float, 1, 1> t(blockIdx.x, A.nx, A.ny, A.nz);
-  if (!t.act) return;
-  const size_t sxy = (size_t)A.nx * A.ny;
-  auto rhs = [&](int k) -> float {
+__device__ __forceinline__ void line_tall32(const LineArgs<CT>& A, const BT* __restrict__ b, OutT* __restrict__ out,
+                                            float* col, int tile) {
+  extern __shared__ float line_shared[];
+  const LineThread<float, 1, kTallNpl> t(tile, A.nx, A.ny, A.nz);
+  const size_t sxy = (size_t)A.nx * A.ny, c = (size_t)t.i + (size_t)A.nx * t.j, tc = (size_t)tile * A.nz;
+  auto rhs = [&](int k0, float (&r)[kTallNpl][1]) {
     if constexpr (FIRST) {
-      return A.deta * (0.0f - (float)b[t.o + sxy * k]);
+#pragma unroll
+      for (int u = 0; u < kTallNpl; ++u)
+        r[u][0] = A.deta * (0.0f - (float)__builtin_nontemporal_load(b + c + sxy * min(k0 + u, A.nz - 1)));
     } else {
-      float r[1][1];
-      line_rhs<float, 1, 1, 0, false, CT, BT>(A.coefs + (t.c + k) * T_COUNT * kTileCols + t.tx, LineRead<1, PRO, CT>{A}, b,
-                                           A.nx, A.ny, A.nz, A.deta, t.i, t.j, k, r);
-      return r[0][0];
+      line_rhs<float, 1, kTallNpl, 0, false, CT, BT>(A.coefs + (tc + k0) * T_COUNT * kTileCols + t.tx,
+                                                     LineRead<1, PRO, CT>{A}, b, A.nx, A.ny, A.nz, A.deta, t.i, t.j,
+                                                     k0, r);
     }
   };
-  line_solve_column<float>(A.factors + t.c * 3 * kTileCols + t.tx, col, t.o, sxy, A.nz, rhs,
-                           [&](int k, float y) { out[t.o + sxy * k] = (OutT)y; });
+  // (idle columns of a partial tile keep nothing: their cells are another's)
+  line_solve_chunks<float, kTallNpl>(
+      A.factors + tc * 3 * kTileCols + t.tx, A.nz, tall_segments(A.nz), t.tx, t.seg, rhs,
+      [&](int k, float s) { if (t.act) col[c + sxy * k] = s; },
+      [&](int k) { return t.act ? col[c + sxy * k] : 0.0f; },
+      [&](int k, float y) { if (t.act) out[c + sxy * k] = (OutT)y; }, line_shared);
+}
+template <bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)))
+    k_line_tall32(LineArgs<CT> A, const BT* __restrict__ b, OutT* __restrict__ out, float* col,
+                  const SolverScalars* sc) {
+  if (sc && sc->done) return;
+  line_tall32<FIRST, PRO, CT, BT, OutT>(A, b, out, col, xcd_block(blockIdx.x, gridDim.x));
 }
 
 __global__ void k_to_f32(const double* a, float* b, size_t n) {
@@ -601,8 +627,6 @@ Lay correction_layout(const MgLevel& L, const MgLevel& C) { return Lay{C.nx, C.n
 
 bool bf16_storage(const pcf_state* st) { return st->cfg.preconditioner_storage == PCF_STORAGE_BF16; }
 
-constexpr int kLineMaxNz = 256;  // levels of k_line_step32's columns (taller ones: k_line_tall32)
-
 // f(W, NPL), the columns and levels per thread of a grid's line steps.  Eight
 // levels per thread up to 128 levels, 16 above (a block has at most 1024
 // threads).  Four columns per thread (16-byte loads, a quarter of the memory
@@ -652,16 +676,18 @@ void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, Out
     using CT = decltype(ct);
     const LineArgs<CT> A = line_args<CT>(L, s, e, C);
     const dim3 grd(LineTile<float>::count(L.nx, L.ny));
-    if (L.nz > kLineMaxNz)
-      hipLaunchKernelGGL((k_line_tall32<FIRST, PRO, CT, BT, OutT>), grd, dim3(kTileCols), 0, st->stream, A, b, out,
-                         L.col, sc);
-    else
+    if (L.nz > kLineMaxNz) {
+      const int threads = kTileCols * tall_segments(L.nz);
+      hipLaunchKernelGGL((k_line_tall32<FIRST, PRO, CT, BT, OutT>), grd, dim3(threads), (line_lds<float, 1>(threads)),
+                         st->stream, A, b, out, L.col, sc);
+    } else {
       with_line_shape(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
         constexpr int W = decltype(w)::value, NPL = decltype(npl)::value;
         const int threads = kTileCols / W * ((L.nz + NPL - 1) / NPL);
         hipLaunchKernelGGL((k_line_step32<W, NPL, FIRST, PRO, CT, BT, OutT>), grd, dim3(threads),
                            (line_lds<float, W>(threads)), st->stream, A, b, out, sc, commit);
       });
+    }
   };
   if constexpr (FIRST) {
     go(float{}, std::false_type{});

@@ -47,6 +47,17 @@ def test_fp32_line_step_matches_the_oracle(pcf, abi, oracle_mod, shape, storage,
     assert err <= 1e-4, err
 
 
+@pytest.mark.parametrize("shape,storage,iterations", [
+    ((33, 3, 257), "fp32", 3), ((8, 3, 272), "bf16", 2), ((31, 5, 512), "fp32", 2), ((66, 1, 513), "bf16", 3),
+    ((34, 3, 600), "fp32", 1), ((34, 3, 601), "fp32", 4)])
+def test_fp32_line_step_of_tall_columns_matches_the_oracle(pcf, abi, oracle_mod, shape, storage, iterations):
+    """Columns of two and three chunks, the last one shorter or full, with
+    partial tiles: the bound above."""
+    err = preconditioned(pcf, abi, oracle_mod, shape, "mixed", storage, iterations)
+    print(shape, storage, iterations, err)
+    assert err <= 1e-4, err
+
+
 @pytest.mark.parametrize("shape,iterations", [
     ((16, 4, 4), 2), ((17, 1, 5), 2), ((15, 3, 129), 2), ((33, 5, 128), 3), ((20, 3, 256), 2), ((20, 3, 257), 2),
     ((120, 50, 100), 2), ((120, 51, 100), 2), ((31, 7, 9), 1)])

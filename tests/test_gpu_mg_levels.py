@@ -1,0 +1,42 @@
+"""The multigrid V-cycle of the mixed solve on the grids whose levels take
+other kernels than the smaller ones of test_gpu_mixed.py, against the FP64
+restatement (mg_reference.py).  FP32 rounding through the levels stays below
+1e-3 of the result's max norm (see test_multigrid_vcycle_matches_fp64_restatement
+for its size); a wrong index, sign, level or coefficient gives errors of order
+one."""
+import numpy as np
+import pytest
+
+import hipmem
+import mg_reference as mg
+
+pytestmark = pytest.mark.gpu
+
+
+def vcycle_error(pcf, shape, storage, nu=2, coarse=4):
+    nx, ny, nz = shape
+    nl = pcf.examples.mountain_wave_3d(x_size=nx, y_size=ny, z_size=nz, iterations=3)
+    p = nl.poisson
+    p.precision, p.preconditioner_type, p.preconditioner_storage = "mixed", "multigrid", storage
+    p.mg_smoothing_steps, p.mg_coarse_steps = nu, coarse
+    gpu = pcf.State(nl)
+    gpu.compute_sponges(0.8, 3.0)
+    gpu.compute_operator(0.8, 1.0)
+    c = pcf.output.constants(nl)
+    lv = mg.levels({n: gpu.get_vector(n) for n in mg.NAMES}, nl.domain.lx / c["lref"] / nx,
+                   nl.domain.ly / c["lref"] / ny, p.dtau, round_apply=mg.bf16 if storage == "bf16" else None)
+    x = np.random.default_rng(5).standard_normal(shape)
+    want = mg.vcycle(lv, x, nu=nu, coarse_steps=coarse)
+    dx, dy = hipmem.DeviceArray(shape).upload(x), hipmem.DeviceArray(shape)
+    gpu.apply_preconditioner_device(dx.ptr, dy.ptr)
+    err = float(np.max(np.abs(dy.download() - want)) / np.max(np.abs(want)))
+    print(shape, storage, nu, coarse, "levels", len(lv), "rel err", err)
+    gpu.close()
+    return err
+
+
+@pytest.mark.parametrize("shape,storage", [((68, 40, 264), "fp32"), ((48, 64, 520), "fp32")])
+def test_tall_levels_match_the_restatement(pcf, shape, storage):
+    """More than 256 levels on the levels smoothed by line steps (2720
+    columns; beyond 512 levels all)."""
+    assert vcycle_error(pcf, shape, storage) <= 1e-3
