@@ -52,18 +52,19 @@ struct LineTile {
   static int count(int nx, int ny) { return ((nx + X - 1) / X) * ((ny + Y - 1) / Y); }
 };
 
-// The columns and levels of a thread of a tile.
+// The columns and levels of a thread of a tile; seg0: the block's first
+// segment.
 template <typename R, int W, int NPL>
 struct LineThread {
   int tx, seg, i, j, k0;
   bool act;
   size_t o, c;  // the first cell in the x-fastest arrays; its level in the tile's arrays
-  __device__ __forceinline__ LineThread(int tile, int nx, int ny, int nz) {
+  __device__ __forceinline__ LineThread(int tile, int nx, int ny, int nz, int seg0 = 0) {
     using T = LineTile<R>;
     constexpr int CX = T::cols / W;
     const int tiles_x = (nx + T::X - 1) / T::X;
     tx = threadIdx.x % CX;
-    seg = threadIdx.x / CX;
+    seg = seg0 + threadIdx.x / CX;
     i = (tile % tiles_x) * T::X + (tx * W) % T::X;
     j = (tile / tiles_x) * T::Y + (tx * W) / T::X;
     act = i < nx && j < ny;

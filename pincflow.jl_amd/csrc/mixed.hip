@@ -344,11 +344,30 @@ __global__ void __launch_bounds__(64) k_mg_factors(const float* ac, const float*
   }
 }
 
-// b_coarse = R (b - A s) on a level of any layout: block (64, FX FY) of 64
+// The operands of A s at cell (i, j, k) of a level: a and x, zero beyond the walls.
+__device__ __forceinline__ void resid_operands(const MgCoefs& A, const float* __restrict__ s, const Lay& l, int i, int j,
+                                               int k, float (&a)[T_COUNT], float (&x)[T_COUNT]) {
+  constexpr int oi[T_COUNT] = {0, -1, 1, 0, 0, 0, 0, -1, -1, 1, 1, 0, 0, 0, 0, 0, 0, -1, -1, 1, 1, 0, 0, 0, 0};
+  constexpr int oj[T_COUNT] = {0, 0, 0, -1, 1, 0, 0, 0, 0, 0, 0, -1, -1, 1, 1, 0, 0, 0, 0, 0, 0, -1, -1, 1, 1};
+  constexpr int ok[T_COUNT] = {0, 0, 0, 0, 0, -1, 1, -1, 1, -1, 1, -1, 1, -1, 1, -2, 2, -2, 2, -2, 2, -2, 2, -2, 2};
+  const size_t o = l.at(i, j, k);
+#pragma unroll
+  for (int t = 0; t < T_COUNT; ++t) {
+    int ii = i + oi[t], jj = j + oj[t];
+    ii = ii < 0 ? ii + l.nx : (ii >= l.nx ? ii - l.nx : ii);
+    jj = jj < 0 ? jj + l.ny : (jj >= l.ny ? jj - l.ny : jj);
+    a[t] = A.a[t][o];
+    x[t] = s[l.at(ii, jj, min(max(k + ok[t], 0), l.nz - 1))];
+  }
+#pragma unroll
+  for (int t = 0; t < T_COUNT; ++t) x[t] = (unsigned)(k + ok[t]) < (unsigned)l.nz ? x[t] : 0.0f;
+}
+
+// b_coarse = R (b - A s) on a z-fastest level: block (64, FX FY) of 64
 // levels of one coarse column, one thread per fine cell, whose residuals are
 // summed in LDS in the order of the fine columns.
 template <int FX, int FY, typename BT>
-__global__ void __launch_bounds__(256) k_resid_restrict_any(MgCoefs A, const BT* __restrict__ b,
+__global__ void __launch_bounds__(256) k_resid_restrict_columns(MgCoefs A, const BT* __restrict__ b,
                                                             const float* __restrict__ s, float* __restrict__ bc,
                                                             Lay l, Lay cl, const SolverScalars* sc) {
   if (sc && sc->done) return;
@@ -357,24 +376,12 @@ __global__ void __launch_bounds__(256) k_resid_restrict_any(MgCoefs A, const BT*
   const int col = blockIdx.x / nkb, k = 64 * (blockIdx.x % nkb) + threadIdx.x;
   const int I = col % cl.nx, J = col / cl.nx, n = threadIdx.y;
   const int i = FX * I + n % FX, j = FY * J + n / FX;
-  constexpr int oi[T_COUNT] = {0, -1, 1, 0, 0, 0, 0, -1, -1, 1, 1, 0, 0, 0, 0, 0, 0, -1, -1, 1, 1, 0, 0, 0, 0};
-  constexpr int oj[T_COUNT] = {0, 0, 0, -1, 1, 0, 0, 0, 0, 0, 0, -1, -1, 1, 1, 0, 0, 0, 0, 0, 0, -1, -1, 1, 1};
-  constexpr int ok[T_COUNT] = {0, 0, 0, 0, 0, -1, 1, -1, 1, -1, 1, -1, 1, -1, 1, -2, 2, -2, 2, -2, 2, -2, 2, -2, 2};
   const int kc = min(k, nz - 1);
-  const size_t o = l.at(i, j, kc);
-  float a[T_COUNT], x[T_COUNT];
+  float a[T_COUNT], x[T_COUNT], v = 0.0f;
+  resid_operands(A, s, l, i, j, kc, a, x);
 #pragma unroll
-  for (int t = 0; t < T_COUNT; ++t) {
-    int ii = i + oi[t], jj = j + oj[t];
-    ii = ii < 0 ? ii + l.nx : (ii >= l.nx ? ii - l.nx : ii);
-    jj = jj < 0 ? jj + l.ny : (jj >= l.ny ? jj - l.ny : jj);
-    a[t] = A.a[t][o];
-    x[t] = s[l.at(ii, jj, min(max(kc + ok[t], 0), nz - 1))];
-  }
-  float v = 0.0f;
-#pragma unroll
-  for (int t = 0; t < T_COUNT; ++t) v += a[t] * ((unsigned)(kc + ok[t]) < (unsigned)nz ? x[t] : 0.0f);
-  part[n][threadIdx.x] = (float)b[o] - v;
+  for (int t = 0; t < T_COUNT; ++t) v += a[t] * x[t];
+  part[n][threadIdx.x] = (float)b[l.at(i, j, kc)] - v;
   __syncthreads();
   if (n == 0 && k < nz) {
     float sum = 0.0f;
@@ -384,9 +391,39 @@ __global__ void __launch_bounds__(256) k_resid_restrict_any(MgCoefs A, const BT*
   }
 }
 
-// b_coarse = R (b - A s) for 2 x 2 aggregation: a block per tile as in the
-// line steps; the x pairs are summed in the thread (W = 4) or across lanes,
-// the rows j and j + 1 of a tile across lanes.
+// The same on an x-fastest level without packed 2 x 2 tiles: one thread per
+// fine x position, level and coarse row, in memory order, so that a
+// wavefront's accesses are contiguous (the kernel above, whose lanes run over
+// z, took 2941 us against 1308 for a V-cycle at 255 x 256 x 64).  The x pairs
+// are summed across lanes.
+template <int FX, int FY, typename BT>
+__global__ void __launch_bounds__(256) k_resid_restrict_rows(MgCoefs A, const BT* __restrict__ b,
+                                                             const float* __restrict__ s, float* __restrict__ bc,
+                                                             Lay l, Lay cl, const SolverScalars* sc) {
+  if (sc && sc->done) return;
+  const unsigned nx = l.nx, cy = cl.ny;
+  const unsigned q = xcd_block(blockIdx.x, gridDim.x) * 256u + threadIdx.x;
+  if (q >= nx * cy * l.nz) return;  // a pair's lanes stay or leave together
+  const int i = q % nx, J = q / nx % cy, k = q / nx / cy;
+  float sum = 0.0f;
+#pragma unroll
+  for (int n = 0; n < FY; ++n) {
+    const int j = FY * J + n;
+    float a[T_COUNT], x[T_COUNT], v = 0.0f;
+    resid_operands(A, s, l, i, j, k, a, x);
+#pragma unroll
+    for (int t = 0; t < T_COUNT; ++t) v += a[t] * x[t];
+    const float r = (float)b[l.at(i, j, k)] - v;
+    sum += r;
+    if constexpr (FX == 2) sum += __shfl_down(r, 1);
+  }
+  if (i % FX == 0) bc[cl.at(i / FX, J, k)] = sum;
+}
+
+// b_coarse = R (b - A s) for 2 x 2 aggregation of a level with packed tiles: a
+// block per tile (blockIdx.y: its part of a column of more levels than a block
+// has) as in the line steps; the x pairs are summed in the thread (W = 4) or
+// across lanes, the rows j and j + 1 of a tile across lanes.
 template <int W, int NPL, typename BT, typename CT>
 __global__ void __launch_bounds__(W == 4 ? 512 : 1024)
     __attribute__((amdgpu_waves_per_eu(W == 4 ? 2 : 4, W == 4 ? 2 : 4))) k_resid_restrict(LineArgs<CT> A, const BT* __restrict__ b,
@@ -394,7 +431,7 @@ __global__ void __launch_bounds__(W == 4 ? 512 : 1024)
   if (sc && sc->done) return;
   const int nx = A.nx, ny = A.ny, nz = A.nz;
   const int tile = xcd_block(blockIdx.x, gridDim.x);
-  const LineThread<float, W, NPL> t(tile, nx, ny, nz);
+  const LineThread<float, W, NPL> t(tile, nx, ny, nz, blockIdx.y * (blockDim.x / (kTileCols / W)));
   float r[NPL][W];
   line_rhs<float, W, NPL, W == 1 && NPL == 8 ? 1 : 0, true, CT, BT>(A.coefs + t.c * T_COUNT * kTileCols + t.tx * W, LineRead<W, false, CT>{A}, b,
                                         nx, ny, nz, A.deta, t.i, t.j, t.k0, r);
@@ -920,13 +957,14 @@ template <typename BT>
 void mg_restrict(pcf_state* st, const MgLevel& L, const MgLevel& C, const BT* b, const float* s,
                  const SolverScalars* sc) {
   ProfScope prof(st, PCF_K_PC_RHS);
-  if (L.coefs && L.fx == 2 && L.fy == 2 && L.nz <= kLineMaxNz) {
+  if (L.coefs && L.fx == 2 && L.fy == 2) {
     auto go = [&](auto ct) {
       using CT = decltype(ct);
       with_line_shape(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
         constexpr int W = decltype(w)::value, NPL = decltype(npl)::value;
-        hipLaunchKernelGGL((k_resid_restrict<W, NPL, BT, CT>), dim3(LineTile<float>::count(L.nx, L.ny)),
-                           dim3(kTileCols / W * ((L.nz + NPL - 1) / NPL)), 0, st->stream,
+        const int segs = (L.nz + NPL - 1) / NPL, parts = (L.nz + kLineMaxNz - 1) / kLineMaxNz;
+        hipLaunchKernelGGL((k_resid_restrict<W, NPL, BT, CT>), dim3(LineTile<float>::count(L.nx, L.ny), parts),
+                           dim3(kTileCols / W * ((segs + parts - 1) / parts)), 0, st->stream,
                            line_args<CT>(L, s, nullptr, &C), b, C.b, sc);
       });
     };
@@ -936,13 +974,19 @@ void mg_restrict(pcf_state* st, const MgLevel& L, const MgLevel& C, const BT* b,
   }
   const MgCoefs A = coefs_of(L);
   const Lay fl = lay_of(L), cl = lay_of(C);
-  const dim3 grd((unsigned)columns(C) * blocks_for(L.nz, 64)), blk(64, L.fx * L.fy);
-  if (L.fx == 2 && L.fy == 2)
-    hipLaunchKernelGGL((k_resid_restrict_any<2, 2, BT>), grd, blk, 0, st->stream, A, b, s, C.b, fl, cl, sc);
-  else if (L.fx == 2)
-    hipLaunchKernelGGL((k_resid_restrict_any<2, 1, BT>), grd, blk, 0, st->stream, A, b, s, C.b, fl, cl, sc);
-  else
-    hipLaunchKernelGGL((k_resid_restrict_any<1, 2, BT>), grd, blk, 0, st->stream, A, b, s, C.b, fl, cl, sc);
+  auto go = [&](auto fx, auto fy) {
+    constexpr int FX = decltype(fx)::value, FY = decltype(fy)::value;
+    if (L.zf)
+      hipLaunchKernelGGL((k_resid_restrict_columns<FX, FY, BT>), dim3((unsigned)columns(C) * blocks_for(L.nz, 64)),
+                         dim3(64, FX * FY), 0, st->stream, A, b, s, C.b, fl, cl, sc);
+    else
+      hipLaunchKernelGGL((k_resid_restrict_rows<FX, FY, BT>), dim3(blocks_for((long long)L.nx * C.ny * L.nz, 256)),
+                         dim3(256), 0, st->stream, A, b, s, C.b, fl, cl, sc);
+  };
+  using std::integral_constant;
+  if (L.fx == 2 && L.fy == 2) go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+  else if (L.fx == 2) go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+  else go(integral_constant<int, 1>{}, integral_constant<int, 2>{});
 }
 
 // The coarsest level: mg_coarse_steps smoothing steps from zero.
@@ -1199,7 +1243,7 @@ int alloc_mixed(pcf_state* st) {
   // FP32 arrays of the finest level where the column kernels or the general
   // residual read them; the line steps read the packed ones
   const bool pair = g.nx % 2 == 0 && g.nx >= kMgMinSize && g.ny % 2 == 0 && g.ny >= kMgMinSize;
-  if (multigrid && (!L0.coefs || !pair || g.nz > kLineMaxNz)) {
+  if (multigrid && (!L0.coefs || !pair)) {
     for (int t = 0; t < T_COUNT; ++t)
       if ((rc = af(&L0.a[t]))) return rc;
     for (float** p : {&L0.P, &L0.E, &L0.Q})

@@ -12,11 +12,12 @@ with deta scaled per level by the aggregation of the couplings.  V-cycle:
 2 pre-smoothing steps from 0, residual restriction, coarse correction with
 weight 1.5, 2 post-smoothing steps; 20 steps from 0 on the coarsest level
 (the defaults of mg_smoothing_steps and mg_coarse_steps).  round_apply
-emulates a reduced storage of the coefficients where the device's row
-kernels apply them: the horizontal part of the smoother on the levels with
-more than row_columns columns, and their residual where it is restricted by
-the fused 2 x 2 kernel (nx % 4 == 0); the line solve keeps the unrounded
-coefficients.
+emulates a reduced storage of the coefficients as the device applies them:
+in the horizontal part of the smoother on the levels with more than 1024
+columns (more than 512 levels: all), and in their residual where the device
+keeps no unrounded copy to read, which is on the coarse levels of at most 2048
+columns (stored z fastest) and where 2 x 2 columns are aggregated; the line
+solve keeps the unrounded coefficients.
 """
 import numpy as np
 
@@ -81,7 +82,7 @@ def coarsen(C, fx, fy):
     return out
 
 
-def levels(C, dx, dy, dtau=1.0, round_apply=None, row_columns=1024):
+def levels(C, dx, dy, dtau=1.0, round_apply=None):
     cx, cy = 1.0 / dx ** 2, 1.0 / dy ** 2
     lv = [{"C": C, "deta": dtau / (2 * (cx + cy))}]
     while True:
@@ -94,11 +95,11 @@ def levels(C, dx, dy, dtau=1.0, round_apply=None, row_columns=1024):
         cx, cy = cx * fy, cy * fx
         lv.append({"C": coarsen(lv[-1]["C"], fx, fy), "deta": dtau / (2 * (cx + cy))})
     if round_apply is not None:
-        for L in lv:
-            nx, ny, _ = L["C"]["AC"].shape
-            if nx * ny > row_columns:
+        for l, L in enumerate(lv):
+            nx, ny, nz = L["C"]["AC"].shape
+            if nx * ny > 1024 or nz > 512:
                 L["A"] = {n: round_apply(c) for n, c in L["C"].items()}
-                if L.get("f") == (2, 2) and nx % 4 == 0:
+                if L.get("f") == (2, 2) or (l > 0 and nx * ny <= 2048 and nz <= 512):
                     L["R"] = L["A"]
     return lv
 

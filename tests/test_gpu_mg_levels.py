@@ -35,8 +35,18 @@ def vcycle_error(pcf, shape, storage, nu=2, coarse=4):
     return err
 
 
-@pytest.mark.parametrize("shape,storage", [((68, 40, 264), "fp32"), ((48, 64, 520), "fp32")])
+@pytest.mark.parametrize("shape,storage", [((68, 40, 264), "fp32"), ((48, 64, 520), "fp32"), ((68, 40, 264), "bf16")])
 def test_tall_levels_match_the_restatement(pcf, shape, storage):
     """More than 256 levels on the levels smoothed by line steps (2720
     columns; beyond 512 levels all)."""
+    assert vcycle_error(pcf, shape, storage) <= 1e-3
+
+
+@pytest.mark.parametrize("storage", ["fp32", "bf16"])
+@pytest.mark.parametrize("shape", [(64, 45, 24), (45, 64, 24), (32, 30, 70), (33, 24, 264)])
+def test_unpaired_levels_match_the_restatement(pcf, shape, storage):
+    """An odd size: 2 x 1 and 1 x 2 aggregation of finest levels smoothed by
+    line steps (2880 columns), whose first coarse levels of 1440 columns are
+    z fastest and rounded with bf16 storage; finest levels of at most 1024
+    columns, paired and not, up to 264 levels."""
     assert vcycle_error(pcf, shape, storage) <= 1e-3
