@@ -221,19 +221,20 @@ __device__ __forceinline__ void line_solve_segments(const R* __restrict__ f, int
     }
 }
 
-// The same line solve for columns of any height, one column wide (W = 1): the
-// block's first `own` segments take the levels in chunks of own NPL, upwards
+// The same line solve for columns of any height, one column wide (W = 1), CB
+// columns a block: its first `own` segments take the levels in chunks of own NPL, upwards
 // and then downwards, the value at a chunk's edge going on to the next one in
 // LDS; idle threads of a wider block run identity maps.  rhs(k0, r): the
 // right-hand sides of the NPL levels from k0; f: the tile's packed factors at
 // the thread's column; keep(k, s) and kept(k): a thread's own scratch for the
 // upward sweep of all chunks but the last, inside the column; put(k, y): the
-// solution at a level inside it.  lds: 2 blockDim.x + cols values.
-template <typename R, int NPL, class Rhs, class Keep, class Kept, class Put>
-__device__ __forceinline__ void line_solve_chunks(const R* __restrict__ f, int nz, int own, int tx, int seg, Rhs rhs,
+// solution at a level inside it.  lds: 2 blockDim.x + CB values.
+template <typename R, int CB, int NPL, class Rhs, class Keep, class Kept, class Put>
+__device__ __forceinline__ void line_solve_chunks(const R* __restrict__ f, int nz, int own, Rhs rhs,
                                                   Keep keep, Kept kept, Put put, R* lds) {
   constexpr int cols = LineTile<R>::cols;
   R *la = lds, *lb = la + blockDim.x, *edge = lb + blockDim.x;
+  const int tx = threadIdx.x % CB, seg = threadIdx.x / CB;
   const int chunk = own * NPL, chunks = (nz + chunk - 1) / chunk;
   R r[NPL][1], in = 0;
   for (int ch = 0; ch < chunks; ++ch) {
@@ -261,7 +262,7 @@ __device__ __forceinline__ void line_solve_chunks(const R* __restrict__ f, int n
     __syncthreads();
     R s = in;
 #pragma unroll 4
-    for (int t = 0; t < seg; ++t) s = la[t * cols + tx] + lb[t * cols + tx] * s;
+    for (int t = 0; t < seg; ++t) s = la[t * CB + tx] + lb[t * CB + tx] * s;
 #pragma unroll
     for (int u = 0; u < NPL; ++u) {
       s = (r[u][0] + e[u] * s) * p[u];
@@ -297,7 +298,7 @@ __device__ __forceinline__ void line_solve_chunks(const R* __restrict__ f, int n
     __syncthreads();
     R y = in;
 #pragma unroll 4
-    for (int t = own - 1; t > seg; --t) y = la[t * cols + tx] + lb[t * cols + tx] * y;
+    for (int t = own - 1; t > seg; --t) y = la[t * CB + tx] + lb[t * CB + tx] * y;
 #pragma unroll
     for (int u = NPL - 1; u >= 0; --u) {
       y = r[u][0] + q[u] * y;

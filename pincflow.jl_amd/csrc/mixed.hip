@@ -189,13 +189,27 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)
 }
 
 constexpr int kLineMaxNz = 256;  // levels of k_line_step32's columns (taller ones: k_line_tall32)
-constexpr int kTallNpl = 16;     // levels per thread of a chunk of a taller column
 
-// segments of a tall column's chunks: the fewest chunks of at most kLineMaxNz
-// levels, and the levels spread over them
-inline __host__ __device__ int tall_segments(int nz) {
-  const int chunks = (nz + kLineMaxNz - 1) / kLineMaxNz, levels = (nz + chunks - 1) / chunks;
-  return (levels + kTallNpl - 1) / kTallNpl;
+// A block of a taller column's step: CB columns of a tile, NPL levels per
+// thread, and the segments of its chunks, the fewest chunks that 1024 threads
+// allow with the levels spread over them.
+template <int CB, int NPL>
+struct TallBlock {
+  static constexpr int columns = CB, npl = NPL, parts = kTileCols / CB;  // blocks per tile
+  static __host__ __device__ int segments(int nz) {
+    const int most = 1024 / CB * NPL, chunks = (nz + most - 1) / most, levels = (nz + chunks - 1) / chunks;
+    return (levels + NPL - 1) / NPL;
+  }
+};
+// Whole tiles, and half tiles on grids of few tiles, whose twice as many blocks
+// do not yet outnumber the 256 CUs and take half the chunks.  Whole / half
+// tiles, bf16, one application of two steps at 300 levels: 76 / 55 us on 64
+// tiles (64 x 64), 88 / 76 on 128 (128 x 64), 92 / 108 on 144 (96 x 96).
+constexpr int kTallFewTiles = 128;
+template <class F>
+void with_tall_block(int nx, int ny, F&& f) {
+  if (LineTile<float>::count(nx, ny) <= kTallFewTiles) f(TallBlock<32, 16>{});
+  else f(TallBlock<64, 16>{});
 }
 
 // The same step for columns of more than kLineMaxNz levels, chunk by chunk;
@@ -204,38 +218,43 @@ inline __host__ __device__ int tall_segments(int nz) {
 // trips of a chunk on a small one.  One application of two steps, FP32 / bf16
 // storage, with a horizontal kernel and a line solve apart, with a thread per
 // column for both, and chunk by chunk:
-//   64 x 64 x 300    145 / 138   632 / 614    92 /  77 us
-//   256 x 128 x 320  382 / 307   836 / 802   307 / 231 us
-template <bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
+//   64 x 64 x 300    145 / 138   632 / 614    63 /  55 us
+//   256 x 128 x 320  382 / 307   836 / 802   312 / 232 us
+template <class TB, bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
 __device__ __forceinline__ void line_tall32(const LineArgs<CT>& A, const BT* __restrict__ b, OutT* __restrict__ out,
-                                            float* col, int tile) {
+                                            float* col, int block) {
   extern __shared__ float line_shared[];
-  const LineThread<float, 1, kTallNpl> t(tile, A.nx, A.ny, A.nz);
-  const size_t sxy = (size_t)A.nx * A.ny, c = (size_t)t.i + (size_t)A.nx * t.j, tc = (size_t)tile * A.nz;
-  auto rhs = [&](int k0, float (&r)[kTallNpl][1]) {
+  constexpr int NPL = TB::npl;
+  const int nx = A.nx, ny = A.ny, nz = A.nz, tile = block / TB::parts;
+  const int tx = block % TB::parts * TB::columns + threadIdx.x % TB::columns, tiles_x = (nx + kTileX - 1) / kTileX;
+  int i = tile % tiles_x * kTileX + tx % kTileX, j = tile / tiles_x * LineTile<float>::Y + tx / kTileX;
+  const bool act = i < nx && j < ny;
+  i = min(i, nx - 1);  // idle threads read cells of the grid
+  j = min(j, ny - 1);
+  const size_t sxy = (size_t)nx * ny, c = (size_t)i + (size_t)nx * j, tc = (size_t)tile * nz;
+  auto rhs = [&](int k0, float (&r)[NPL][1]) {
     if constexpr (FIRST) {
 #pragma unroll
-      for (int u = 0; u < kTallNpl; ++u)
-        r[u][0] = A.deta * (0.0f - (float)__builtin_nontemporal_load(b + c + sxy * min(k0 + u, A.nz - 1)));
+      for (int u = 0; u < NPL; ++u)
+        r[u][0] = A.deta * (0.0f - (float)__builtin_nontemporal_load(b + c + sxy * min(k0 + u, nz - 1)));
     } else {
-      line_rhs<float, 1, kTallNpl, 0, false, CT, BT>(A.coefs + (tc + k0) * T_COUNT * kTileCols + t.tx,
-                                                     LineRead<1, PRO, CT>{A}, b, A.nx, A.ny, A.nz, A.deta, t.i, t.j,
-                                                     k0, r);
+      line_rhs<float, 1, NPL, 0, false, CT, BT>(
+          A.coefs + (tc + k0) * T_COUNT * kTileCols + tx, LineRead<1, PRO, CT>{A}, b, nx, ny, nz, A.deta, i, j, k0, r);
     }
   };
   // (idle columns of a partial tile keep nothing: their cells are another's)
-  line_solve_chunks<float, kTallNpl>(
-      A.factors + tc * 3 * kTileCols + t.tx, A.nz, tall_segments(A.nz), t.tx, t.seg, rhs,
-      [&](int k, float s) { if (t.act) col[c + sxy * k] = s; },
-      [&](int k) { return t.act ? col[c + sxy * k] : 0.0f; },
-      [&](int k, float y) { if (t.act) out[c + sxy * k] = (OutT)y; }, line_shared);
+  line_solve_chunks<float, TB::columns, NPL>(
+      A.factors + tc * 3 * kTileCols + tx, nz, TB::segments(nz), rhs,
+      [&](int k, float s) { if (act) col[c + sxy * k] = s; },
+      [&](int k) { return act ? col[c + sxy * k] : 0.0f; },
+      [&](int k, float y) { if (act) out[c + sxy * k] = (OutT)y; }, line_shared);
 }
-template <bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
+template <class TB, bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)))
     k_line_tall32(LineArgs<CT> A, const BT* __restrict__ b, OutT* __restrict__ out, float* col,
                   const SolverScalars* sc) {
   if (sc && sc->done) return;
-  line_tall32<FIRST, PRO, CT, BT, OutT>(A, b, out, col, xcd_block(blockIdx.x, gridDim.x));
+  line_tall32<TB, FIRST, PRO, CT, BT, OutT>(A, b, out, col, xcd_block(blockIdx.x, gridDim.x));
 }
 
 __global__ void k_to_f32(const double* a, float* b, size_t n) {
@@ -714,9 +733,12 @@ void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, Out
     const LineArgs<CT> A = line_args<CT>(L, s, e, C);
     const dim3 grd(LineTile<float>::count(L.nx, L.ny));
     if (L.nz > kLineMaxNz) {
-      const int threads = kTileCols * tall_segments(L.nz);
-      hipLaunchKernelGGL((k_line_tall32<FIRST, PRO, CT, BT, OutT>), grd, dim3(threads), (line_lds<float, 1>(threads)),
-                         st->stream, A, b, out, L.col, sc);
+      with_tall_block(L.nx, L.ny, [&](auto tb) {
+        using TB = decltype(tb);
+        const int threads = TB::columns * TB::segments(L.nz);
+        hipLaunchKernelGGL((k_line_tall32<TB, FIRST, PRO, CT, BT, OutT>), dim3(grd.x * TB::parts), dim3(threads),
+                           (line_lds<float, 1>(threads)), st->stream, A, b, out, L.col, sc);
+      });
     } else {
       with_line_shape(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
         constexpr int W = decltype(w)::value, NPL = decltype(npl)::value;

@@ -49,10 +49,12 @@ def test_fp32_line_step_matches_the_oracle(pcf, abi, oracle_mod, shape, storage,
 
 @pytest.mark.parametrize("shape,storage,iterations", [
     ((33, 3, 257), "fp32", 3), ((8, 3, 272), "bf16", 2), ((31, 5, 512), "fp32", 2), ((66, 1, 513), "bf16", 3),
-    ((34, 3, 600), "fp32", 1), ((34, 3, 601), "fp32", 4)])
+    ((34, 3, 600), "fp32", 1), ((34, 3, 601), "fp32", 4), ((33, 3, 1030), "bf16", 2),
+    ((256, 33, 257), "fp32", 3), ((250, 34, 300), "bf16", 2), ((260, 30, 520), "fp32", 2)])
 def test_fp32_line_step_of_tall_columns_matches_the_oracle(pcf, abi, oracle_mod, shape, storage, iterations):
-    """Columns of two and three chunks, the last one shorter or full, with
-    partial tiles: the bound above."""
+    """Columns of one to three chunks, the last one shorter or full, in half
+    tiles (grids of up to 128 tiles) and whole ones, with partial tiles: the
+    bound above."""
     err = preconditioned(pcf, abi, oracle_mod, shape, "mixed", storage, iterations)
     print(shape, storage, iterations, err)
     assert err <= 1e-4, err
