@@ -560,7 +560,10 @@ __device__ __forceinline__ void column_step(const MgCoefs& A, const float* P, co
   // every load is unconditional, at a level inside the column (zeroed beyond
   // the walls where it is used): a branch per neighbour made each load wait
   // for the one before (14 us against 7 for a first post-smoothing step at
-  // 32 x 32 x 128)
+  // 32 x 32 x 128).  With four levels per lane or more the barrier below keeps
+  // one level's loads in flight: those of all spilt (k_coarse_solve at 10 x 1 x
+  // 160: 15.4 us a step against 6.7; the 26 x 16 x 400 level's post-smoothing
+  // 55 against 52).
 #pragma unroll
   for (int u = 0; u < NPL; ++u) {
     const int k = NPL * lane + u;
@@ -597,6 +600,7 @@ __device__ __forceinline__ void column_step(const MgCoefs& A, const float* P, co
       r = s[0][2] + deta * (v - bv);
     }
     line_maps(p, e, qv, k, nz, r, fa[u], fb[u], q[u]);
+    if (!FIRST && NPL >= 4 && u + 1 < NPL) asm volatile("" : "+v"(fa[u])::"memory");
   }
   scan_line<NPL>(fa, fb, q, nz, y);
 }
@@ -755,7 +759,7 @@ void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, Out
       if (e) go(ct, std::true_type{});
       else go(ct, std::false_type{});
     };
-    if (bf16_storage(st)) pick(uint16_t{});
+    if (L.bf16) pick(uint16_t{});
     else pick(float{});
   }
 }
@@ -778,7 +782,7 @@ void line_fuse(pcf_state* st, const MgLevel& L, const BicgFuse& F, int fuse, flo
 // Pack a level's coefficients and factors for the line steps.
 template <typename SrcT>
 void line_pack(pcf_state* st, const MgLevel& L, const LineCoefs<SrcT>& A) {
-  if (bf16_storage(st)) launch_line_pack(st->stream, A, (uint16_t*)L.coefs, L.factors, L.nx, L.ny, L.nz);
+  if (L.bf16) launch_line_pack(st->stream, A, (uint16_t*)L.coefs, L.factors, L.nx, L.ny, L.nz);
   else launch_line_pack(st->stream, A, (float*)L.coefs, L.factors, L.nx, L.ny, L.nz);
 }
 
@@ -786,15 +790,22 @@ void line_pack(pcf_state* st, const MgLevel& L, const LineCoefs<SrcT>& A) {
 // z fastest and smoothed one wavefront per column, larger ones x fastest by
 // line steps (48 x 40 x 64: 5 us per step against 11, where a tile per
 // workgroup leaves the chip empty; 64 x 64 x 128 keeps line steps).  A finest
-// level, always x fastest, is smoothed column by column up to kColumnCols.
+// level, always x fastest, is smoothed column by column up to kColumnCols
+// columns, 256 levels and kColumnCells cells: lanes along z of an x-fastest
+// array touch a cache line each, which a small grid's caches hold (V-cycle by
+// column / by line steps: 208 / 238 us at 16 x 16 x 200, 234 / 236 at
+// 28 x 28 x 200, 373 / 302 at 32 x 32 x 200, 323 / 293 at 16 x 16 x 300).
 // The coarsest level runs all its steps in one workgroup when it has at most
 // 16 columns.
-constexpr size_t kColumnCols = 1024, kCoarseColumnCols = 2048;
+constexpr size_t kColumnCols = 1024, kCoarseColumnCols = 2048, kColumnCells = 160000;
 constexpr int kScanMaxNz = 512;
 constexpr size_t kCoarseLdsFloats = 16384;
 
 size_t columns(const MgLevel& L) { return (size_t)L.nx * L.ny; }
-bool column_path(const MgLevel& L) { return (L.zf || columns(L) <= kColumnCols) && L.nz <= kScanMaxNz; }
+bool column_path(const MgLevel& L) {
+  if (L.zf) return L.nz <= kScanMaxNz;
+  return columns(L) <= kColumnCols && L.nz <= 256 && columns(L) * L.nz <= kColumnCells;
+}
 
 MgCoefs coefs_of(const MgLevel& L) {
   MgCoefs A;
@@ -990,7 +1001,7 @@ void mg_restrict(pcf_state* st, const MgLevel& L, const MgLevel& C, const BT* b,
                            line_args<CT>(L, s, nullptr, &C), b, C.b, sc);
       });
     };
-    if (bf16_storage(st)) go(uint16_t{});
+    if (L.bf16) go(uint16_t{});
     else go(float{});
     return;
   }
@@ -1236,10 +1247,13 @@ int alloc_mixed(pcf_state* st) {
   const size_t N = st->g.nv();
   const bool multigrid = st->cfg.preconditioner_type == PCF_PC_MULTIGRID;
   auto af = [&](float** p) -> int { return device_alloc(st, p, N); };
-  // the packed arrays of a level smoothed by line steps
+  // the packed arrays of a level smoothed by line steps; in multigrid, bf16
+  // storage covers the levels of more than kColumnCols columns and those too
+  // tall to be smoothed column by column
   auto packed = [&](MgLevel& L) -> int {
+    L.bf16 = bf16_storage(st) && (!multigrid || columns(L) > kColumnCols || L.nz > kScanMaxNz);
     const size_t n = (size_t)LineTile<float>::count(L.nx, L.ny) * kTileCols * L.nz;
-    int rc1 = device_alloc(st, &L.coefs, n * T_COUNT * (bf16_storage(st) ? 2 : 4));
+    int rc1 = device_alloc(st, &L.coefs, n * T_COUNT * (L.bf16 ? 2 : 4));
     return rc1 ? rc1 : device_alloc(st, &L.factors, 3 * n);
   };
   int rc;

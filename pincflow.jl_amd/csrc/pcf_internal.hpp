@@ -82,8 +82,9 @@ struct MgLevel {
   bool zf = false;  // arrays stored z fastest (else x fastest)
   float deta = 0.0f;
   float* a[T_COUNT] = {};
-  // levels smoothed by line steps: packed coefficients (float or bf16 bits)
-  // and line-solve factors (k_line_pack)
+  // levels smoothed by line steps: packed coefficients (float, or bf16 bits
+  // with bf16 set) and line-solve factors (k_line_pack)
+  bool bf16 = false;
   char* coefs = nullptr;
   float* factors = nullptr;
   float *P = nullptr, *E = nullptr, *Q = nullptr;

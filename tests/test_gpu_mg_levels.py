@@ -50,3 +50,17 @@ def test_unpaired_levels_match_the_restatement(pcf, shape, storage):
     z fastest and rounded with bf16 storage; finest levels of at most 1024
     columns, paired and not, up to 264 levels."""
     assert vcycle_error(pcf, shape, storage) <= 1e-3
+
+
+@pytest.mark.parametrize("shape,storage", [
+    ((16, 16, 160), "fp32"), ((28, 24, 238), "fp32"), ((28, 24, 239), "bf16"), ((32, 32, 200), "bf16"),
+    ((16, 12, 257), "bf16"), ((32, 30, 200), "fp32"), ((44, 48, 200), "bf16")])
+def test_small_levels_of_many_levels_match_the_restatement(pcf, shape, storage):
+    """129 to 512 levels, four and eight per lane, of levels smoothed column
+    by column and of the coarsest one; both sides of the finest level's rule
+    (1024 columns, 256 levels, 160000 cells), whose line steps read unrounded
+    coefficients up to 1024 columns with either storage.  Four steps on the
+    coarsest level as above: the twenty of the default leave 2e-3 at
+    16 x 16 x 160, the rounding of the scan over a wavefront's lanes on the
+    nearly singular level."""
+    assert vcycle_error(pcf, shape, storage) <= 1e-3
