@@ -188,9 +188,10 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)
   }
 }
 
-constexpr int kLineMaxNz = 256;  // levels of k_line_step32's columns (taller ones: k_line_tall32)
+constexpr int kLineMaxNz = 256;  // most levels of k_line_step32's columns (taller ones, and on few tiles those of
+                                 // more than 128: k_line_tall32)
 
-// A block of a taller column's step: CB columns of a tile, NPL levels per
+// A block of a tall column's step: CB columns of a tile, NPL levels per
 // thread, and the segments of its chunks, the fewest chunks that 1024 threads
 // allow with the levels spread over them.
 template <int CB, int NPL>
@@ -204,16 +205,23 @@ struct TallBlock {
 // Whole tiles, and half tiles on grids of few tiles, whose twice as many blocks
 // do not yet outnumber the 256 CUs and take half the chunks.  Whole / half
 // tiles, bf16, one application of two steps at 300 levels: 76 / 55 us on 64
-// tiles (64 x 64), 88 / 76 on 128 (128 x 64), 92 / 108 on 144 (96 x 96).
+// tiles (64 x 64), 88 / 76 on 128 (128 x 64), 92 / 108 on 144 (96 x 96).  The
+// step that adds the coarse correction (PRO) spills with 16 levels per thread
+// and takes smaller blocks of 8 on few tiles: V-cycles of 1105 / 1007 us at
+// 64 x 64 x 600, 270 / 241 at 48 x 40 x 200.
 constexpr int kTallFewTiles = 128;
-template <class F>
-void with_tall_block(int nx, int ny, F&& f) {
-  if (LineTile<float>::count(nx, ny) <= kTallFewTiles) f(TallBlock<32, 16>{});
+template <bool PRO, class F>
+void with_tall_block(int nx, int ny, int nz, F&& f) {
+  const bool few = LineTile<float>::count(nx, ny) <= kTallFewTiles;
+  if (PRO && few && nz <= 256) f(TallBlock<32, 8>{});
+  else if (PRO && few) f(TallBlock<16, 8>{});
+  else if (few) f(TallBlock<32, 16>{});
   else f(TallBlock<64, 16>{});
 }
 
-// The same step for columns of more than kLineMaxNz levels, chunk by chunk;
-// col: FP32 scratch of the grid's size, which keeps the upward sweep.  Like
+// The same step for tall columns, chunk by chunk;
+// col: FP32 scratch of the grid's size, which keeps the upward sweep of all
+// chunks but the last (null up to kLineMaxNz levels, one chunk).  Like
 // the shorter columns it is bound by memory on a large grid and by the round
 // trips of a chunk on a small one.  One application of two steps, FP32 / bf16
 // storage, with a horizontal kernel and a line solve apart, with a thread per
@@ -252,8 +260,12 @@ __device__ __forceinline__ void line_tall32(const LineArgs<CT>& A, const BT* __r
 template <class TB, bool FIRST, bool PRO, typename CT, typename BT, typename OutT>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4)))
     k_line_tall32(LineArgs<CT> A, const BT* __restrict__ b, OutT* __restrict__ out, float* col,
-                  const SolverScalars* sc) {
-  if (sc && sc->done) return;
+                  const SolverScalars* sc, SolverScalars* commit) {
+  if (!FIRST && commit) {
+    if (!fuse_commit(commit)) return;
+  } else if (sc && sc->done) {
+    return;
+  }
   line_tall32<TB, FIRST, PRO, CT, BT, OutT>(A, b, out, col, xcd_block(blockIdx.x, gridDim.x));
 }
 
@@ -695,12 +707,13 @@ bool bf16_storage(const pcf_state* st) { return st->cfg.preconditioner_storage =
 // 128 x 128 x 128 and 18 against 14 at 48 x 40 x 64, where the threads do.
 // The results do not depend on W.
 constexpr long long kLineWideCells = 4 << 20;
+bool line_wide(int nx, int ny, int nz) { return nx % 4 == 0 && (long long)nx * ny * nz >= kLineWideCells; }
 template <class F>
 void with_line_shape(int nx, int ny, int nz, F&& f) {
   using std::integral_constant;
   if (nz > 128)
     f(integral_constant<int, 1>{}, integral_constant<int, 16>{});
-  else if (nx % 4 == 0 && (long long)nx * ny * nz >= kLineWideCells)
+  else if (line_wide(nx, ny, nz))
     f(integral_constant<int, 4>{}, integral_constant<int, 8>{});
   else
     f(integral_constant<int, 1>{}, integral_constant<int, 8>{});
@@ -736,12 +749,12 @@ void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, Out
     using CT = decltype(ct);
     const LineArgs<CT> A = line_args<CT>(L, s, e, C);
     const dim3 grd(LineTile<float>::count(L.nx, L.ny));
-    if (L.nz > kLineMaxNz) {
-      with_tall_block(L.nx, L.ny, [&](auto tb) {
+    if (L.nz > kLineMaxNz || (L.nz > 128 && LineTile<float>::count(L.nx, L.ny) <= kTallFewTiles)) {
+      with_tall_block<PRO>(L.nx, L.ny, L.nz, [&](auto tb) {
         using TB = decltype(tb);
         const int threads = TB::columns * TB::segments(L.nz);
         hipLaunchKernelGGL((k_line_tall32<TB, FIRST, PRO, CT, BT, OutT>), dim3(grd.x * TB::parts), dim3(threads),
-                           (line_lds<float, 1>(threads)), st->stream, A, b, out, L.col, sc);
+                           (line_lds<float, 1>(threads)), st->stream, A, b, out, L.col, sc, commit);
       });
     } else {
       with_line_shape(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
@@ -993,13 +1006,17 @@ void mg_restrict(pcf_state* st, const MgLevel& L, const MgLevel& C, const BT* b,
   if (L.coefs && L.fx == 2 && L.fy == 2) {
     auto go = [&](auto ct) {
       using CT = decltype(ct);
-      with_line_shape(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
-        constexpr int W = decltype(w)::value, NPL = decltype(npl)::value;
-        const int segs = (L.nz + NPL - 1) / NPL, parts = (L.nz + kLineMaxNz - 1) / kLineMaxNz;
+      // 8 levels per thread at any height, as no level waits for another (16:
+      // 20 us against 13 at 44 x 44 x 130)
+      auto launch = [&](auto w) {
+        constexpr int W = decltype(w)::value, NPL = 8, most = (W == 4 ? 512 : 1024) / (kTileCols / W);
+        const int segs = (L.nz + NPL - 1) / NPL, parts = (segs + most - 1) / most;
         hipLaunchKernelGGL((k_resid_restrict<W, NPL, BT, CT>), dim3(LineTile<float>::count(L.nx, L.ny), parts),
                            dim3(kTileCols / W * ((segs + parts - 1) / parts)), 0, st->stream,
                            line_args<CT>(L, s, nullptr, &C), b, C.b, sc);
-      });
+      };
+      if (line_wide(L.nx, L.ny, L.nz)) launch(std::integral_constant<int, 4>{});
+      else launch(std::integral_constant<int, 1>{});
     };
     if (L.bf16) go(uint16_t{});
     else go(float{});
