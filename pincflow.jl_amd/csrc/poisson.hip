@@ -1474,11 +1474,16 @@ int pc_factors(pcf_state* st) {
 // solve apart, both bound by memory, are faster.  Measured per application:
 // 30 us against 49 at 75 x 53 x 41, 18 against 36 at 40 x 1 x 40, even at
 // 120 x 96 x 72, 568 against 416 at 256 x 256 x 128.  A column's right-hand
-// sides and factors must fit in LDS (kLine64MaxNz levels: 128 KiB).  Both
-// paths round alike.
+// sides and factors must fit in LDS (kLine64MaxNz levels: 128 KiB), and on
+// many tiles of fewer than 8 levels half of a block's threads or more are idle
+// (an iteration at 200 x 200 x 6, 2600 tiles: 118 us against 113; at 60 x 60 x
+// 6, 240 tiles: 67 against 88; at 200 x 200 x 15: 178 against 198).  Both paths
+// round alike.
 constexpr long long kLine64Cells = 600000;
+constexpr int kLine64FlatTiles = 1024;
 static bool use_line64(const Geo& g) {
-  return g.nz <= kLine64MaxNz && (long long)g.nx * g.ny * g.nz <= kLine64Cells;
+  return g.nz <= kLine64MaxNz && (long long)g.nx * g.ny * g.nz <= kLine64Cells &&
+         (g.nz >= 8 || LineTile<double>::count(g.nx, g.ny) <= kLine64FlatTiles);
 }
 
 // The packed arrays of the FP64 line steps (pcf_create)
@@ -1633,10 +1638,21 @@ int dot(pcf_state* st, const double* a, const double* b, double* out) {
 // leaves a residual no smaller than |b|, in which case it starts from 0.
 //
 // Most partials of an apply that the blocks of a fused iteration sum again
-// each, and the solves that run fused iterations: those whose preconditioner
-// is line steps of two pseudo-time steps or more.
-constexpr int kFusePartials = 2048;
-static bool fusable(const pcf_state* st) { return st->pc_coefs && st->cfg.preconditioner_iterations >= 2; }
+// each, and the FP64 solves that run fused iterations: those whose
+// preconditioner is line steps of two pseudo-time steps or more, with blocks of
+// three wavefronts or more, which share the sums, and at most two blocks per
+// CU.  An iteration, fused / unfused: 98 / 104 us at 96 x 1 x 128 (6 blocks of
+// 512 threads), 101 / 103 at 75 x 53 x 41 (265 of 192), 236 / 234 at 100 x 60 x
+// 100 (420 of 448), but 73 / 71 at 60 x 60 x 15 (240 of 64) and 194 / 169 at
+// 400 x 100 x 15 (2500 of 64).
+constexpr int kFusePartials = 2048, kFuseThreads = 192, kFuseTiles = 512;
+static bool fusable(const pcf_state* st) {
+  const Geo& g = st->g;
+  bool fits = false;
+  with_line64(g, [&](auto npl) { fits = (int)line_block64(g, decltype(npl)::value).x >= kFuseThreads; });
+  return st->pc_coefs && st->cfg.preconditioner_iterations >= 2 && fits &&
+         LineTile<double>::count(g.nx, g.ny) <= kFuseTiles;
+}
 
 int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess, double guess_scale,
                   int* niter_out) {
