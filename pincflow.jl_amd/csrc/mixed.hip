@@ -128,7 +128,7 @@ __device__ __forceinline__ void line_step32(const LineArgs<CT>& A, const BT* __r
     }
   } else {
     // what the registers allow
-    constexpr int DEPTH = W == 1 && NPL == 8 && !PRO ? 1 : W == 4 && !PRO && sizeof(CT) == 2 ? -1 : 0;
+    constexpr int DEPTH = W == 1 && NPL <= 8 && !PRO ? 1 : W == 4 && !PRO && sizeof(CT) == 2 ? -1 : 0;
     line_rhs<float, W, NPL, DEPTH, false, CT, BT>(A.coefs + t.c * T_COUNT * kTileCols + t.tx * W, LineRead<W, PRO, CT>{A}, b,
                                            nx, ny, nz, A.deta, t.i, t.j, t.k0, r);
   }
@@ -707,10 +707,26 @@ bool bf16_storage(const pcf_state* st) { return st->cfg.preconditioner_storage =
 // 128 x 128 x 128 and 18 against 14 at 48 x 40 x 64, where the threads do.
 // The results do not depend on W.
 constexpr long long kLineWideCells = 4 << 20;
-bool line_wide(int nx, int ny, int nz) { return nx % 4 == 0 && (long long)nx * ny * nz >= kLineWideCells; }
-template <class F>
+__host__ __device__ inline bool line_wide(int nx, int ny, int nz) {
+  return nx % 4 == 0 && (long long)nx * ny * nz >= kLineWideCells;
+}
+// STEP (a step that is not from zero, with coefficients CT): four levels per
+// thread on a flat grid where eight would leave half a segment or more beyond
+// the top, with bf16 coefficients on a wide grid only.  Eight / four levels:
+// FP32 166 / 145 us at 512 x 512 x 17, 341 / 309 at 512 x 512 x 41, 64 / 54 at
+// 300 x 200 x 25; bf16 202 / 189 at 512 x 512 x 33, but 44 / 46 at 300 x 200 x 25.
+__host__ __device__ inline bool line_short(int nx, int ny, int nz, bool bf16) {
+  return nz <= 64 && (nz - 1) % 8 < 4 && (!bf16 || line_wide(nx, ny, nz));
+}
+template <bool STEP, typename CT, class F>
 void with_line_shape(int nx, int ny, int nz, F&& f) {
   using std::integral_constant;
+  if constexpr (STEP)
+    if (line_short(nx, ny, nz, sizeof(CT) == 2)) {
+      if (line_wide(nx, ny, nz)) f(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+      else if constexpr (sizeof(CT) == 4) f(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+      return;
+    }
   if (nz > 128)
     f(integral_constant<int, 1>{}, integral_constant<int, 16>{});
   else if (line_wide(nx, ny, nz))
@@ -757,7 +773,7 @@ void line_step(pcf_state* st, const MgLevel& L, const BT* b, const float* s, Out
                            (line_lds<float, 1>(threads)), st->stream, A, b, out, L.col, sc, commit);
       });
     } else {
-      with_line_shape(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
+      with_line_shape<!FIRST, CT>(L.nx, L.ny, L.nz, [&](auto w, auto npl) {
         constexpr int W = decltype(w)::value, NPL = decltype(npl)::value;
         const int threads = kTileCols / W * ((L.nz + NPL - 1) / NPL);
         hipLaunchKernelGGL((k_line_step32<W, NPL, FIRST, PRO, CT, BT, OutT>), grd, dim3(threads),
@@ -1219,7 +1235,9 @@ __global__ void __launch_bounds__(1024) kEm_line(const EnsTable* __restrict__ E,
   if constexpr (sizeof(OutT) == 8) dst = M.v[out];
   else dst = FIRST || from == 1 ? M.cur32 : M.rhs32;
   const double* v = M.v[in];
-  if (M.nz > 128)
+  if (!FIRST && line_short(M.nx, M.ny, M.nz, sizeof(CT) == 2))
+    line_step32<1, 4, FIRST, false, CT, double, OutT>(A, v, dst, b);
+  else if (M.nz > 128)
     line_step32<1, 16, FIRST, false, CT, double, OutT>(A, v, dst, b);
   else
     line_step32<1, 8, FIRST, false, CT, double, OutT>(A, v, dst, b);
@@ -1230,7 +1248,7 @@ __global__ void __launch_bounds__(1024) kEm_line(const EnsTable* __restrict__ E,
 // blocks and threads per block of a member's line steps
 int ensemble_line_blocks(const pcf_state* st) { return LineTile<float>::count(st->g.nx, st->g.ny); }
 int ensemble_line_threads(const pcf_state* st) {
-  const int npl = st->g.nz > 128 ? 16 : 8;
+  const int npl = line_short(st->g.nx, st->g.ny, st->g.nz, st->mg[0].bf16) ? 4 : st->g.nz > 128 ? 16 : 8;
   return kTileCols * ((st->g.nz + npl - 1) / npl);
 }
 bool ensemble_line_covers(const pcf_state* st) { return st->g.nz <= kLineMaxNz; }

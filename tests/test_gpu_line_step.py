@@ -48,6 +48,19 @@ def test_fp32_line_step_matches_the_oracle(pcf, abi, oracle_mod, shape, storage,
 
 
 @pytest.mark.parametrize("shape,storage,iterations", [
+    ((31, 3, 4), "fp32", 3), ((40, 5, 17), "fp32", 2), ((33, 4, 41), "fp32", 3), ((64, 3, 60), "fp32", 2),
+    ((33, 3, 61), "fp32", 2), ((260, 254, 64), "fp32", 2), ((516, 480, 17), "fp32", 2), ((516, 480, 17), "bf16", 3),
+    ((40, 5, 17), "bf16", 2)])
+def test_fp32_line_step_of_flat_grids_matches_the_oracle(pcf, abi, oracle_mod, shape, storage, iterations):
+    """Four levels per thread (up to 64 levels where eight leave half a
+    segment beyond the top, with bf16 storage on wide grids) and the sizes
+    beside them, one and four columns per thread: the bound above."""
+    err = preconditioned(pcf, abi, oracle_mod, shape, "mixed", storage, iterations)
+    print(shape, storage, iterations, err)
+    assert err <= 1e-4, err
+
+
+@pytest.mark.parametrize("shape,storage,iterations", [
     ((33, 3, 257), "fp32", 3), ((8, 3, 272), "bf16", 2), ((31, 5, 512), "fp32", 2), ((66, 1, 513), "bf16", 3),
     ((34, 3, 600), "fp32", 1), ((34, 3, 601), "fp32", 4), ((33, 3, 1030), "bf16", 2),
     ((256, 33, 257), "fp32", 3), ((250, 34, 300), "bf16", 2), ((260, 30, 520), "fp32", 2)])
