@@ -483,7 +483,7 @@ int pcf_set_solver_graphs(pcf_state* st, int32_t on);
  * reached its poisson_iterations.  Members step independently; every member
  * gets the bits of its own solve.  The batch
  * covers the line preconditioner (FP64, or FP32 in the mixed solve) on grids
- * with an even x_size (at most 256 levels in the mixed solve); other solves of
+ * with an even x_size; other solves of
  * a member run on their own.  A member's thread detaches when it stops
  * stepping. */
 typedef struct pcf_ensemble pcf_ensemble;

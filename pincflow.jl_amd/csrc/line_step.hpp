@@ -49,7 +49,7 @@ struct LineCoefs {
 template <typename R>
 struct LineTile {
   static constexpr int X = sizeof(R) == 8 ? 16 : 32, Y = sizeof(R) == 8 ? 1 : 2, cols = X * Y;
-  static int count(int nx, int ny) { return ((nx + X - 1) / X) * ((ny + Y - 1) / Y); }
+  static __host__ __device__ int count(int nx, int ny) { return ((nx + X - 1) / X) * ((ny + Y - 1) / Y); }
 };
 
 // The columns and levels of a thread of a tile; seg0: the block's first

@@ -211,7 +211,7 @@ struct TallBlock {
 // 64 x 64 x 600, 270 / 241 at 48 x 40 x 200.
 constexpr int kTallFewTiles = 128;
 template <bool PRO, class F>
-void with_tall_block(int nx, int ny, int nz, F&& f) {
+__host__ __device__ inline void with_tall_block(int nx, int ny, int nz, F&& f) {
   const bool few = LineTile<float>::count(nx, ny) <= kTallFewTiles;
   if (PRO && few && nz <= 256) f(TallBlock<32, 8>{});
   else if (PRO && few) f(TallBlock<16, 8>{});
@@ -1212,7 +1212,8 @@ __device__ __forceinline__ int ens_member32(const int* start, int count, int b) 
 // the member's FP32 iterate `from` (0: cur32, 1: rhs32), to v[out] (OutT
 // double) or the other FP32 buffer.  The members' columns may have different
 // heights: the segments beyond a column's top are identity maps.
-template <bool FIRST, typename CT, typename OutT>
+// TALL: columns of more than kLineMaxNz levels, in the blocks of line_step.
+template <bool TALL, bool FIRST, typename CT, typename OutT>
 __global__ void __launch_bounds__(1024) kEm_line(const EnsTable* __restrict__ E, const EnsList* __restrict__ L, int in,
                                                  int from, int out) {
   const int a = ens_member32(L->line_start, L->count, blockIdx.x);
@@ -1235,7 +1236,11 @@ __global__ void __launch_bounds__(1024) kEm_line(const EnsTable* __restrict__ E,
   if constexpr (sizeof(OutT) == 8) dst = M.v[out];
   else dst = FIRST || from == 1 ? M.cur32 : M.rhs32;
   const double* v = M.v[in];
-  if (!FIRST && line_short(M.nx, M.ny, M.nz, sizeof(CT) == 2))
+  if constexpr (TALL)
+    with_tall_block<false>(M.nx, M.ny, M.nz, [&](auto tb) {
+      line_tall32<decltype(tb), FIRST, false, CT, double, OutT>(A, v, dst, M.col32, b);
+    });
+  else if (!FIRST && line_short(M.nx, M.ny, M.nz, sizeof(CT) == 2))
     line_step32<1, 4, FIRST, false, CT, double, OutT>(A, v, dst, b);
   else if (M.nz > 128)
     line_step32<1, 16, FIRST, false, CT, double, OutT>(A, v, dst, b);
@@ -1246,35 +1251,55 @@ __global__ void __launch_bounds__(1024) kEm_line(const EnsTable* __restrict__ E,
 }  // namespace
 
 // blocks and threads per block of a member's line steps
-int ensemble_line_blocks(const pcf_state* st) { return LineTile<float>::count(st->g.nx, st->g.ny); }
-int ensemble_line_threads(const pcf_state* st) {
-  const int npl = line_short(st->g.nx, st->g.ny, st->g.nz, st->mg[0].bf16) ? 4 : st->g.nz > 128 ? 16 : 8;
-  return kTileCols * ((st->g.nz + npl - 1) / npl);
+bool ensemble_line_tall(const pcf_state* st) { return st->g.nz > kLineMaxNz; }
+int ensemble_line_blocks(const pcf_state* st) {
+  const Geo& g = st->g;
+  int blocks = LineTile<float>::count(g.nx, g.ny);
+  if (ensemble_line_tall(st))
+    with_tall_block<false>(g.nx, g.ny, g.nz, [&](auto tb) { blocks *= decltype(tb)::parts; });
+  return blocks;
 }
-bool ensemble_line_covers(const pcf_state* st) { return st->g.nz <= kLineMaxNz; }
+int ensemble_line_threads(const pcf_state* st) {
+  const Geo& g = st->g;
+  int threads = 0;
+  if (ensemble_line_tall(st)) {
+    with_tall_block<false>(g.nx, g.ny, g.nz,
+                           [&](auto tb) { threads = decltype(tb)::columns * decltype(tb)::segments(g.nz); });
+  } else {
+    const int npl = line_short(g.nx, g.ny, g.nz, st->mg[0].bf16) ? 4 : g.nz > 128 ? 16 : 8;
+    threads = kTileCols * ((g.nz + npl - 1) / npl);
+  }
+  return threads;
+}
 
 // M^-1 v[in] -> v[out] for every solve of the list (precondition_mixed's
 // line branch); threads: the largest of the members' blocks
-void ensemble_precondition_mixed(hipStream_t s, const EnsTable* dT, const EnsList* dL, const EnsList& L, int threads,
+template <bool TALL>
+static void precondition_members(hipStream_t s, const EnsTable* dT, const EnsList* dL, const EnsList& L, int threads,
                                  int iters, bool bf16, int in, int out) {
   const dim3 grd(L.line_start[L.count]), blk(threads);
   const unsigned lds = 4 * threads * sizeof(float);
   if (iters == 1) {
-    hipLaunchKernelGGL((kEm_line<true, float, double>), grd, blk, lds, s, dT, dL, in, 0, out);
+    hipLaunchKernelGGL((kEm_line<TALL, true, float, double>), grd, blk, lds, s, dT, dL, in, 0, out);
     return;
   }
-  hipLaunchKernelGGL((kEm_line<true, float, float>), grd, blk, lds, s, dT, dL, in, 0, out);
+  hipLaunchKernelGGL((kEm_line<TALL, true, float, float>), grd, blk, lds, s, dT, dL, in, 0, out);
   int from = 0;
   for (int it = 2; it <= iters; ++it, from ^= 1) {
     if (it == iters && bf16)
-      hipLaunchKernelGGL((kEm_line<false, uint16_t, double>), grd, blk, lds, s, dT, dL, in, from, out);
+      hipLaunchKernelGGL((kEm_line<TALL, false, uint16_t, double>), grd, blk, lds, s, dT, dL, in, from, out);
     else if (it == iters)
-      hipLaunchKernelGGL((kEm_line<false, float, double>), grd, blk, lds, s, dT, dL, in, from, out);
+      hipLaunchKernelGGL((kEm_line<TALL, false, float, double>), grd, blk, lds, s, dT, dL, in, from, out);
     else if (bf16)
-      hipLaunchKernelGGL((kEm_line<false, uint16_t, float>), grd, blk, lds, s, dT, dL, in, from, out);
+      hipLaunchKernelGGL((kEm_line<TALL, false, uint16_t, float>), grd, blk, lds, s, dT, dL, in, from, out);
     else
-      hipLaunchKernelGGL((kEm_line<false, float, float>), grd, blk, lds, s, dT, dL, in, from, out);
+      hipLaunchKernelGGL((kEm_line<TALL, false, float, float>), grd, blk, lds, s, dT, dL, in, from, out);
   }
+}
+void ensemble_precondition_mixed(hipStream_t s, const EnsTable* dT, const EnsList* dL, const EnsList& L, int threads,
+                                 bool tall, int iters, bool bf16, int in, int out) {
+  if (tall) precondition_members<true>(s, dT, dL, L, threads, iters, bf16, in, out);
+  else precondition_members<false>(s, dT, dL, L, threads, iters, bf16, in, out);
 }
 
 // Allocation of the mixed-precision buffers (pcf_create, precision MIXED).

@@ -153,7 +153,7 @@ struct EnsMember {
   const double *P, *E, *Q;          // FP64 line-solve factors
   const char* coefs32;              // mixed: packed coefficients and factors, FP32 iterates
   const float* factors32;
-  float *cur32, *rhs32;
+  float *cur32, *rhs32, *col32;
   double* partials;
   SolverScalars* sc;
   size_t n;                         // cells
@@ -440,13 +440,14 @@ int apply_bicgstab_mixed(pcf_state* st, double tolref, double dt, int* niter);
 int precondition_mixed(pcf_state* st, const double* sin, double* sout, const SolverScalars* sc, const BicgFuse* F,
                        int fuse);
 bool fusable_mixed(const pcf_state* st);
-// the ensemble batch's FP32 line preconditioner: a member's grid, whether it
-// covers the member, and the launches over a list (threads: the largest block)
+// the ensemble batch's FP32 line preconditioner: a member's grid, whether its
+// columns are tall, and the launches over a list of members with or without
+// tall columns (threads: the largest block)
 int ensemble_line_blocks(const pcf_state* st);
 int ensemble_line_threads(const pcf_state* st);
-bool ensemble_line_covers(const pcf_state* st);
+bool ensemble_line_tall(const pcf_state* st);
 void ensemble_precondition_mixed(hipStream_t s, const EnsTable* dT, const EnsList* dL, const EnsList& L, int threads,
-                                 int iters, bool bf16, int in, int out);
+                                 bool tall, int iters, bool bf16, int in, int out);
 int alloc_mixed(pcf_state* st);
 // Device buffer of `bytes` owned by the state (freed by pcf_destroy).  The
 // start of the n-th buffer is offset by (n mod 28) x 2304 B within its

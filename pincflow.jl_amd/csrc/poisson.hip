@@ -1869,16 +1869,16 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
 // ---------------------------------------------------------------------------
 
 // The member table covers the line preconditioner (FP64, or FP32 in the
-// mixed solve) on grids with an even x_size (the two-cell apply kernels; in
-// the mixed solve columns the line steps cover).  Members with the same key
-// share a table; -1: not covered.
+// mixed solve) on grids with an even x_size (the two-cell apply kernels).
+// Members with the same key share a table; -1: not covered.
 int ensemble_key(const pcf_state* st) {
   const pcf_config& n = st->cfg;
   const bool mixed = n.precision == PCF_PRECISION_MIXED;
   if (n.preconditioner == 0 || !use_pairs(st->g)) return -1;
-  if (mixed && (n.preconditioner_type == PCF_PC_MULTIGRID || !ensemble_line_covers(st))) return -1;
+  if (mixed && n.preconditioner_type == PCF_PC_MULTIGRID) return -1;
+  const int tall = mixed && ensemble_line_tall(st) ? 1 : 0;
   const int bf16 = mixed && n.preconditioner_storage == PCF_STORAGE_BF16 ? 1 : 0;
-  return (mixed ? 1 : 0) | bf16 << 1 | n.preconditioner_iterations << 2;
+  return (mixed ? 1 : 0) | bf16 << 1 | tall << 2 | n.preconditioner_iterations << 3;
 }
 
 // A solve joins the batch when its member is in a table and the solve is
@@ -1928,6 +1928,7 @@ static void ensemble_fill(pcf_ensemble::Group& grp) {
       M.factors32 = L0.factors;
       M.cur32 = L0.s;
       M.rhs32 = L0.rhs;
+      M.col32 = L0.col;
     }
     M.partials = st->partials;
     M.sc = st->sc;
@@ -1974,7 +1975,8 @@ int ensemble_iterate(pcf_ensemble* e, pcf_ensemble::Group& grp, int parity, int3
   if (cnt == 0) return PCF_OK;
   const bool mixed = (grp.key & 1) != 0;
   const bool bf16 = (grp.key & 2) != 0;
-  const int iters = grp.key >> 2;
+  const bool tall = (grp.key & 4) != 0;
+  const int iters = grp.key >> 3;
   hipStream_t s = e->stream;
   EnsList& L = grp.list_host[parity];
   L.count = cnt;
@@ -1995,7 +1997,7 @@ int ensemble_iterate(pcf_ensemble* e, pcf_ensemble::Group& grp, int parity, int3
   const EnsList* dL = grp.list;
   const int vb = cnt * kVecGrid;
   auto prec = [&](int in, int out) {
-    if (mixed) ensemble_precondition_mixed(s, dT, dL, L, threads, iters, bf16, in, out);
+    if (mixed) ensemble_precondition_mixed(s, dT, dL, L, threads, tall, iters, bf16, in, out);
     else ensemble_precondition(s, dT, dL, L, iters, in, out);
   };
   prec(EV_P, EV_Y);

@@ -29,8 +29,8 @@ from .state import PinCFlowError, State, integrate
 class SolveBatch:
     """The pcf_ensemble of a set of states: their BiCGSTAB solves run in one
     batch, one launch per kernel of an iteration over all solves in progress
-    (the line preconditioner in FP64 or FP32, x_size even, at most 256 levels
-    in the mixed solve; other solves run on their own); a solve joins and leaves
+    (the line preconditioner in FP64 or FP32, x_size even; other solves run on
+    their own); a solve joins and leaves
     the batch at iteration boundaries.  A state is attached from the thread
     that steps it and detached when that thread stops stepping it."""
 

@@ -2,6 +2,8 @@
 checks and error reporting on the CPU, the seeded bubble members on the
 oracle, and on the GPU members that share the device reproduce their
 standalone runs bit for bit."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -113,6 +115,53 @@ def test_batched_solves_give_each_member_its_standalone_bits(pcf, tmp_path, prec
         for f in ("RHOP", "U", "V", "W", "PIP", "RHO"):
             assert np.array_equal(st.get(f), alone.get(f)), (seed, f)
         alone.close()
+
+
+def _same_bits(pcf, sims):
+    """Two steps of each member, batched with the others and alone."""
+    def run(nl, batch):
+        st = pcf.State(nl)
+        if batch:
+            batch.attach(st)
+        its = [st.initial_cleaning()]
+        for _ in range(2):
+            its += list(st.step().niter)
+        fields = {f: st.get(f) for f in ("RHOP", "U", "V", "W", "PIP", "RHO")}
+        if batch:
+            batch.detach(st)
+        st.close()
+        return its, fields
+
+    batch, together = pcf.SolveBatch(), [None] * len(sims)
+    threads = [threading.Thread(target=lambda c=c: together.__setitem__(c, run(sims[c](), batch)))
+               for c in range(len(sims))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    stats = batch.stats()
+    batch.close()
+    for c, sim in enumerate(sims):
+        its, fields = run(sim(), None)
+        assert together[c][0] == its, (c, together[c][0], its)
+        for f in fields:
+            assert np.array_equal(fields[f], together[c][1][f]), (c, f)
+    return stats
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage", ["fp32", "bf16"])
+def test_mixed_members_of_any_even_width_and_height_are_batched(pcf, storage):
+    """x sizes 2 and 0 mod 4 and heights of one segment up to three chunks of
+    the FP32 line steps, in one batch (columns of more than 256 levels share a
+    table of their own): no solve runs alone, every member has its own bits."""
+    def member(seed, x_size, z_size):
+        nl = pcf.examples.bubble_member(seed=seed, x_size=x_size, z_size=z_size, iterations=2, precision="mixed")
+        nl.poisson.preconditioner_storage = storage
+        return nl
+    sizes = [(18, 12), (16, 41), (22, 130), (16, 300), (18, 257), (20, 530)]
+    stats = _same_bits(pcf, [lambda s=s, xz=xz: member(s, *xz) for s, xz in enumerate(sizes)])
+    assert stats["member_solves"] > 0 and stats["solves_alone"] == 0, stats
 
 
 @pytest.mark.gpu
