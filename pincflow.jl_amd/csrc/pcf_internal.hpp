@@ -298,6 +298,7 @@ struct pcf_state {
   double *pc_P, *pc_E, *pc_Q;         // line-solve factors of the current operator
   bool pc_factors_valid = false;
   double *pc_coefs = nullptr, *pc_factors = nullptr;  // packed for the line steps (line_step.hpp)
+  bool pc_packed_valid = false;
   // mixed precision (allocated when cfg.precision == PCF_PRECISION_MIXED):
   // the preconditioner's levels (mg below) and z = M^-1 s
   double* bzpc = nullptr;

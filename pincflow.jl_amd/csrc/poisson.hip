@@ -1456,16 +1456,26 @@ int pc_factors(pcf_state* st) {
   const Geo& g = st->g;
   hipLaunchKernelGGL(k_pc_factors, dim3(blocks_for(g.nx, 64), g.ny), dim3(64), 0, st->stream, st->T.a[T_AC],
                      st->T.a[T_AD], st->T.a[T_AU], st->pc_P, st->pc_E, st->pc_Q, g.nx, g.ny, g.nz, st->deta);
-  if (st->pc_coefs) {
-    LineCoefs<double> A;
-    for (int t = 0; t < T_COUNT; ++t) A.a[t] = st->T.a[t];
-    A.P = st->pc_P;
-    A.E = st->pc_E;
-    A.Q = st->pc_Q;
-    launch_line_pack(st->stream, A, st->pc_coefs, st->pc_factors, g.nx, g.ny, g.nz);
-  }
   PCF_HIP(hipGetLastError());
   st->pc_factors_valid = true;
+  st->pc_packed_valid = false;
+  return PCF_OK;
+}
+
+// The factors and, for a state whose preconditioner runs as line steps, their
+// packed copies with the coefficients'.
+static int pc_packed(pcf_state* st) {
+  int rc = pc_factors(st);
+  if (rc || !st->pc_coefs || st->pc_packed_valid) return rc;
+  const Geo& g = st->g;
+  LineCoefs<double> A;
+  for (int t = 0; t < T_COUNT; ++t) A.a[t] = st->T.a[t];
+  A.P = st->pc_P;
+  A.E = st->pc_E;
+  A.Q = st->pc_Q;
+  launch_line_pack(st->stream, A, st->pc_coefs, st->pc_factors, g.nx, g.ny, g.nz);
+  PCF_HIP(hipGetLastError());
+  st->pc_packed_valid = true;
   return PCF_OK;
 }
 
@@ -1489,7 +1499,7 @@ static bool use_line64(const Geo& g) {
 // The packed arrays of the FP64 line steps (pcf_create)
 int alloc_line64(pcf_state* st) {
   const Geo& g = st->g;
-  if (st->cfg.precision == PCF_PRECISION_MIXED || !use_line64(g)) return PCF_OK;
+  if (st->cfg.precision == PCF_PRECISION_MIXED || !st->cfg.preconditioner || !use_line64(g)) return PCF_OK;
   const size_t n = (size_t)LineTile<double>::count(g.nx, g.ny) * LineTile<double>::cols * g.nz;
   int rc = device_alloc(st, &st->pc_coefs, n * T_COUNT);
   return rc ? rc : device_alloc(st, &st->pc_factors, 3 * n);
@@ -1560,14 +1570,17 @@ static void line_step(pcf_state* st, const double* b, const double* s, double* o
 // M^-1 sin -> sout with preconditioner_iterations pseudo-time steps.  sout
 // must not alias sin.  `sc` (may be null) lets a converged solve skip it.
 // fuse != FUSE_NONE (line steps, two pseudo-time steps or more): F's BiCGSTAB
-// step runs in the first kernel, sin being the vector it updates.
+// step runs in the first kernel, sin being the vector it updates.  line = false:
+// not as line steps (the same bits), for a single application that is not
+// worth packing the coefficients.
 static int precondition(pcf_state* st, const double* sin, double* sout, const SolverScalars* sc,
-                        const BicgFuse* F = nullptr, int fuse = FUSE_NONE) {
+                        const BicgFuse* F = nullptr, int fuse = FUSE_NONE, bool line = true) {
   const Geo& g = st->g;
-  int rc = pc_factors(st);
+  line = line && st->pc_coefs;
+  int rc = line ? pc_packed(st) : pc_factors(st);
   if (rc) return rc;
   const int iters = st->cfg.preconditioner_iterations;
-  if (st->pc_coefs) {
+  if (line) {
     double* cur = iters == 1 ? sout : st->pc_tmp;
     {
       ProfScope prof(st, PCF_K_PC_THOMAS);
@@ -1704,10 +1717,12 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
   }
   const int aparts = apply_parts(g);
   const int maxit = n.poisson_iterations;
-  // the line-solve factors of this operator, before any capture of the
-  // iteration (precondition() computes them on first use)
+  const bool batched = st->ens && ensemble_batchable(st, mixed, stage);
+  // the line-solve factors of this operator and their packed copies, before
+  // any capture of the iteration (precondition() computes them on first use);
+  // the batch reads no packed copies
   if (pc && !mixed) {
-    int rcf = pc_factors(st);
+    int rcf = batched ? pc_factors(st) : pc_packed(st);
     if (rcf) return rcf;
   }
   // y = M^-1 p and z = M^-1 s are both kept for the textbook update
@@ -1719,13 +1734,13 @@ int bicgstab_core(pcf_state* st, double tolref, bool mixed, const double* guess,
   auto finish = [&]() -> int {
     if (pc && !yz) {
       hipLaunchKernelGGL(k_copy, dim3(kVecGrid), dim3(256), 0, st->stream, st->bs, st->solution, N);
-      int rc1 = precondition(st, st->bs, st->solution, nullptr);
+      int rc1 = precondition(st, st->bs, st->solution, nullptr, nullptr, FUSE_NONE, !batched);
       if (rc1) return rc1;
     }
     PCF_HIP(hipGetLastError());
     return PCF_OK;
   };
-  if (st->ens && ensemble_batchable(st, mixed, stage)) {
+  if (batched) {
     // the iterations run in the ensemble's batch, which leaves the final
     // scalars in sc_host[0]
     int rce = ensemble_solve(st);
