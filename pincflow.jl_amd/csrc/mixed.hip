@@ -27,8 +27,6 @@ namespace pcf {
 
 namespace {
 
-typedef float flt4 __attribute__((ext_vector_type(4)));
-
 // Memory layout of a level's arrays: x fastest (the finest level and the
 // levels smoothed with row-parallel kernels) or z fastest (the coarse levels
 // smoothed one column per wavefront, whose accesses are then contiguous
@@ -40,7 +38,8 @@ struct Lay {
     return zf ? (size_t)k + (size_t)nz * ((size_t)i + (size_t)nx * j)
               : (size_t)i + (size_t)nx * ((size_t)j + (size_t)ny * k);
   }
-  // 32-bit form for the levels of at most kColumnCols x kScanMaxNz cells
+  // 32-bit form for the levels smoothed column by column (at most
+  // kCoarseColumnCols x kScanMaxNz cells)
   __device__ int at32(int i, int j, int k) const { return zf ? k + nz * (i + nx * j) : i + nx * (j + ny * k); }
   __host__ __device__ size_t count() const { return (size_t)nx * ny * nz; }
   // the cell of the t-th element in memory order
@@ -1314,7 +1313,9 @@ int alloc_mixed(pcf_state* st) {
     L.bf16 = bf16_storage(st) && (!multigrid || columns(L) > kColumnCols || L.nz > kScanMaxNz);
     const size_t n = (size_t)LineTile<float>::count(L.nx, L.ny) * kTileCols * L.nz;
     int rc1 = device_alloc(st, &L.coefs, n * T_COUNT * (L.bf16 ? 2 : 4));
-    return rc1 ? rc1 : device_alloc(st, &L.factors, 3 * n);
+    if (!rc1) rc1 = device_alloc(st, &L.factors, 3 * n);
+    if (!rc1 && L.nz > kLineMaxNz) rc1 = device_alloc(st, &L.col, columns(L) * L.nz);
+    return rc1;
   };
   int rc;
   double** dl[] = {&st->bzpc, &st->m_prev[0], &st->m_prev[1]};
@@ -1332,7 +1333,7 @@ int alloc_mixed(pcf_state* st) {
   L0.ny = g.ny;
   L0.nz = g.nz;
   L0.deta = (float)st->deta;
-  for (float** p : {&L0.s, &L0.rhs, &L0.col})
+  for (float** p : {&L0.s, &L0.rhs})
     if ((rc = af(p))) return rc;
   if (!multigrid || !column_path(L0))
     if ((rc = packed(L0))) return rc;
@@ -1371,7 +1372,7 @@ int alloc_mixed(pcf_state* st) {
     auto ac = [&](float** p) -> int { return device_alloc(st, p, Nc); };
     for (int t = 0; t < T_COUNT; ++t)
       if ((rc = ac(&C.a[t]))) return rc;
-    float** v[] = {&C.P, &C.E, &C.Q, &C.b, &C.s, &C.rhs, &C.col};
+    float** v[] = {&C.P, &C.E, &C.Q, &C.b, &C.s, &C.rhs};
     for (float** p : v)
       if ((rc = ac(p))) return rc;
     C.zf = columns(C) <= kCoarseColumnCols && C.nz <= kScanMaxNz;  // smoothed column by column

@@ -88,7 +88,8 @@ struct MgLevel {
   char* coefs = nullptr;
   float* factors = nullptr;
   float *P = nullptr, *E = nullptr, *Q = nullptr;
-  float *b = nullptr, *s = nullptr, *rhs = nullptr, *col = nullptr;
+  float *b = nullptr, *s = nullptr, *rhs = nullptr;
+  float* col = nullptr;  // the upward sweep of tall columns (k_line_tall32)
 };
 
 // BiCGSTAB scalars kept on the device between kernels (apply_bicgstab!.jl:24-150).
