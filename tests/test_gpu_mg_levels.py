@@ -64,3 +64,13 @@ def test_small_levels_of_many_levels_match_the_restatement(pcf, shape, storage):
     16 x 16 x 160, the rounding of the scan over a wavefront's lanes on the
     nearly singular level."""
     assert vcycle_error(pcf, shape, storage) <= 1e-3
+
+
+@pytest.mark.parametrize("storage", ["fp32", "bf16"])
+@pytest.mark.parametrize("shape", [(260, 128, 128), (132, 66, 136)])
+def test_production_levels_match_the_restatement(pcf, shape, storage):
+    """Four columns per thread (4.26 million cells, a partial tile in x), whose
+    step with the correction reads two coarse cells at once and whose residual
+    sums x pairs in the thread; 136 levels on more than 128 tiles, sixteen
+    levels per thread."""
+    assert vcycle_error(pcf, shape, storage) <= 1e-3
