@@ -36,17 +36,15 @@ def configs(pcf):
         "cold_bubble": pcf.examples.cold_bubble(x_size=12, z_size=10),
         # the compressible model: the dP/dpi term on the operator's diagonal
         "hot_bubble": pcf.examples.hot_bubble(x_size=12, z_size=10),
-        # multigrid level paths: 64 x 64 row-path finest level with the fused
-        # restriction and wavefront-per-column line solves, 72 levels (two
-        # per lane); 256 x 72 with thread-per-column line solves and 2 x 1
-        # aggregation once ny is odd
+        # multigrid level paths: a 64 x 64 finest level of line steps with the
+        # packed residual, coarse levels smoothed column by column with 72
+        # levels (two per lane); 256 x 72 with two levels of line steps and
+        # 2 x 1 aggregation once ny is odd
         "mg_deep": pcf.examples.mountain_wave_3d(x_size=64, y_size=64, z_size=72, iterations=3),
         "mg_wide": pcf.examples.mountain_wave_3d(x_size=256, y_size=72, z_size=8, iterations=3),
-        # 32768 columns: the finest level's line solves keep their upward
-        # sweep in LDS, the coarser levels' in their scratch column
+        # 32768 columns, three levels of line steps of one segment
         "mg_lds": pcf.examples.mountain_wave_3d(x_size=256, y_size=128, z_size=8, iterations=3),
-        # 136 levels: the FP32 line solve of the line relaxation keeps 128 in
-        # LDS and the rest in its scratch column
+        # 136 levels: sixteen levels per thread in the line steps
         "tall": pcf.examples.mountain_wave_3d(x_size=16, y_size=12, z_size=136, iterations=3),
     }
 
@@ -67,7 +65,7 @@ def test_tall_columns_line_relaxation_meets_reference_criterion(pcf, abi, oracle
 
 @pytest.mark.parametrize("pc", ["line_relaxation", "multigrid"])
 def test_bf16_storage_solve_meets_reference_criterion(pcf, abi, oracle_mod, pc):
-    """bf16 coefficients in the preconditioner's row kernels (a finest level
+    """bf16 coefficients in the preconditioner's line steps (a finest level
     wide enough for them): the accuracy is the reference criterion's, as for
     any preconditioner."""
     solve_case(pcf, abi, oracle_mod, "mg_deep", pc, "bf16")
@@ -168,7 +166,7 @@ def test_multigrid_vcycle_matches_fp64_restatement(pcf, name, storage, nu, coars
     wrong index, sign or coefficient gives errors of order one.  With bf16
     storage the restatement rounds the finest level's applied coefficients
     the same way (FP64 -> FP32 -> bf16, nearest even); the cases with bf16 have
-    a finest level wide enough for the row kernels, which read bf16."""
+    a finest level of more than 1024 columns, which reads bf16."""
     import hipmem
     import mg_reference as mg
 
